@@ -18,11 +18,9 @@
 
 namespace sph {
 
-constexpr int kGradThreads = 256;
-constexpr int kChunk = 64;          // samples per block iteration
-constexpr int kLd = 65;             // padded LDS row stride (conflict-free columns)
-constexpr int kXd = 17;
-constexpr int kMaxGradBlocks = 1024;
+constexpr int kGradGroup = 32;      // samples of a wave's pass through the network
+constexpr int kGradWaves = 8;       // waves per block of the gradient kernel
+constexpr int kMaxGradBlocks = 256; // one block per CU
 constexpr int kMomentCols = 2 * (kMlpIn + 1);  // sums and squares of 12 features + target
 constexpr int kMomentBlocks = 512;
 
@@ -39,202 +37,443 @@ __device__ __forceinline__ uint64_t batch_row(uint64_t k, uint64_t count, uint64
   return random ? mix64(seed ^ mix64(k)) % count : k;
 }
 
-constexpr size_t kGradLdsFloats =
-    kMlpParams + 3 + kMlpH * kLd /* W2 transposed */ + kChunk * kXd + 4 * kChunk * kLd + kChunk;
+// ---------------------------------------------------------------------------
+// FP32 network on the matrix cores
+// ---------------------------------------------------------------------------
+// All products of the training and of the FP32 forward pass are FP32 MFMA
+// (v_mfma_f32_32x32x2_f32, FP32 inputs and accumulation).  A wave takes 32
+// samples as the columns of Z^T = W^T X^T, hidden units as rows, so a lane
+// holds one sample (lane % 32) and, in accumulator v of row block rb, hidden
+// unit 32 rb + mfma_drow(v, lane / 32).  An MFMA's B operand wants k = lane / 32
+// of column lane % 32, so accumulator (rb, v) is by itself a B operand whose
+// two k are the units the two lane halves hold: the next layer takes it as its
+// k chunk 16 rb + v without moving data, and the weights (its A operand) are
+// laid out in LDS in that order of k.  Lane half h reads features 6 h .. 6 h + 5
+// of its sample, chunk c of layer 1 being features (c, 6 + c).
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Per-block partial gradient of L = 0.5/B sum (y - t_n)^2 over a batch, with
-// x normalised by (x - mu) * inv_sigma and t_n = (t - y_shift) / y_scale.
-// 256 threads work on 64 samples at a time: in the forward and backward
-// passes thread (s = tid / 4, g = tid % 4) owns hidden units g + 4m of sample s.
-__global__ __launch_bounds__(kGradThreads) void k_mlp_grad(
-    uint64_t batch, uint64_t count, const float *__restrict__ x, const float *__restrict__ t,
-    uint64_t seed, int random, const float *__restrict__ theta, const float *__restrict__ norm,
-    float inv_batch, float *__restrict__ partial, float *__restrict__ loss_partial) {
-  extern __shared__ float sm[];
-  float *sW = sm;
-  float *sW2T = sW + kMlpParams + 3;
-  float *sX = sW2T + kMlpH * kLd;
-  float *sH1 = sX + kChunk * kXd;
-  float *sD1 = sH1 + kChunk * kLd;
-  float *sH2 = sD1 + kChunk * kLd;
-  float *sD2 = sH2 + kChunk * kLd;
-  float *sdy = sD2 + kChunk * kLd;
-  __shared__ float snorm[kNormWords];
-  __shared__ float sloss[kGradThreads / 64];
-  const int tid = threadIdx.x;
-  for (int i = tid; i < kMlpParams; i += kGradThreads) sW[i] = theta[i];
-  for (int i = tid; i < kMlpH * kMlpH; i += kGradThreads)
-    sW2T[(i & 63) * kLd + (i >> 6)] = theta[kMlpW2 + i];
-  if (tid < kNormWords) snorm[tid] = norm[tid];
-  __syncthreads();
-  const float *W1 = sW + kMlpW1, *b1 = sW + kMlpB1, *W2 = sW + kMlpW2, *b2 = sW + kMlpB2,
-              *w3 = sW + kMlpW3;
-  const float b3 = sW[kMlpB3];
-  const float y_shift = snorm[kNormYShift], inv_scale = 1.0f / snorm[kNormYScale];
-  const int sf = tid >> 2, gf = tid & 3;
-  float gW2[16], gW1[4], gv = 0.0f, loss = 0.0f;
-#pragma unroll
-  for (int m = 0; m < 16; ++m) gW2[m] = 0.0f;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) gW1[m] = 0.0f;
+constexpr int kHalfIn = kMlpIn / 2;
+constexpr int kSA1 = 0;                         // W1 operands [rb][2][lane][4]: 6 chunks, 2 unused
+constexpr int kSA2 = kSA1 + 2 * 2 * 64 * 4;     // W2^T operands [out block][8][lane][4]
+constexpr int kSBias = kSA2 + 2 * 8 * 64 * 4;   // b1, b2, w3 by [rb][half][v]
+constexpr int kSNorm = kSBias + 3 * kMlpH;      // feature means and reciprocal deviations
+constexpr int kSForward = kSNorm + 2 * kMlpPad; // floats of the forward pass
+constexpr int kSA3 = kSForward;                 // W2 operands [in block][8][lane][4]
+constexpr int kSGrad = kSA3 + 2 * 8 * 64 * 4;   // floats of the gradient pass
 
-  const uint64_t nchunks = (batch + kChunk - 1) / kChunk;
-  for (uint64_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    for (int e = tid; e < kChunk * kMlpPad; e += kGradThreads) {
-      const int s = e >> 4, i = e & 15;
-      const uint64_t k = ch * kChunk + s;
-      float val = 0.0f;
-      if (k < batch && i < kMlpIn) {
-        const uint64_t row = batch_row(k, count, seed, random);
-        val = (x[row * kMlpPad + i] - snorm[kNormMu + i]) * snorm[kNormIsd + i];
-      }
-      sX[s * kXd + i] = val;
-    }
-    __syncthreads();
-    {  // layer 1
-      float z[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) z[m] = b1[gf + 4 * m];
-      for (int i = 0; i < kMlpIn; ++i) {
-        const float xi = sX[sf * kXd + i];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) z[m] += xi * W1[i * kMlpH + gf + 4 * m];
-      }
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        sH1[sf * kLd + gf + 4 * m] = silu(z[m]);
-        sD1[sf * kLd + gf + 4 * m] = dsilu(z[m]);
-      }
-    }
-    __syncthreads();
-    float yp = 0.0f;
-    {  // layer 2 and the output unit
-      float z[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) z[m] = b2[gf + 4 * m];
-      for (int k = 0; k < kMlpH; ++k) {
-        const float hk = sH1[sf * kLd + k];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) z[m] += hk * W2[k * kMlpH + gf + 4 * m];
-      }
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        const float h = silu(z[m]);
-        sH2[sf * kLd + gf + 4 * m] = h;
-        sD2[sf * kLd + gf + 4 * m] = dsilu(z[m]);
-        yp += w3[gf + 4 * m] * h;
-      }
-    }
-    yp += __shfl_xor(yp, 1, 64);
-    yp += __shfl_xor(yp, 2, 64);
-    if (gf == 0) {
-      const uint64_t k = ch * kChunk + sf;
-      float dy = 0.0f;
-      if (k < batch) {
-        const uint64_t row = batch_row(k, count, seed, random);
-        const float r = yp + b3 - (t[row] - y_shift) * inv_scale;
-        loss += r * r;
-        dy = r * inv_batch;
-      }
-      sdy[sf] = dy;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) sD2[sf * kLd + gf + 4 * m] *= sdy[sf] * w3[gf + 4 * m];  // dZ2
-    __syncthreads();
-    {  // dZ1 = (dZ2 W2^T) * silu'(Z1)
-      float a[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) a[m] = 0.0f;
-      for (int k = 0; k < kMlpH; ++k) {
-        const float dk = sD2[sf * kLd + k];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) a[m] += dk * sW2T[k * kLd + gf + 4 * m];
-      }
-#pragma unroll
-      for (int m = 0; m < 16; ++m) sD1[sf * kLd + gf + 4 * m] *= a[m];
-    }
-    __syncthreads();
-    {  // dW2[j][g + 4m] += sum_s H1[s][j] dZ2[s][g + 4m]
-      const int j = tid >> 2, g = tid & 3;
-      for (int s = 0; s < kChunk; ++s) {
-        const float hj = sH1[s * kLd + j];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) gW2[m] += hj * sD2[s * kLd + g + 4 * m];
-      }
-    }
-    {  // dW1[i][jj + 16m] += sum_s X[s][i] dZ1[s][jj + 16m]
-      const int i = tid >> 4, jj = tid & 15;
-      for (int s = 0; s < kChunk; ++s) {
-        const float xi = sX[s * kXd + i];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) gW1[m] += xi * sD1[s * kLd + jj + 16 * m];
-      }
-    }
-    if (tid < 64) {
-      for (int s = 0; s < kChunk; ++s) gv += sD1[s * kLd + tid];
-    } else if (tid < 128) {
-      for (int s = 0; s < kChunk; ++s) gv += sD2[s * kLd + tid - 64];
-    } else if (tid < 192) {
-      for (int s = 0; s < kChunk; ++s) gv += sH2[s * kLd + tid - 128] * sdy[s];
-    } else if (tid == 192) {
-      for (int s = 0; s < kChunk; ++s) gv += sdy[s];
-    }
-    __syncthreads();
+// LDS word of the operand element (row `row`, k = hidden unit u) of a 64 x 64
+// operand [row block][8][lane][4]: unit u is k chunk 16 rb + v of lane half hf
+// where u = 32 rb + mfma_drow(v, hf).
+__device__ __forceinline__ int mlp32_slot(int row, int u) {
+  const int kc = 16 * (u >> 5) + 4 * ((u >> 3) & 3) + (u & 3);
+  return (((row >> 5) * 8 + (kc >> 2)) * 64 + 32 * ((u >> 2) & 1) + (row & 31)) * 4 + (kc & 3);
+}
+
+// Lays the weights out in LDS as the operands above (all threads of a block).
+template <bool GRAD>
+__device__ __forceinline__ void mlp32_weights(const float *__restrict__ theta,
+                                              const float *__restrict__ norm, float *sm) {
+  static_assert(kNormMu == 0 && kNormIsd == kMlpPad, "means, then reciprocal deviations");
+  if (threadIdx.x < 2 * kMlpPad) sm[kSNorm + threadIdx.x] = norm[threadIdx.x];
+  for (int e = threadIdx.x; e < 2 * 2 * 64 * 4; e += blockDim.x) {
+    const int rb = e >> 9, c = ((e >> 8) & 1) * 4 + (e & 3), l = (e >> 2) & 63;
+    sm[kSA1 + e] = c < kHalfIn
+                       ? theta[kMlpW1 + (c + kHalfIn * (l >> 5)) * kMlpH + 32 * rb + (l & 31)]
+                       : 0.0f;
   }
-  float *P = partial + (size_t)blockIdx.x * kMlpParams;
-  {
-    const int j = tid >> 2, g = tid & 3;
-#pragma unroll
-    for (int m = 0; m < 16; ++m) P[kMlpW2 + j * kMlpH + g + 4 * m] = gW2[m];
+  // W2 is read in its own order (coalesced) and scattered in LDS
+  for (int e = threadIdx.x; e < kMlpH * kMlpH; e += blockDim.x) {
+    const int r = e >> 6, c = e & 63;
+    const float w = theta[kMlpW2 + e];
+    sm[kSA2 + mlp32_slot(c, r)] = w;
+    if (GRAD) sm[kSA3 + mlp32_slot(r, c)] = w;
   }
-  {
-    const int i = tid >> 4, jj = tid & 15;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) P[kMlpW1 + i * kMlpH + jj + 16 * m] = gW1[m];
-  }
-  if (tid < 64) P[kMlpB1 + tid] = gv;
-  else if (tid < 128) P[kMlpB2 + tid - 64] = gv;
-  else if (tid < 192) P[kMlpW3 + tid - 128] = gv;
-  else if (tid == 192) P[kMlpB3] = gv;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) loss += __shfl_xor(loss, o, 64);
-  if ((tid & 63) == 0) sloss[tid >> 6] = loss;
-  __syncthreads();
-  if (tid == 0) {
-    float l = 0.0f;
-    for (int w = 0; w < kGradThreads / 64; ++w) l += sloss[w];
-    loss_partial[blockIdx.x] = 0.5f * l;
+  if (threadIdx.x < kMlpH) {
+    const int e = threadIdx.x, u = 32 * (e >> 5) + mfma_drow(e & 15, (e >> 4) & 1);
+    sm[kSBias + e] = theta[kMlpB1 + u];
+    sm[kSBias + kMlpH + e] = theta[kMlpB2 + u];
+    sm[kSBias + 2 * kMlpH + e] = theta[kMlpW3 + u];
   }
 }
 
-// Sums the block partials in a fixed order (deterministic), zeroes the
-// gradient of the padding inputs and optionally applies one Adam step
-// (Kingma & Ba, beta1 0.9, beta2 0.999, eps 1e-8; bc = bias corrections).
-__global__ __launch_bounds__(kBlock) void k_mlp_adam(int nblocks, const float *__restrict__ partial,
-                                                     const float *__restrict__ loss_partial,
-                                                     float *__restrict__ theta, float *__restrict__ mom,
-                                                     float *__restrict__ vel, float *__restrict__ grad,
-                                                     float *__restrict__ loss_out, float inv_batch,
-                                                     float lr, float bc1, float bc2, int apply) {
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p < kMlpParams) {
-    float g = 0.0f;
-    for (int b = 0; b < nblocks; ++b) g += partial[(size_t)b * kMlpParams + p];
-    if (p >= kMlpW1 + kMlpIn * kMlpH && p < kMlpB1) g = 0.0f;
-    grad[p] = g;
-    if (apply) {
-      const float m = 0.9f * mom[p] + 0.1f * g;
-      const float v = 0.999f * vel[p] + 0.001f * g * g;
-      mom[p] = m;
-      vel[p] = v;
-      theta[p] -= lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f);
-    }
+// This lane's 16 values of a [rb][half][v] vector.
+__device__ __forceinline__ void mlp32_vec(const float *v, int rb, int half, float (&out)[16]) {
+  const float4 *q = reinterpret_cast<const float4 *>(v) + (rb * 2 + half) * 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 a = q[i];
+    out[4 * i] = a.x; out[4 * i + 1] = a.y; out[4 * i + 2] = a.z; out[4 * i + 3] = a.w;
   }
-  if (p == 0) {
-    float l = 0.0f;
-    for (int b = 0; b < nblocks; ++b) l += loss_partial[b];
-    *loss_out = l * inv_batch;
+}
+
+__device__ __forceinline__ floatx16_t mlp32_bias(const float *v, int rb, int half) {
+  float b[16];
+  mlp32_vec(v, rb, half, b);
+  floatx16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = b[i];
+  return acc;
+}
+
+// Layer 1: z[rb] from this lane's six features.
+__device__ __forceinline__ void mlp32_layer1(const float *sm, const float (&x)[kHalfIn], int lane,
+                                             floatx16_t (&z)[2]) {
+  const float4 *A = reinterpret_cast<const float4 *>(sm + kSA1);
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const float4 a = A[(rb * 2) * 64 + lane], b = A[(rb * 2 + 1) * 64 + lane];
+    const float w[kHalfIn] = {a.x, a.y, a.z, a.w, b.x, b.y};
+    floatx16_t acc = mlp32_bias(sm + kSBias, rb, lane >> 5);
+#pragma unroll
+    for (int c = 0; c < kHalfIn; ++c)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w[c], x[c], acc, 0, 0, 0);
+    z[rb] = acc;
+  }
+}
+
+// z[ob] += (64 x 64 operands at A) h, over the 32 k chunks that h's
+// accumulators are.
+__device__ __forceinline__ void mlp32_square(const float *ops, const floatx16_t (&h)[2], int lane,
+                                             floatx16_t (&z)[2]) {
+  const float4 *A = reinterpret_cast<const float4 *>(ops);
+  float4 a = A[lane], b = A[8 * 64 + lane];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w};
+    if (q < 7) {  // the next operands come in under this chunk's products
+      a = A[(q + 1) * 64 + lane];
+      b = A[(9 + q) * 64 + lane];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float k = h[q >> 2][(q & 3) * 4 + e];
+      z[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], k, z[0], 0, 0, 0);
+      z[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb[e], k, z[1], 0, 0, 0);
+    }
+    // without it the compiler loads all operands first and spills
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// 1 / (1 + e^-z) to about 1 ulp: e^-z as the hardware exp2 of -z log2(e) in two
+// floats, and the hardware reciprocal with one Newton step (8 VALU and two
+// transcendentals; expf and two IEEE divisions are about 40).  z is held to
+// [-87, 100] for the exponential only, past which e^-z is 0 or the sigmoid
+// below 2e-38.
+__device__ __forceinline__ float sigmoid32(float z) {
+  const float zc = __builtin_amdgcn_fmed3f(z, -87.0f, 100.0f);
+  const float t = -1.44269504f * zc;  // log2(e) = 1.44269502 + 1.92596303e-8
+  const float lo = fmaf(-1.92596303e-8f, zc, fmaf(-1.44269504f, zc, -t));
+  const float p = __builtin_amdgcn_exp2f(t);
+  const float d = 1.0f + fmaf(0.693147182f * p, lo, p);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(r, fmaf(-d, r, 1.0f), r);
+}
+
+// The LDS writes of a wave before, its reads after: a lane reads what other
+// lanes of its own wave wrote (LDS operations of a wave complete in order).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // and nothing of the next phase moves up into this one's registers
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Gradient sums leave a block in register order, slot x 64 lanes, and
+// k_mlp_adam finds each parameter in it (grad_param): slots 0-63 dW2, 64-79 dW1
+// with db1 as its thirteenth row, 80 dw3, 81 db2, 82 db3 and the loss.
+constexpr int kSlotW2 = 0, kSlotW1 = 64, kSlotW3 = 80, kSlotB2 = 81, kSlotMisc = 82,
+              kGradSlots = 83;
+constexpr int kGradWords = kGradSlots * 64;
+
+// Parameter of word (slot, lane), -1 for none, -2 for the loss.
+__device__ __forceinline__ int grad_param(int slot, int lane) {
+  if (slot < kSlotW1) {
+    const int jb = slot >> 5, mb = (slot >> 4) & 1;
+    return kMlpW2 + (32 * jb + mfma_drow(slot & 15, lane >> 5)) * kMlpH + 32 * mb + (lane & 31);
+  }
+  if (slot < kSlotW3) {
+    const int q = slot - kSlotW1, i = lane & 15;
+    const int j = 16 * (q >> 2) + 4 * (lane >> 4) + (q & 3);
+    return i < kMlpIn ? kMlpW1 + i * kMlpH + j : (i == kMlpIn ? kMlpB1 + j : -1);
+  }
+  if (slot == kSlotW3) return kMlpW3 + lane;
+  if (slot == kSlotB2) return kMlpB2 + lane;
+  return lane == 0 ? kMlpB3 : (lane == 1 ? -2 : -1);
+}
+
+constexpr int kTLd = 68;  // LDS row of 64 units (16-byte aligned, rows 4 banks apart)
+constexpr int kWaveLds = kGradGroup * kTLd + kGradGroup * 16;
+
+constexpr size_t kGradLds = sizeof(float) * (kSGrad + kGradWaves * kWaveLds);
+static_assert(4 * kGradWords * sizeof(float) <= kGradLds && kGradLds <= 160 * 1024,
+              "four waves' sums fit in the LDS of the pass");
+
+// Per-block partial gradient of L = 0.5/B sum (y - t_n)^2 over a batch, with
+// x normalised by (x - mu) * inv_sigma and t_n = (t - y_shift) / y_scale.
+//
+// A wave takes 32 samples at a time through both passes in registers: 216 MFMA
+// of 64 cycles and 32 of half the size, 14,800 matrix cycles, and about 1,800
+// VALU.  FP32 MFMA runs in the vector units' time on this target (with two
+// waves per SIMD the counters show the two one after the other, 47% MFMA busy),
+// so their sum bounds it: 16 us for 65,536 samples.  The weight gradients sum
+// over samples, so H1, dZ2 and dZ1 go through a 32 x 64 LDS tile of the wave's
+// own to become operands with k = sample.  A block is a CU's worth of waves
+// (two per SIMD, at 256 registers) and adds their sums in LDS, so that at most
+// 256 partials leave the chip instead of one per 64 samples.  Measured with
+// k_mlp_adam per step of 65,536 samples: 434 us with the products on the vector
+// units, each reading its weight from LDS, to 44 us (39 of them here); of
+// 1,000,003: 373 us.
+__global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(
+    uint64_t batch, uint64_t count, const float *__restrict__ x, const float *__restrict__ t,
+    uint64_t seed, int random, const float *__restrict__ theta, const float *__restrict__ norm,
+    float inv_batch, float *__restrict__ partial) {
+  extern __shared__ __align__(16) float sm[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int half = lane >> 5, col = lane & 31;
+  const uint64_t groups = (batch + kGradGroup - 1) / kGradGroup;
+  const uint64_t g0 = (uint64_t)wave * gridDim.x + blockIdx.x, gstep = (uint64_t)gridDim.x * kGradWaves;
+  // a group's raw rows, loaded before the work that hides their latency: the
+  // weights' way into LDS for the first group
+  f2u raw[kHalfIn / 2];
+  float traw = 0.0f;
+  auto fetch = [&](uint64_t g) {
+    const uint64_t k = g * kGradGroup + col;
+#pragma unroll
+    for (int c = 0; c < kHalfIn / 2; ++c) raw[c] = f2u{0.0f, 0.0f};
+    if (k < batch) {
+      const uint64_t row = batch_row(k, count, seed, random);
+      const float *r = x + row * kMlpPad + kHalfIn * half;
+#pragma unroll
+      for (int c = 0; c < kHalfIn / 2; ++c) raw[c] = reinterpret_cast<const f2u *>(r)[c];
+      traw = t[row];
+    }
+  };
+  fetch(g0);
+  mlp32_weights<true>(theta, norm, sm);
+  float *T = sm + kSGrad + wave * kWaveLds;  // [sample][unit]
+  float *X = T + kGradGroup * kTLd;          // [sample][feature], feature 12 = 1
+  const float y_shift = norm[kNormYShift], inv_scale = 1.0f / norm[kNormYScale];
+  const float b3 = theta[kMlpB3];
+  __syncthreads();
+
+  floatx16_t gW2[2][2] = {};  // [row block of W2's inputs][column block of its outputs]
+  floatx4_t gW1[4] = {};
+  float gw3 = 0.0f, gb2[2] = {0.0f, 0.0f}, gb3 = 0.0f, loss = 0.0f;
+  for (uint64_t g = g0; g < groups; g += gstep) {
+    // the operands are read again for each group: kept in registers over the
+    // loop, as the compiler would, they cost 120 that the sums need
+    int again = 0;
+    asm volatile("" : "+s"(again));
+    const float *W = sm + again;
+    const uint64_t k = g * kGradGroup + col;
+    const float tn = (traw - y_shift) * inv_scale;
+    float xn[kHalfIn];
+    const float *mu = W + kSNorm + kHalfIn * half, *isd = mu + kMlpPad;
+#pragma unroll
+    for (int c = 0; c < kHalfIn; ++c)  // a sample past the batch is zero after normalisation
+      xn[c] = k < batch ? (raw[c / 2][c & 1] - mu[c]) * isd[c] : 0.0f;
+#pragma unroll
+    for (int c = 0; c < kHalfIn; ++c) X[col * 16 + kHalfIn * half + c] = xn[c];
+    if (half) {
+      X[col * 16 + 12] = 1.0f;
+      X[col * 16 + 13] = X[col * 16 + 14] = X[col * 16 + 15] = 0.0f;
+    }
+    floatx16_t h1[2];
+    mlp32_layer1(W, xn, lane, h1);
+    if (g + gstep < groups) fetch(g + gstep);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float z = h1[rb][v];
+        h1[rb][v] = z * sigmoid32(z);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    floatx16_t d2[2];
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob) d2[ob] = mlp32_bias(W + kSBias + kMlpH, ob, half);
+    mlp32_square(W + kSA2, h1, lane, d2);
+    // H1 as dW2's A operand: unit lane % 32 of sample 2 c + half
+    float4 *Tw = reinterpret_cast<float4 *>(T + col * kTLd + 4 * half);
+    auto put = [&](const floatx16_t &m, int rb) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        Tw[8 * rb + 2 * q] = make_float4(m[4 * q], m[4 * q + 1], m[4 * q + 2], m[4 * q + 3]);
+    };
+    put(h1[0], 0);
+    put(h1[1], 1);
+    wave_lds_fence();
+    float h1t[2][16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      h1t[0][c] = T[(2 * c + half) * kTLd + col];
+      h1t[1][c] = T[(2 * c + half) * kTLd + 32 + col];
+    }
+    wave_lds_fence();
+    float yp = 0.0f;
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob) {
+      float w3[16];
+      mlp32_vec(W + kSBias + 2 * kMlpH, ob, half, w3);
+      floatx16_t h2;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float z = d2[ob][v], s = sigmoid32(z);
+        h2[v] = z * s;
+        d2[ob][v] = s * fmaf(z, 1.0f - s, 1.0f) * w3[v];
+        yp = fmaf(w3[v], h2[v], yp);
+      }
+      put(h2, ob);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    yp += __shfl_xor(yp, 32, 64);
+    float dy = 0.0f;
+    if (k < batch) {
+      const float r = yp + b3 - tn;
+      if (!half) loss = fmaf(r, r, loss);
+      dy = r * inv_batch;
+    }
+    if (!half) gb3 += dy;
+    wave_lds_fence();
+#pragma unroll
+    for (int s = 0; s < kGradGroup; ++s)
+      gw3 = fmaf(T[s * kTLd + lane],
+                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dy), s)), gw3);
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) d2[ob][v] *= dy;  // dZ2
+    wave_lds_fence();
+    put(d2[0], 0);
+    put(d2[1], 1);
+    wave_lds_fence();
+    // dW2 += H1^T dZ2, two samples a chunk
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const float z0 = T[(2 * c + half) * kTLd + col], z1 = T[(2 * c + half) * kTLd + 32 + col];
+      gb2[0] += z0;
+      gb2[1] += z1;
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) {
+        gW2[jb][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(h1t[jb][c], z0, gW2[jb][0], 0, 0, 0);
+        gW2[jb][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(h1t[jb][c], z1, gW2[jb][1], 0, 0, 0);
+      }
+      if ((c & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    // dZ1 = (W2 dZ2) * silu'(Z1), Z1 computed again: held since the forward
+    // pass its derivative took 32 registers, and spilled
+    floatx16_t a1[2] = {};
+    mlp32_square(W + kSA3, d2, lane, a1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < kHalfIn; ++c) xn[c] = X[col * 16 + kHalfIn * half + c];
+    mlp32_layer1(W, xn, lane, d2);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float z = d2[rb][v], s = sigmoid32(z);
+        a1[rb][v] *= s * fmaf(z, 1.0f - s, 1.0f);
+      }
+    wave_lds_fence();
+    put(a1[0], 0);
+    put(a1[1], 1);
+    wave_lds_fence();
+    // [dW1; db1]^T += dZ1^T [X 1], four samples a chunk
+    const int r4 = lane >> 4, c16 = lane & 15;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float xv = X[(4 * c + r4) * 16 + c16];
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb)
+        gW1[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            T[(4 * c + r4) * kTLd + 16 * jb + c16], xv, gW1[jb], 0, 0, 0);
+      if (c & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    wave_lds_fence();
+  }
+
+  float sum[kGradSlots];
+#pragma unroll
+  for (int q = 0; q < 64; ++q) sum[kSlotW2 + q] = gW2[q >> 5][(q >> 4) & 1][q & 15];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) sum[kSlotW1 + q] = gW1[q >> 2][q & 3];
+  sum[kSlotW3] = gw3;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) gb2[b] += __shfl_xor(gb2[b], 32, 64);
+  sum[kSlotB2] = half ? gb2[1] : gb2[0];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    gb3 += __shfl_xor(gb3, o, 64);
+    loss += __shfl_xor(loss, o, 64);
+  }
+  sum[kSlotMisc] = lane == 0 ? gb3 : (lane == 1 ? loss : 0.0f);
+  // sums of the waves that had samples: the upper four onto the lower four,
+  // then those by all threads (the weights' LDS is free by now)
+  const int busy = (int)min((uint64_t)kGradWaves, (groups + gridDim.x - 1) / gridDim.x);
+  __syncthreads();
+  if (busy > 4) {
+    if (wave >= 4 && wave < busy) {
+#pragma unroll
+      for (int q = 0; q < kGradSlots; ++q) sm[(wave - 4) * kGradWords + q * 64 + lane] = sum[q];
+    }
+    __syncthreads();
+    if (wave + 4 < busy) {
+#pragma unroll
+      for (int q = 0; q < kGradSlots; ++q) sum[q] += sm[wave * kGradWords + q * 64 + lane];
+    }
+    __syncthreads();
+  }
+  const int left = min(busy, 4);
+  if (wave < left) {
+#pragma unroll
+    for (int q = 0; q < kGradSlots; ++q) sm[wave * kGradWords + q * 64 + lane] = sum[q];
+  }
+  __syncthreads();
+  float *P = partial + (size_t)blockIdx.x * kGradWords;
+  for (int e = threadIdx.x; e < kGradWords; e += blockDim.x) {
+    float a = sm[e];
+    for (int w = 1; w < left; ++w) a += sm[w * kGradWords + e];
+    P[e] = a;
+  }
+}
+
+// Sums the block partials in a fixed order (deterministic) and optionally
+// applies one Adam step (Kingma & Ba, beta1 0.9, beta2 0.999, eps 1e-8; bc =
+// bias corrections).  One block per slot of 64 parameters, its eight waves
+// taking every eighth partial: with one thread walking all partials of a
+// parameter in turn (1024 of them, 21 blocks) this took 279 us, now 5.4 us
+// (256 partials).  The padding inputs have no word here; their gradient stays
+// the zero it was created as.
+constexpr int kAdamWaves = 8;
+__global__ __launch_bounds__(64 * kAdamWaves) void k_mlp_adam(
+    int nblocks, const float *__restrict__ partial, float *__restrict__ theta,
+    float *__restrict__ mom, float *__restrict__ vel, float *__restrict__ grad,
+    float *__restrict__ loss_out, float inv_batch, float lr, float bc1, float bc2, int apply) {
+  __shared__ float part[kAdamWaves][64];
+  const int slot = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float g = 0.0f;
+#pragma unroll 8
+  for (int b = wave; b < nblocks; b += kAdamWaves)
+    g += partial[(size_t)b * kGradWords + slot * 64 + lane];
+  part[wave][lane] = g;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 1; w < kAdamWaves; ++w) g += part[w][lane];
+  const int p = grad_param(slot, lane);
+  if (p == -2) *loss_out = 0.5f * g * inv_batch;
+  if (p < 0) return;
+  grad[p] = g;
+  if (apply) {
+    const float m = 0.9f * mom[p] + 0.1f * g;
+    const float v = 0.999f * vel[p] + 0.001f * g * g;
+    mom[p] = m;
+    vel[p] = v;
+    theta[p] -= lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f);
   }
 }
 
@@ -362,7 +601,7 @@ static int mlp_configure() {
   if (done) return SPH_OK;
   SPH_HIP(hipFuncSetAttribute((const void *)k_mlp_grad,
                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)(kGradLdsFloats * sizeof(float))));
+                              (int)kGradLds));
   done = 1;
   return SPH_OK;
 }
@@ -376,7 +615,7 @@ struct sph_mlp {
   hipStream_t stream = nullptr;
   float *theta = nullptr, *mom = nullptr, *vel = nullptr, *grad = nullptr;
   float *norm = nullptr;
-  float *partial = nullptr, *loss_partial = nullptr, *loss = nullptr;
+  float *partial = nullptr, *loss = nullptr;
   double *moments = nullptr;
   MlpPacked *packed = nullptr;
   float host_norm[kNormWords] = {};
@@ -397,7 +636,7 @@ static int upload_norm(sph_mlp *m) {
 
 static void mlp_free(sph_mlp *m) {
   void *bufs[] = {m->theta, m->mom, m->vel, m->grad, m->norm, m->partial,
-                  m->loss_partial, m->loss, m->moments, m->packed};
+                  m->loss, m->moments, m->packed};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -417,17 +656,15 @@ extern "C" int sph_mlp_create(sph_mlp **out) {
       {(void **)&m->vel, sizeof(float) * kMlpParams},
       {(void **)&m->grad, sizeof(float) * kMlpParams},
       {(void **)&m->norm, sizeof(float) * kNormWords},
-      {(void **)&m->partial, sizeof(float) * kMlpParams * kMaxGradBlocks},
-      {(void **)&m->loss_partial, sizeof(float) * kMaxGradBlocks},
+      {(void **)&m->partial, sizeof(float) * kGradWords * kMaxGradBlocks},
       {(void **)&m->loss, sizeof(float)},
       {(void **)&m->moments, sizeof(double) * kMomentCols * kMomentBlocks},
       {(void **)&m->packed, sizeof(MlpPacked)},
   };
   for (auto &a : allocs)
     if (e == hipSuccess) e = hipMalloc(a.p, a.bytes);
-  for (int i = 0; i < 3 && e == hipSuccess; ++i)
-    e = hipMemsetAsync(i == 0 ? m->theta : i == 1 ? m->mom : m->vel, 0,
-                       sizeof(float) * kMlpParams, m->stream);
+  for (float *z : {m->theta, m->mom, m->vel, m->grad})
+    if (e == hipSuccess) e = hipMemsetAsync(z, 0, sizeof(float) * kMlpParams, m->stream);
   if (e != hipSuccess) {
     mlp_free(m);
     delete m;
@@ -580,12 +817,11 @@ extern "C" int sph_mlp_fit_normalization(sph_mlp *m, const float *x, const float
 
 static int grad_pass(sph_mlp *m, const float *x, const float *t, size_t count, size_t batch,
                      uint64_t seed, int random, float lr, int apply) {
-  const uint64_t nchunks = (batch + kChunk - 1) / kChunk;
-  const int nb = (int)std::min<uint64_t>(kMaxGradBlocks, nchunks);
+  const uint64_t groups = (batch + kGradGroup - 1) / kGradGroup;
+  const int nb = (int)std::min<uint64_t>(kMaxGradBlocks, groups);
   const float inv_batch = (float)(1.0 / (double)batch);
-  k_mlp_grad<<<nb, kGradThreads, kGradLdsFloats * sizeof(float), m->stream>>>(
-      batch, count, x, t, seed, random, m->theta, m->norm, inv_batch, m->partial,
-      m->loss_partial);
+  k_mlp_grad<<<nb, 64 * kGradWaves, kGradLds, m->stream>>>(
+      batch, count, x, t, seed, random, m->theta, m->norm, inv_batch, m->partial);
   SPH_HIP(hipGetLastError());
   float bc1 = 1.0f, bc2 = 1.0f;
   if (apply) {
@@ -593,9 +829,8 @@ static int grad_pass(sph_mlp *m, const float *x, const float *t, size_t count, s
     bc1 = (float)(1.0 - pow(0.9, (double)m->step));
     bc2 = (float)(1.0 - pow(0.999, (double)m->step));
   }
-  k_mlp_adam<<<blocks_for(kMlpParams), kBlock, 0, m->stream>>>(
-      nb, m->partial, m->loss_partial, m->theta, m->mom, m->vel, m->grad, m->loss, inv_batch, lr,
-      bc1, bc2, apply);
+  k_mlp_adam<<<kGradSlots, 64 * kAdamWaves, 0, m->stream>>>(
+      nb, m->partial, m->theta, m->mom, m->vel, m->grad, m->loss, inv_batch, lr, bc1, bc2, apply);
   SPH_HIP(hipGetLastError());
   return SPH_OK;
 }

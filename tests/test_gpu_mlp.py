@@ -65,6 +65,14 @@ def test_gradient_matches_oracle(count):
     assert np.all(g[12 * 64:16 * 64] == 0.0)  # padding inputs
 
 
+# Edges of the gradient kernel's split: 32 samples a wave, 256 blocks, 8 waves a
+# block, more than one pass.  Its FP32 sums hold the bound of the other counts.
+@pytest.mark.parametrize("count", [31, 32, 33, 256 * 32, 256 * 32 + 1, 5 * 256 * 32 + 7,
+                                   8 * 256 * 32 + 33])
+def test_gradient_at_the_edges_of_its_split(count):
+    test_gradient_matches_oracle(count)
+
+
 def test_adam_steps_match_oracle():
     count = 4096
     x, t, shift, scale = _dataset(count, 7)
@@ -85,8 +93,13 @@ def test_adam_steps_match_oracle():
         th = got  # continue from the device's FP32 weights
 
 
-def test_forward_fp32_matches_oracle():
-    count = 10_000
+# 32 rows a wave, 4 waves a block, 1024 blocks before a second pass
+@pytest.mark.parametrize("count", [1, 31, 32, 33, 129, 1024 * 128 + 1])
+def test_forward_fp32_at_the_edges_of_its_split(count):
+    test_forward_fp32_matches_oracle(count)
+
+
+def test_forward_fp32_matches_oracle(count=10_000):
     x, t, shift, scale = _dataset(count, 3)
     net, theta = _net(3, shift, scale, 0.02, 0.5)
     xb = sa.DeviceBuffer.from_array(x)
