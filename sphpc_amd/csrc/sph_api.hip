@@ -89,7 +89,7 @@ static const char *kKernelNames[K_COUNT] = {
     "predict_hash", "hash", "gravity", "predict", "radix_upsweep", "radix_downsweep",
     "scan", "reorder", "build_lists", "density_lambda", "density", "lambda", "dp",
     "dp_update", "position_stars", "velocity", "color", "surface", "xsph", "vorticity",
-    "confine", "commit", "aux", "warm_lambda", "collide", "lambda_copy"};
+    "confine", "commit", "aux", "warm_lambda", "collide", "lambda_copy", "place"};
 
 // Derived FP32 constants (SetParameters, simulation.c:147-177; the constants
 // of particles.c named in DevParams).  Computed in double, rounded once.
@@ -182,8 +182,8 @@ static void graph_reset(sph_ctx *c) {
 
 static void free_all(sph_ctx *c) {
   graph_reset(c);
-  void *bufs[] = {c->x_can, c->v_can, c->xs_can, c->keys, c->keys_alt, c->ids, c->ids_alt,
-                  c->hist, c->cell_end, c->cell_start, c->pos_a, c->pos_b, c->xold,
+  void *bufs[] = {c->x_can, c->v_can, c->xs_can, c->keys, c->cell_rank, c->slots,
+                  c->key_s, c->id_s, c->cell_count, c->cell_start, c->pos_a, c->pos_b, c->xold,
                   c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage, c->lam_stage,
                   c->list, c->list_head,
                   c->stats, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
@@ -260,8 +260,8 @@ extern "C" void sph_default_params(sph_params *p, double h) {
   p->vorticity_model = 0;
 }
 
-// Device buffers, stream and kernel set-up of a context whose grid (cells,
-// key_bits) and capacity are known.  Frees the context on failure.
+// Device buffers, stream and kernel set-up of a context whose grid (cells)
+// and capacity are known.  Frees the context on failure.
 static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
   auto fail = [&](int code) {
     free_all(c);
@@ -283,8 +283,9 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
   } allocs[] = {
       {(void **)&c->x_can, f4},       {(void **)&c->v_can, f4},
       {(void **)&c->xs_can, f4},      {(void **)&c->keys, u4},
-      {(void **)&c->keys_alt, u4},    {(void **)&c->ids, u4},
-      {(void **)&c->ids_alt, u4},     {(void **)&c->cell_end, sizeof(uint32_t) * (c->cells + 1ull)},
+      {(void **)&c->cell_rank, u4},   {(void **)&c->slots, sizeof(uint2) * cap},
+      {(void **)&c->key_s, u4},       {(void **)&c->id_s, u4},
+      {(void **)&c->cell_count, sizeof(uint32_t) * (c->cells + 1ull)},
       {(void **)&c->cell_start, sizeof(uint32_t) * (c->cells + 1ull)},
       {(void **)&c->pos_a, f4 + sizeof(float4) * kPosPad},
       {(void **)&c->pos_b, f4 + sizeof(float4) * kPosPad},
@@ -297,6 +298,9 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       {(void **)&c->list_head, sizeof(uint4) * cap},
       {(void **)&c->pw, f4},
       {(void **)&c->sx, sizeof(float) * 3 * (cap + kPosPad)},
+      // here and not on first use: a search must not end between its counts and
+      // their placing, which zeroes them
+      {(void **)&c->scan.tile_sums, sizeof(uint32_t) * scan_tiles(c->cells)},
       {(void **)&c->stats, sizeof(uint32_t) * STAT_WORDS},
       {(void **)&c->pair_partial, sizeof(uint32_t) * blocks_for((uint32_t)cap, kWave)},
       {(void **)&c->red, sizeof(double) * std::max<size_t>(4, blocks_for((uint32_t)cap))},
@@ -305,7 +309,7 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
     e = hipMalloc(a.p, a.bytes);
     if (e != hipSuccess) return fail(hip_fail(e, "hipMalloc (context buffers)"));
   }
-  e = hipMemsetAsync(c->cell_end, 0, sizeof(uint32_t) * (c->cells + 1ull), c->stream);
+  e = hipMemsetAsync(c->cell_count, 0, sizeof(uint32_t) * (c->cells + 1ull), c->stream);
   if (e == hipSuccess) e = hipMemsetAsync(c->stats, 0, sizeof(uint32_t) * STAT_WORDS, c->stream);
   if (e == hipSuccess) e = hipMemsetAsync(c->list_head, 0, sizeof(uint4) * cap, c->stream);
   // C = 0 until a density stage runs (lambda from it is zero, as the
@@ -318,6 +322,7 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
   if (e != hipSuccess) return fail(hip_fail(e, "context initialisation"));
   c->pos = c->pos_a;
   c->soa_stride = (uint32_t)(cap + kPosPad);
+  c->scan.tile_cap = scan_tiles(c->cells);
   c->vel = c->vel_a;
   *out = c;
   return SPH_OK;
@@ -357,8 +362,6 @@ extern "C" int sph_create(const sph_params *params, const sph_aabb *boundary, in
   c->dev.nz = (uint32_t)nzd;
   c->dev.nxy = c->dev.nx * c->dev.ny;
   c->cells = c->dev.nxy * c->dev.nz;
-  c->key_bits = 1;
-  while (c->key_bits < 32 && ((uint64_t)1 << c->key_bits) < (uint64_t)c->cells) c->key_bits++;
   derive(c);
   return ctx_allocate(c, max_particles, out);
 }
@@ -426,8 +429,6 @@ extern "C" int sph_create_batch(const sph_params *params, int nscenes, const sph
   c->P = *params;
   c->box = sph_aabb{0.0, ext[0], 0.0, ext[1], 0.0, ext[2]};
   c->cells = (uint32_t)cells;
-  c->key_bits = 1;
-  while (c->key_bits < 32 && ((uint64_t)1 << c->key_bits) < cells) c->key_bits++;
   c->dev.nx = c->dev.ny = c->dev.nz = c->dev.nxy = 1;  // per scene instead
   derive(c);
   rc = ctx_allocate(c, (int)total, out);
@@ -715,8 +716,6 @@ extern "C" int sph_predict_positions(sph_ctx *c) {
 extern "C" int sph_find_all_neighbors(sph_ctx *c) {
   int rc = require_state(c);
   if (rc) return rc;
-  rc = launch_substep_init(c);
-  if (rc) return rc;
   c->staged_slot = 0;
   return launch_neighbor_search(c, false);
 }
@@ -811,9 +810,7 @@ extern "C" int sph_update_positions(sph_ctx *c) {
 // --------------------------------------------------------------------------
 // Device work of one fused substep, all on the context stream (capturable).
 static int substep_launch(sph_ctx *c, bool *warm_out) {
-  int rc = launch_substep_init(c);
-  if (rc) return rc;
-  rc = launch_neighbor_search(c, true);
+  int rc = launch_neighbor_search(c, true);
   if (rc) return rc;
   const int iters = c->P.solve_iterations;
   // Logged or warm-started solve: the first iteration's lambda pass also
@@ -898,8 +895,7 @@ static int capture_substep(sph_ctx *c) {
     return hip_fail(ei, "hipGraphInstantiate");
   }
   c->graph = g;
-  c->graph_after = {c->pos, c->vel, c->key_s, c->id_s, c->pair_blocks,
-                    c->last_err_slot, warm};
+  c->graph_after = {c->pos, c->vel, c->pair_blocks, c->last_err_slot, warm};
   c->graph_valid = true;
   return SPH_OK;
 }
@@ -909,8 +905,6 @@ static int substep_graph(sph_ctx *c) {
   const auto &a = c->graph_after;
   c->pos = a.pos;
   c->vel = a.vel;
-  c->key_s = a.key_s;
-  c->id_s = a.id_s;
   c->pair_blocks = a.pair_blocks;
   c->last_err_slot = a.last_err_slot;
   c->sorted_valid = c->lists_valid = true;

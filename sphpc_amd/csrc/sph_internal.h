@@ -135,11 +135,13 @@ struct MlpPacked {
   float b3;
 };
 
+// The order is that of sph_profile_kernel_name and of saved tunings; the two
+// radix entries stay for it (the search has counted by cell since).
 enum KernelId {
   K_PREDICT_HASH = 0, K_HASH, K_GRAVITY, K_PREDICT, K_RADIX_UP, K_RADIX_DOWN, K_SCAN,
   K_REORDER, K_BUILD_LISTS, K_DENSITY_LAMBDA, K_DENSITY, K_LAMBDA, K_DP, K_DP_UPDATE,
   K_POS_STARS, K_VELOCITY, K_COLOR, K_SURFACE, K_XSPH, K_VORTICITY, K_CONFINE, K_COMMIT,
-  K_AUX, K_WARM_LAMBDA, K_COLLIDE, K_LAMBDA_COPY, K_COUNT
+  K_AUX, K_WARM_LAMBDA, K_COLLIDE, K_LAMBDA_COPY, K_PLACE, K_COUNT
 };
 
 struct ScanScratch {
@@ -168,20 +170,18 @@ struct sph_ctx {
   float *sdf_buf = nullptr;
 
   uint32_t cells = 0;
-  int key_bits = 1;
   int cap = 0;
   int n = 0;
 
   // canonical (particle-id order) state
   float4 *x_can = nullptr, *v_can = nullptr, *xs_can = nullptr;
-  // sort
-  uint32_t *keys = nullptr, *keys_alt = nullptr, *ids = nullptr, *ids_alt = nullptr;
-  uint32_t *hist = nullptr;
-  size_t hist_cap = 0;
-  const uint32_t *key_s = nullptr, *id_s = nullptr;  // final sorted buffers
-  // cells + 1 entries; cell_end holds the run ends of the sorted keys, zero
-  // between searches
-  uint32_t *cell_end = nullptr, *cell_start = nullptr;
+  // counting sort by cell: each particle's cell key and its place among the
+  // cell's particles as they were counted (id order), then (id, key) by place
+  uint32_t *keys = nullptr, *cell_rank = nullptr;
+  uint2 *slots = nullptr;
+  uint32_t *key_s = nullptr, *id_s = nullptr;  // (key, id) in sorted order
+  // cells + 1 entries; cell_count is zero between searches
+  uint32_t *cell_count = nullptr, *cell_start = nullptr;
   sph::ScanScratch scan;
   // sorted working set
   float4 *pos_a = nullptr, *pos_b = nullptr, *pos = nullptr;  // pos: current x*
@@ -243,7 +243,6 @@ struct sph_ctx {
   hipGraphExec_t graph_exec = nullptr;
   struct {
     float4 *pos, *vel;
-    const uint32_t *key_s, *id_s;
     uint32_t pair_blocks;
     int last_err_slot;
     bool warm;
@@ -280,13 +279,17 @@ inline uint32_t blocks_for(uint32_t n, uint32_t per = kBlock) { return (n + per 
 void prof_begin(sph_ctx *c, int kernel, hipEvent_t *a);
 void prof_end(sph_ctx *c, int kernel, hipEvent_t a);
 
-// Sort / scan (sph_sort.hip).  out[i] = in[0] + ... + in[i-1] (max_op: the
-// maximum of those, 0 for none); write_total also sets out[len].
-int exclusive_scan(uint32_t *in, uint32_t *out, uint32_t len, bool zero_in, bool write_total,
-                   ScanScratch *scratch, hipStream_t s, sph_ctx *prof, bool max_op = false);
+// Words of scan scratch for `len` entries.
+constexpr uint32_t kScanTile = 4096;
+inline size_t scan_tiles(size_t len) { return (len + kScanTile - 1) / kScanTile + 1; }
+
+// Sort / scan (sph_sort.hip).  out[i] = in[0] + ... + in[i-1] (inclusive: + in[i]);
+// write_total also sets out[len].
+int scan(const uint32_t *in, uint32_t *out, uint32_t len, bool inclusive, bool write_total,
+         ScanScratch *scratch, hipStream_t s, sph_ctx *prof);
 int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uint32_t *v0,
                      uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t **hist,
-                     size_t *hist_cap, ScanScratch *scratch, hipStream_t s, sph_ctx *prof,
+                     size_t *hist_cap, ScanScratch *scratch, hipStream_t s,
                      const uint32_t **kout, const uint32_t **vout);
 int count_keys(const uint32_t *keys, uint32_t n, uint32_t *count, uint32_t cells,
                hipStream_t s);
@@ -311,7 +314,6 @@ int launch_xsph(sph_ctx *c);
 int launch_vorticity(sph_ctx *c);
 int launch_confine(sph_ctx *c, bool commit);
 int launch_commit(sph_ctx *c);
-int launch_substep_init(sph_ctx *c);
 int launch_collide_soa(float *x, float *y, float *z, uint32_t n, const SdfDev &o,
                        hipStream_t s);
 int launch_collide_soa_f64(double *x, double *y, double *z, uint32_t n, const SdfDev &o,

@@ -23,45 +23,36 @@ constexpr int RS_WAVES = RS_THREADS / 64;
 constexpr int SC_THREADS = 256;
 constexpr int SC_ITEMS = 16;
 constexpr int SC_TILE = SC_THREADS * SC_ITEMS;
+static_assert(SC_TILE == kScanTile, "scratch sized by scan_tiles");
 
-// Scan operators (identity 0 for both: the values are unsigned).
-struct OpAdd {
-  static __device__ __forceinline__ uint32_t f(uint32_t a, uint32_t b) { return a + b; }
-};
-struct OpMax {
-  static __device__ __forceinline__ uint32_t f(uint32_t a, uint32_t b) { return max(a, b); }
-};
-
-template <class Op = OpAdd>
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x = Op::f(x, y);
+    if (lane >= o) x += y;
   }
   return x;
 }
 
 // Exclusive scan over a 256-thread block; *tot receives the block total.
-template <class Op = OpAdd>
 __device__ __forceinline__ uint32_t block_excl_scan_256(uint32_t x, uint32_t *wtot,
                                                         uint32_t *tot) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint32_t inc = wave_incl_scan<Op>(x);
+  const uint32_t inc = wave_incl_scan(x);
   if (lane == 63) wtot[w] = inc;
   __syncthreads();
   uint32_t pre = 0, all = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t t = wtot[i];
-    if (i < w) pre = Op::f(pre, t);
-    all = Op::f(all, t);
+    if (i < w) pre += t;
+    all += t;
   }
   __syncthreads();
   *tot = all;
   const uint32_t before = __shfl_up(inc, 1, 64);
-  return Op::f(pre, lane ? before : 0u);
+  return pre + (lane ? before : 0u);
 }
 
 // Lanes of the wave holding the same 8-bit digit (valid lanes only).
@@ -104,7 +95,6 @@ __device__ __forceinline__ void load_items(const uint32_t *in, uint32_t i0, uint
   }
 }
 
-template <class Op>
 __global__ __launch_bounds__(SC_THREADS) void k_scan_tile_sums(const uint32_t *__restrict__ in,
                                                                uint32_t len,
                                                                uint32_t *__restrict__ sums) {
@@ -113,13 +103,12 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_tile_sums(const uint32_t *_
   load_items(in, blockIdx.x * SC_TILE + threadIdx.x * SC_ITEMS, len, x);
   uint32_t s = 0;
 #pragma unroll
-  for (int r = 0; r < SC_ITEMS; ++r) s = Op::f(s, x[r]);
+  for (int r = 0; r < SC_ITEMS; ++r) s += x[r];
   uint32_t tot;
-  block_excl_scan_256<Op>(s, wtot, &tot);
+  block_excl_scan_256(s, wtot, &tot);
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-template <class Op>
 __global__ __launch_bounds__(SC_THREADS) void k_scan_spine(uint32_t *sums, uint32_t tiles) {
   __shared__ uint32_t wtot[4];
   uint32_t carry = 0;
@@ -127,50 +116,72 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_spine(uint32_t *sums, uint3
     const uint32_t i = base + threadIdx.x;
     const uint32_t x = i < tiles ? sums[i] : 0u;
     uint32_t tot;
-    const uint32_t e = block_excl_scan_256<Op>(x, wtot, &tot);
-    if (i < tiles) sums[i] = Op::f(carry, e);
-    carry = Op::f(carry, tot);
+    const uint32_t e = block_excl_scan_256(x, wtot, &tot);
+    if (i < tiles) sums[i] = carry + e;
+    carry += tot;
   }
 }
 
-// in and out may alias (in-place scan).
-template <class Op>
-__global__ __launch_bounds__(SC_THREADS) void k_scan_apply(uint32_t *in, uint32_t *out,
+// Where a tile takes the sum of the tiles before it from.
+enum ScanFrom {
+  SCAN_INPUT,  // the input itself (up to kScanSelfTiles tiles: no other launch)
+  SCAN_SUMS,   // the tiles' sums (up to kScanSumTiles tiles)
+  SCAN_SPINE   // their exclusive scan
+};
+// One launch costs 4-5 us of a small substep (kernel and gap), and reading up
+// to 7 tiles (28,672 words, all of L2) again costs less; a block reads 2048
+// sums in 8 loads per thread, less than the spine's launch.
+constexpr uint32_t kScanSelfTiles = 8, kScanSumTiles = 2048;
+
+// in and out may alias with SCAN_SUMS and SCAN_SPINE (in-place scan).
+template <ScanFrom FROM>
+__global__ __launch_bounds__(SC_THREADS) void k_scan_apply(const uint32_t *in, uint32_t *out,
                                                            uint32_t len,
                                                            const uint32_t *__restrict__ sums,
-                                                           int zero_in, int write_total) {
+                                                           int inclusive, int write_total) {
   __shared__ uint32_t wtot[4];
   const uint32_t i0 = blockIdx.x * SC_TILE + threadIdx.x * SC_ITEMS;
   uint32_t x[SC_ITEMS];
   load_items(in, i0, len, x);
+  uint32_t before = 0;
+  if (FROM == SCAN_SPINE) {
+    before = sums[blockIdx.x];
+  } else {
+    uint32_t own = 0;
+    if (FROM == SCAN_SUMS) {
+      for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SC_THREADS) own += sums[t];
+    } else {
+      for (uint32_t t = 0; t < blockIdx.x; ++t) {
+        const uint4 *v = reinterpret_cast<const uint4 *>(in + t * SC_TILE) + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < SC_ITEMS / 4; ++q) {
+          const uint4 a = v[q * SC_THREADS];
+          own += (a.x + a.y) + (a.z + a.w);
+        }
+      }
+    }
+    block_excl_scan_256(own, wtot, &before);
+  }
   uint32_t own = 0;
 #pragma unroll
-  for (int r = 0; r < SC_ITEMS; ++r) own = Op::f(own, x[r]);
+  for (int r = 0; r < SC_ITEMS; ++r) own += x[r];
   uint32_t tot;
-  uint32_t run = Op::f(sums[blockIdx.x], block_excl_scan_256<Op>(own, wtot, &tot));
+  uint32_t run = before + block_excl_scan_256(own, wtot, &tot);
 #pragma unroll
   for (int r = 0; r < SC_ITEMS; ++r) {
     const uint32_t e = run;
-    run = Op::f(run, x[r]);
-    x[r] = e;
+    run += x[r];
+    x[r] = inclusive ? run : e;
   }
-  if (i0 + SC_ITEMS <= len) {
+  if (i0 + SC_ITEMS <= len && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
     uint4 *o = reinterpret_cast<uint4 *>(out + i0);
 #pragma unroll
     for (int q = 0; q < SC_ITEMS / 4; ++q)
       o[q] = make_uint4(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
-    if (zero_in) {
-      uint4 *z = reinterpret_cast<uint4 *>(in + i0);
-#pragma unroll
-      for (int q = 0; q < SC_ITEMS / 4; ++q) z[q] = make_uint4(0u, 0u, 0u, 0u);
-    }
   } else {
 #pragma unroll
     for (int r = 0; r < SC_ITEMS; ++r)
-      if (i0 + r < len) {
-        out[i0 + r] = x[r];
-        if (zero_in) in[i0 + r] = 0u;
-      }
+      if (i0 + r < len) out[i0 + r] = x[r];
   }
   // the thread holding entry len-1 writes the total after it
   if (write_total && i0 < len && len <= i0 + SC_ITEMS) out[len] = run;
@@ -181,8 +192,8 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, uint32_t len) {
   if (i < len) p[i] = v;
 }
 
-int exclusive_scan(uint32_t *in, uint32_t *out, uint32_t len, bool zero_in, bool write_total,
-                   ScanScratch *sc, hipStream_t s, sph_ctx *prof, bool max_op) {
+int scan(const uint32_t *in, uint32_t *out, uint32_t len, bool inclusive, bool write_total,
+         ScanScratch *sc, hipStream_t s, sph_ctx *prof) {
   if (len == 0) {
     if (write_total) {
       k_fill_u32<<<1, 64, 0, s>>>(out, 0u, 1u);
@@ -190,29 +201,33 @@ int exclusive_scan(uint32_t *in, uint32_t *out, uint32_t len, bool zero_in, bool
     }
     return SPH_OK;
   }
-  if (((uintptr_t)in | (uintptr_t)out) & 15u) {
-    set_error("exclusive_scan: buffers must be 16-byte aligned");
+  if ((uintptr_t)in & 15u) {
+    set_error("scan: the input must be 16-byte aligned");
     return SPH_ERR_ARG;
   }
   const uint32_t tiles = (len + SC_TILE - 1) / SC_TILE;
-  if (sc->tile_cap < tiles) {
+  const bool self = tiles <= kScanSelfTiles && in != out;
+  if (!self && sc->tile_cap < tiles) {
     if (sc->tile_sums) SPH_HIP(hipFree(sc->tile_sums));
     sc->tile_sums = nullptr;
     SPH_HIP(hipMalloc(&sc->tile_sums, sizeof(uint32_t) * tiles));
     sc->tile_cap = tiles;
   }
+  const int incl = inclusive ? 1 : 0, total = write_total ? 1 : 0;
   hipEvent_t ev = nullptr;
   if (prof) prof_begin(prof, K_SCAN, &ev);
-  if (max_op) {
-    k_scan_tile_sums<OpMax><<<tiles, SC_THREADS, 0, s>>>(in, len, sc->tile_sums);
-    k_scan_spine<OpMax><<<1, SC_THREADS, 0, s>>>(sc->tile_sums, tiles);
-    k_scan_apply<OpMax><<<tiles, SC_THREADS, 0, s>>>(in, out, len, sc->tile_sums,
-                                                     zero_in ? 1 : 0, write_total ? 1 : 0);
+  if (self) {
+    k_scan_apply<SCAN_INPUT><<<tiles, SC_THREADS, 0, s>>>(in, out, len, nullptr, incl, total);
   } else {
-    k_scan_tile_sums<OpAdd><<<tiles, SC_THREADS, 0, s>>>(in, len, sc->tile_sums);
-    k_scan_spine<OpAdd><<<1, SC_THREADS, 0, s>>>(sc->tile_sums, tiles);
-    k_scan_apply<OpAdd><<<tiles, SC_THREADS, 0, s>>>(in, out, len, sc->tile_sums,
-                                                     zero_in ? 1 : 0, write_total ? 1 : 0);
+    k_scan_tile_sums<<<tiles, SC_THREADS, 0, s>>>(in, len, sc->tile_sums);
+    if (tiles <= kScanSumTiles) {
+      k_scan_apply<SCAN_SUMS><<<tiles, SC_THREADS, 0, s>>>(in, out, len, sc->tile_sums, incl,
+                                                           total);
+    } else {
+      k_scan_spine<<<1, SC_THREADS, 0, s>>>(sc->tile_sums, tiles);
+      k_scan_apply<SCAN_SPINE><<<tiles, SC_THREADS, 0, s>>>(in, out, len, sc->tile_sums, incl,
+                                                            total);
+    }
   }
   if (prof) prof_end(prof, K_SCAN, ev);
   SPH_HIP(hipGetLastError());
@@ -331,7 +346,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_downsweep(
 
 int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uint32_t *v0,
                      uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t **hist,
-                     size_t *hist_cap, ScanScratch *sc, hipStream_t s, sph_ctx *prof,
+                     size_t *hist_cap, ScanScratch *sc, hipStream_t s,
                      const uint32_t **kout, const uint32_t **vout) {
   *kout = kin;
   *vout = vin;
@@ -350,16 +365,11 @@ int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uin
     uint32_t *ok = (p & 1) ? k1 : k0;
     uint32_t *ov = (p & 1) ? v1 : v0;
     const int shift = 8 * p;
-    hipEvent_t ev = nullptr;
-    if (prof) prof_begin(prof, K_RADIX_UP, &ev);
     k_radix_upsweep<<<tiles, RS_THREADS, 0, s>>>(ck, n, shift, *hist, tiles);
-    if (prof) prof_end(prof, K_RADIX_UP, ev);
     SPH_HIP(hipGetLastError());
-    int rc = exclusive_scan(*hist, *hist, (uint32_t)need, false, false, sc, s, prof);
+    int rc = scan(*hist, *hist, (uint32_t)need, false, false, sc, s, nullptr);
     if (rc) return rc;
-    if (prof) prof_begin(prof, K_RADIX_DOWN, &ev);
     k_radix_downsweep<<<tiles, RS_THREADS, 0, s>>>(ck, cv, ok, ov, n, shift, *hist, tiles);
-    if (prof) prof_end(prof, K_RADIX_DOWN, ev);
     SPH_HIP(hipGetLastError());
     ck = ok;
     cv = ov;
@@ -480,7 +490,7 @@ static int sort_impl(uint32_t *keys, uint32_t *values, int n, int key_bits, void
   }
   const uint32_t *kout = nullptr, *vout = nullptr;
   rc = radix_sort_pairs(keys, values, w->a, w->b, keys, values, (uint32_t)n, key_bits, &w->hist,
-                        &w->hist_cap, &w->sc, s, nullptr, &kout, &vout);
+                        &w->hist_cap, &w->sc, s, &kout, &vout);
   if (rc == SPH_OK && kout != keys) {
     hipError_t e =
         hipMemcpyAsync(keys, kout, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, s);
@@ -575,7 +585,7 @@ extern "C" int sph_sort_by_key_bits_noalloc(uint32_t *keys, uint32_t *values, in
   sc.tile_cap = kStaticScanTiles;
   const uint32_t *kout = nullptr, *vout = nullptr;
   rc = radix_sort_pairs(keys, values, a, b, keys, values, (uint32_t)n, key_bits, &hist,
-                        &hist_cap, &sc, s, nullptr, &kout, &vout);
+                        &hist_cap, &sc, s, &kout, &vout);
   if (rc) return rc;
   if (kout != keys) {  // an odd number of passes ends in the scratch buffers
     SPH_HIP(hipMemcpyAsync(keys, kout, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice,
@@ -602,7 +612,7 @@ static int bounds_impl(const uint32_t *keys, int n, int cells, uint32_t *out, vo
   uint32_t *count = w->a, *start = w->b;
   rc = count_keys(keys, (uint32_t)n, count, (uint32_t)cells, s);
   if (rc == SPH_OK)
-    rc = exclusive_scan(count, start, (uint32_t)cells, false, true, &w->sc, s, nullptr);
+    rc = scan(count, start, (uint32_t)cells, false, true, &w->sc, s, nullptr);
   if (rc == SPH_OK) {
     const hipError_t e = hipMemcpyAsync(out, start + (upper ? 1 : 0),
                                         sizeof(uint32_t) * (size_t)cells,

@@ -69,6 +69,14 @@ def test_cell_bounds_bit_exact(n, cells):
     assert np.array_equal(hi, np.searchsorted(keys, c, "right"))
 
 
+@pytest.mark.parametrize("cells", [4095, 4096, 4097, 8 * 4096, 8 * 4096 + 1, 2048 * 4096,
+                                   2048 * 4096 + 1])
+def test_cell_bounds_at_the_edges_of_the_scan(cells):
+    """The scan's tiles of 4096 cells and its two limits: up to 8 tiles sum the
+    input itself, up to 2048 the tiles' sums."""
+    test_cell_bounds_bit_exact(20_000, cells)
+
+
 # ---------------------------------------------------------------------------
 # Neighbour search in the staged pipeline (neighbors.c:68-298)
 # ---------------------------------------------------------------------------
@@ -125,6 +133,34 @@ def test_neighbor_search_bit_exact(spread, seed, wide):
     assert st_gpu.cell_clamps == 0
     if spread < 1.0:
         assert cnt.max() == orc.MAXN and ol["dropped"] > 0
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 10007])
+@pytest.mark.parametrize("cells_used", [1, 3, 4000])
+def test_counting_sort_of_scattered_ids(n, cells_used):
+    """Stable order whatever the order the counts were taken in: ids scattered
+    over few and many cells, whole wavefronts and partial ones."""
+    s = 0.02
+    sc = Scene(s, (1.0, 0.8, 0.6))
+    rng = np.random.default_rng(n + cells_used)
+    corner = rng.integers(0, 15, (cells_used, 3)) * sc.h
+    pos = (corner[rng.integers(0, cells_used, n)] + rng.uniform(0.1, 0.9, (n, 3)) * sc.h)
+    pos = pos.astype(np.float32)
+    with sc.context(n) as ctx:
+        ctx.upload(pos)
+        for _ in range(2):  # the second search finds the counts zero again
+            ctx.predict_positions()
+            ctx.find_all_neighbors()
+            xs, ys, zs = _soa(ctx.field(sa.FIELD_POSITION_STAR))
+            keys = np.zeros(n, np.uint32)
+            L.orc_hash_particles(n, xs, ys, zs, C.byref(sc.o), keys, np.zeros(n, np.uint32))
+            order = np.argsort(keys, kind="stable").astype(np.uint32)
+            k, i = ctx.sorted_pairs()
+            assert np.array_equal(i, order) and np.array_equal(k, keys[order])
+            st, en = ctx.cell_bounds()
+            c = np.arange(len(st))
+            assert np.array_equal(st, np.searchsorted(k, c, "left"))
+            assert np.array_equal(en, np.searchsorted(k, c, "right"))
 
 
 def test_cell_tables_at_the_grid_ends_and_a_crowded_cell():
