@@ -756,6 +756,171 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
   block_sum_to(pair_partial, (uint32_t)c);
 }
 
+// The same lists with several wavefronts per 64-particle group, each walking
+// ROWS of a particle's nine (dz, dy) rows (one row, or a dz layer's three): the
+// waves count their hits side by side, take their places in the list from the
+// counts of the waves before them, and write the group's quads out of one LDS
+// buffer.  For the sizes at which k_build_lists leaves the chip idle and its
+// time is one wave's walk through nine rows in turn, about 20 us whatever the
+// size; with more particles the particle's set-up made several times over costs
+// more than the shorter walk gives.  Measured (us, events included), k_build_lists
+// / three waves a group / nine: 4k particles 23.0 / 13.5 / 9.2, 33k 23.9 / 14.9 /
+// 11.6, 47k 24.8 / 16.1 / 16.9, 133k 30.9 / 26.1 / 36.7, 185k 32.4 / 32.2 / 47.6,
+// 262k 38.3 / 39.9 / 63.9, 8.4M (no events) 871 / 902 / 1833.
+constexpr uint32_t kOneRowBuildMax = 40960, kRowBuildMax = 196608;
+
+template <bool BATCH, int ROWS>
+__global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
+    uint32_t n, const float4 *__restrict__ pos, const float *__restrict__ sx, uint32_t stride,
+    const uint32_t *__restrict__ key_s, const uint32_t *__restrict__ cstart, DevParams P,
+    uint32_t *__restrict__ list, uint4 *__restrict__ head, uint32_t *__restrict__ stats,
+    uint32_t *__restrict__ pair_partial, int force_wide, BatchDev B) {
+  constexpr int WAVES = 9 / ROWS;
+  __shared__ uint16_t hits[kMaxNb][kWave];  // offsets from the layer's first candidate
+  __shared__ uint32_t count[WAVES][kWave], layer[3][kWave];
+  const uint32_t lane = threadIdx.x & 63u;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t group = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t s = group * kWave + lane;
+  const int l = wave * ROWS / 3;                      // dz layer of this wave
+  const int dz = l - 1, dy0 = wave * ROWS - 3 * l - 1;  // its first row
+  uint32_t j0[ROWS], j1[ROWS], base = s;
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) j0[k] = j1[k] = 0u;
+  float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  bool direct = force_wide != 0;
+  if (s < n) {
+    p = pos[s];
+    const Geo G = geo_of<BATCH>(s, P, B);
+    const uint32_t key = key_s[s] - G.base;
+    const uint32_t cz = key / G.nxy;
+    const uint32_t rem = key - cz * G.nxy;
+    const uint32_t cy = rem / G.nx;
+    const uint32_t cx = rem - cy * G.nx;
+    const uint32_t x0 = cx > 0 ? cx - 1 : 0;
+    const uint32_t x1 = cx + 1 < G.nx ? cx + 1 : G.nx - 1;
+    const int z = (int)cz + dz;
+    if (z >= 0 && z < (int)G.nz) {
+      const uint32_t zrow = G.base + (uint32_t)z * G.nxy;
+      const uint32_t y0 = cy > 0 ? cy - 1 : 0;
+      const uint32_t y1 = cy + 1 < G.ny ? cy + 1 : G.ny - 1;
+      const uint32_t first = cstart[zrow + y0 * G.nx + x0];
+      const uint32_t span = cstart[zrow + y1 * G.nx + x1 + 1] - first;
+#pragma unroll
+      for (int k = 0; k < ROWS; ++k) {
+        const int y = (int)cy + dy0 + k;
+        const bool in = y >= 0 && y < (int)G.ny;
+        const uint32_t r = zrow + (in ? (uint32_t)y : cy) * G.nx;
+        j0[k] = cstart[r + x0];
+        j1[k] = cstart[r + x1 + 1];
+        if (!in) j1[k] = j0[k];
+      }
+      if (span > 0u) base = first;
+      if (span > kCompactSpan) direct = true;
+    }
+  }
+  // hits of the up to 32 candidates [cb, end) as a mask
+  auto test = [&](uint32_t cb, uint32_t end) {
+    const uint32_t len = end - cb;
+    uint32_t lo = 0u, hi = 0u;  // bits: r2 < h2_lo, r2 < h2_hi (as in k_build_lists)
+#pragma unroll
+    for (int g = 3; g >= 0; --g) {
+      if (8u * g < len) {
+        const float *X = sx + cb + 8 * g;
+        const f4u x0 = ld4u(X), x1 = ld4u(X + 4);
+        const f4u y0 = ld4u(X + stride), y1 = ld4u(X + stride + 4);
+        const f4u z0 = ld4u(X + 2u * stride), z1 = ld4u(X + 2u * stride + 4);
+        const float qx[kBatch] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        const float qy[kBatch] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+        const float qz[kBatch] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
+#pragma unroll
+        for (int t = kBatch - 1; t >= 0; --t) {
+          const float r2 = sq3(p.x - qx[t], p.y - qy[t], p.z - qz[t]);
+          candidate_bits(lo, hi, r2, P.h2_lo, P.h2_hi);
+        }
+      }
+    }
+    uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
+    if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
+    lo &= keep;
+    uint32_t band = hi & keep & ~lo;
+    while (band) {
+      const int t = __builtin_ctz(band);
+      band &= band - 1u;
+      const float4 q = pos[cb + t];
+      if (inside_exact(p.x, p.y, p.z, q.x, q.y, q.z, P.h2d)) lo |= 1u << t;
+    }
+    return lo;
+  };
+  // a row's first mask is kept, later ones (rows of more than 32, in compressed
+  // fluid) are made again when the hits are stored
+  uint32_t m0[ROWS], mine = 0u;
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    m0[k] = 0u;
+    for (uint32_t cb = j0[k]; cb < j1[k]; cb += 32u) {
+      const uint32_t m = test(cb, j1[k]);
+      mine += (uint32_t)__builtin_popcount(m);
+      if (cb == j0[k]) m0[k] = m;
+    }
+  }
+  count[wave][lane] = mine;
+  if (wave * ROWS == 3 * l) layer[l][lane] = base;
+  const bool wide = __syncthreads_or(direct ? 1 : 0) != 0;
+  uint32_t at = 0u, all = 0u, c1 = 0u, c2 = 0u;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    if (w == wave) at = all;
+    if (w == 3 / ROWS) c1 = all;
+    if (w == 6 / ROWS) c2 = all;
+    all += count[w][lane];
+  }
+  uint32_t *out = list + (size_t)group * kListStride + lane * 4u;
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    for (uint32_t cb = j0[k]; cb < j1[k] && at < (uint32_t)kMaxNb; cb += 32u) {
+      uint32_t m = cb == j0[k] ? m0[k] : test(cb, j1[k]);
+      while (m && at < (uint32_t)kMaxNb) {
+        const uint32_t j = cb + (uint32_t)__builtin_ctz(m);
+        m &= m - 1u;
+        if (wide)
+          out[(size_t)(at >> 2) * kQuadStride + (at & 3u)] = j;
+        else
+          hits[at][lane] = (uint16_t)(j - base);
+        ++at;
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t c = min(all, (uint32_t)kMaxNb);
+  for (uint32_t q = wave; !wide && 8u * q < (uint32_t)kMaxNb; q += WAVES) {
+    const uint32_t k = 8u * q;
+    if (k < c) {
+      uint32_t w[4];
+#pragma unroll
+      for (uint32_t t = 0; t < 4; ++t) {
+        const uint32_t lo = k + 2 * t < c ? hits[k + 2 * t][lane] : 0u;
+        const uint32_t hi = k + 2 * t + 1 < c ? hits[k + 2 * t + 1][lane] : 0u;
+        w[t] = lo | (hi << 16);
+      }
+      *reinterpret_cast<uint4 *>(out + (size_t)q * kQuadStride) =
+          make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+  if (wave == WAVES - 1) {
+    c1 = min(c1, (uint32_t)kMaxNb);
+    c2 = min(c2, (uint32_t)kMaxNb);
+    if (s < n)
+      head[s] = make_uint4(layer[0][lane], layer[1][lane], layer[2][lane],
+                           c | (c1 << 8) | (c2 << 16) | (wide ? kHeadWide : 0u));
+    add_counter64_wave(stats, STAT_DROPPED, all - c);
+    uint32_t t = c;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o, 64);
+    if (lane == 0) pair_partial[blockIdx.x] = t;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Jacobi constraint loop
 // ---------------------------------------------------------------------------
@@ -1747,21 +1912,36 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
     SPH_HIP(hipGetLastError());
   }
   if (n) {
-    const uint32_t bs = tuned_block(c, K_BUILD_LISTS);
-    const uint32_t nb = blocks_for(n, bs);
-    if (c->nscenes)
-      LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
-                   k_build_lists<true><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
-                       n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
-                       c->list, c->list_head, c->stats, c->pair_partial,
-                       c->tune.wide_lists ? 1 : 0, B));
-    else
-      LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
-                   k_build_lists<false><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
-                       n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
-                       c->list, c->list_head, c->stats, c->pair_partial,
-                       c->tune.wide_lists ? 1 : 0, B));
-    c->pair_blocks = nb;
+    const int wide = c->tune.wide_lists ? 1 : 0;
+    if (n <= kRowBuildMax) {
+      const uint32_t groups = blocks_for(n, kWave);
+#define BUILD_ROWS(BAT, ROWS)                                                                  \
+  LAUNCH_TIMED(c, K_BUILD_LISTS, 0,                                                            \
+               (k_build_rows<BAT, ROWS><<<groups, 9 / ROWS * kWave, 0, s>>>(                   \
+                   n, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev, c->list,  \
+                   c->list_head, c->stats, c->pair_partial, wide, B)))
+      if (n <= kOneRowBuildMax) {
+        if (c->nscenes) BUILD_ROWS(true, 1); else BUILD_ROWS(false, 1);
+      } else {
+        if (c->nscenes) BUILD_ROWS(true, 3); else BUILD_ROWS(false, 3);
+      }
+#undef BUILD_ROWS
+      c->pair_blocks = groups;
+    } else {
+      const uint32_t bs = tuned_block(c, K_BUILD_LISTS);
+      const uint32_t nb = blocks_for(n, bs);
+      if (c->nscenes)
+        LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
+                     k_build_lists<true><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
+                         n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
+                         c->list, c->list_head, c->stats, c->pair_partial, wide, B));
+      else
+        LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
+                     k_build_lists<false><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
+                         n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
+                         c->list, c->list_head, c->stats, c->pair_partial, wide, B));
+      c->pair_blocks = nb;
+    }
     SPH_HIP(hipGetLastError());
   }
   c->vel = c->vel_a;

@@ -163,6 +163,27 @@ def test_counting_sort_of_scattered_ids(n, cells_used):
             assert np.array_equal(en, np.searchsorted(k, c, "right"))
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (13, 5, 1), (34, 34, 35), (35, 35, 34),
+                                  (58, 58, 58), (59, 59, 59)])
+def test_lists_on_both_sides_of_the_build_kernels_limits(dims, wide):
+    """One wave per row up to 40,960 particles, one per dz layer up to 196,608,
+    one per 64 particles above; compressed, so that rows hold more than 32
+    candidates and lists reach the cap, and with a ragged last group."""
+    sc, pos, vel = _scene_dam_block(n=dims, spread=0.5, seed=3)
+    ctx = _staged_search(sc, pos, vel, wide)
+    n = len(pos)
+    ol = oracle_lists(sc.o, *_soa(ctx.field(sa.FIELD_POSITION_STAR)))
+    ids, cnt = ctx.neighbors()
+    assert np.array_equal(cnt, ol["cnt"])
+    mask = np.arange(orc.MAXN)[None, :] < cnt[:, None]
+    assert np.array_equal(ids.reshape(n, -1)[mask], ol["nbr"].reshape(n, -1)[mask])
+    st = ctx.stats()
+    assert st.neighbor_overflow == ol["dropped"] and st.neighbor_pairs == cnt.sum()
+    if n > 1000:
+        assert cnt.max() == orc.MAXN and ol["dropped"] > 0
+
+
 def test_cell_tables_at_the_grid_ends_and_a_crowded_cell():
     """Cell tables from the sorted keys' run ends: runs in the first and the
     last cell of the grid, particles clamped onto the box faces from outside,
