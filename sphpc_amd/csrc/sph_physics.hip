@@ -64,26 +64,39 @@ __device__ __forceinline__ NbList nb_list(const uint32_t *list, const uint4 *hea
 }
 
 // Launch bounds of the delta-p, density, colour and confinement kernels: at
-// up to 16 gathers in flight at most 128 VGPRs, i.e. 4 waves per SIMD.  With
-// 64-bit gather addresses delta p took 139 VGPRs (3 waves) and the bound made
-// it 7% faster at 8M particles despite a few spilled registers (colour and
-// confinement, at 138-140, were 1-4% slower with it).  With the buffer gathers
-// below delta p spills 20 bytes under the bound, and colour and confinement
-// (130-133 VGPRs without it) 12-16 bytes, and run 2-3% faster than at 3 waves.
-// Five waves (96 VGPRs) would spill 164-220 bytes per lane.
+// up to 16 gathers in flight at most 128 VGPRs, i.e. 4 waves per SIMD, which all
+// of them meet without spilling (at 3 waves delta p measured 7% slower, colour
+// and confinement 2-3%).  Five waves (96 VGPRs) would spill 164-220 bytes.
 #define GATHER_BOUNDS(NB) __launch_bounds__(kBlock, (NB) <= 16 ? 4 : 1)
 
-// Visits the c neighbours of a particle in list order, NB at a time: first the
-// batch's list quads, then its NB dependent gathers, then the arithmetic.  The
-// gathers are latency-bound, so the depth NB (gathers in flight per wave) sets
-// the speed: 16 was 13-22% faster than 8 in every gather pass on MI355X; the
-// autotuner chooses 8, 16 or 32 per kernel.  With PREFETCH the list quads of
-// batch k+1 are issued right after the gathers of batch k, so a batch costs
-// one memory round trip instead of two; that pays for 16-byte gathers, and of
-// the 32-byte (Pair4) ones only in the XSPH pass.  Slots past c are never used; their gathers
-// load a valid index (the particle itself in a wide list, the layer-2 base in
-// a compact one, which the build sets to the particle itself when that layer
-// has no candidates).
+// Visits the c neighbours of a particle in list order, NB at a time: the
+// batch's list quads (raw, as stored), their decoding to indices, the NB gathers
+// in one burst, then the arithmetic.  NB gathers in flight per wave: 16 was
+// 13-22% faster than 8 in every gather pass on MI355X; the autotuner chooses 8,
+// 16 or 32 per kernel.
+//
+// What bounds it: the vector L1's return path is 93-96% busy in every pass.  A
+// gather of 16-byte records costs it 1, 1.5 or 2.3 cycles per four lanes whose
+// records lie in 1, 2 or 4 cache lines (16, 24, 38 cycles per wave, measured on a
+// resident window), and here four neighbouring lanes touch three lines on
+// average, 31 cycles; the 16-byte passes are at the same time 80-90% VALU-busy.
+//
+// The first batch's quads are loaded together with the particle and its head
+// (their place does not depend on it), which takes one memory round trip off
+// every pass.  With PREFETCH the quads of batch k+1 are issued right after the
+// gathers of batch k and stay raw until their batch: 8 registers, where decoded
+// indices took 16 and spilled (20 bytes in delta p), and a last half batch
+// decodes only its own half.  Decoding in a block of its own, before the first
+// gather issues, keeps the gathers together: interleaved with it, the surface
+// pass took 643 us against 551 and every other pass 1-7% more.  Measured at 8.4M
+// particles against decoded prefetch: density+lambda 358 -> 323 us, delta p 317
+// -> 303, surface 562 -> 551, colour, confinement and vorticity within 1%, XSPH
+// (whose two-array gathers take no prefetch now, 546 us with it) 527 -> 539.
+// Slots past c are never used; their gathers load a valid index (the particle
+// itself in a wide list, the layer-2 base in a compact one, which the build sets
+// to the particle itself when that layer has no candidates), which costs less
+// than it seems: an index past the records instead, which touches no line, made
+// no pass faster.
 constexpr int kBatch = 8;  // candidate batch of the list build
 constexpr uint32_t kQuadStride = kWave * 4;  // list words between a lane's quads
 // Hits the list build buffers in LDS per thread (16 bits each) for the
@@ -102,47 +115,50 @@ __device__ __forceinline__ void store_entry16(uint32_t *out, int e, uint32_t v) 
   w[e & 1] = (uint16_t)v;
 }
 
-template <int NB>
-__device__ __forceinline__ void load_wide(const NbList &nl, int k0, uint32_t self,
-                                          uint32_t (&j)[NB]) {
-  const uint4 *Q = reinterpret_cast<const uint4 *>(nl.L);
-  const int q0 = k0 >> 2;
+// Raw quads of the NB entries from k0 on; those past the last quad stay as they
+// were (decode does not use them).
+template <int NB, bool WIDE>
+struct Quads {
+  static constexpr int kPer = WIDE ? 4 : 8, kCount = NB / kPer;
+  uint4 q[kCount];
+  __device__ __forceinline__ void load(const NbList &nl, int k0) {
+    const uint4 *Q = reinterpret_cast<const uint4 *>(nl.L) + (size_t)(k0 / kPer) * kWave;
 #pragma unroll
-  for (int u = 0; u < NB / 4; ++u) {
-    uint4 a = make_uint4(self, self, self, self);
-    if (k0 + 4 * u < nl.c) a = Q[(size_t)(q0 + u) * kWave];
-    j[4 * u] = a.x;
-    j[4 * u + 1] = a.y;
-    j[4 * u + 2] = a.z;
-    j[4 * u + 3] = a.w;
+    for (int u = 0; u < kCount; ++u)
+      if (k0 + kPer * u < nl.c) q[u] = Q[(size_t)u * kWave];
   }
-#pragma unroll
-  for (int t = 0; t < NB; ++t)
-    if (k0 + t >= nl.c) j[t] = self;
-}
+};
 
-// Compact quads: entry k = base of its layer + 16-bit offset; padding entries
-// are offset 0 from the layer-2 base.
-template <int NB>
-__device__ __forceinline__ void load_compact(const NbList &nl, int k0, uint32_t (&j)[NB]) {
-  static_assert(NB % 8 == 0, "compact quads hold 8 entries");
-  const uint4 *Q = reinterpret_cast<const uint4 *>(nl.L);
-  const int q0 = k0 >> 3;
+// Sorted indices of entries [k0, k0 + M) from their quads.  Wide: as stored, the
+// particle itself past c.  Compact: base of the entry's layer + 16-bit offset;
+// past the last quad, offset 0 from the layer-2 base.
+template <int M, int NB, bool WIDE>
+__device__ __forceinline__ void decode(const NbList &nl, const Quads<NB, WIDE> &r, int k0,
+                                       uint32_t self, uint32_t (&j)[M]) {
   // values, not member lvalues: a select between member addresses would
   // keep the struct in memory (and the compiler moves such memory to LDS)
   const uint32_t b0 = nl.h.x, b1 = nl.h.y, b2 = nl.h.z;
   const int e0 = nl.e0, e1 = nl.e1, c = nl.c;
+  if (WIDE) {
 #pragma unroll
-  for (int u = 0; u < NB / 8; ++u) {
-    uint4 a = make_uint4(0u, 0u, 0u, 0u);
-    if (k0 + 8 * u < c) a = Q[(size_t)(q0 + u) * kWave];
-    const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+    for (int t = 0; t < M; ++t) {
+      const uint4 a = r.q[t / 4];
+      const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+      j[t] = k0 + t < c ? w[t & 3] : self;
+    }
+  } else {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int k = k0 + 8 * u + t;
-      const uint32_t off = (t & 1) ? (w[t >> 1] >> 16) : (w[t >> 1] & 0xFFFFu);
-      const uint32_t lb = k < e1 ? b1 : b2;
-      j[8 * u + t] = (k < e0 ? b0 : lb) + off;
+    for (int u = 0; u < M / 8; ++u) {
+      const bool in = k0 + 8 * u < c;
+      const uint4 a = r.q[u];
+      const uint32_t w[4] = {in ? a.x : 0u, in ? a.y : 0u, in ? a.z : 0u, in ? a.w : 0u};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int k = k0 + 8 * u + t;
+        const uint32_t off = (t & 1) ? (w[t >> 1] >> 16) : (w[t >> 1] & 0xFFFFu);
+        const uint32_t lb = k < e1 ? b1 : b2;
+        j[8 * u + t] = (k < e0 ? b0 : lb) + off;
+      }
     }
   }
 }
@@ -151,37 +167,38 @@ __device__ __forceinline__ void load_compact(const NbList &nl, int k0, uint32_t 
 // list ends skip the per-neighbour count test, and a last batch in which every
 // lane ends within NB/2 neighbours runs only NB/2 of them (the wave's longest
 // list, not the mean, sets the work: half batches cut the padding slots).
-template <typename T, int NB, bool PREFETCH, bool WIDE, bool LAST_SKIP, typename Load,
-          typename Body>
-__device__ __forceinline__ void gather_loop(const NbList &nl, uint32_t self, Load &load,
-                                            Body &body) {
-  uint32_t jn[NB];
-  auto fetch = [&](int k0) {
-    if (WIDE)
-      load_wide<NB>(nl, k0, self, jn);
-    else
-      load_compact<NB>(nl, k0, jn);
-  };
+template <typename T, int NB, bool PREFETCH, bool WIDE, typename Load, typename Body>
+__device__ __forceinline__ void gather_loop(const NbList &nl, const uint4 *first, uint32_t self,
+                                            Load &load, Body &body) {
+  Quads<NB, WIDE> r;
   const int c = nl.c;
-  fetch(0);
+  if (WIDE) {
+    r.load(nl, 0);
+  } else {
+#pragma unroll
+    for (int u = 0; u < Quads<NB, WIDE>::kCount; ++u) r.q[u] = first[u];
+  }
   for (int k0 = 0; k0 < c; k0 += NB) {
     // the lanes still in the loop have c > k0
-    if (!PREFETCH && k0 > 0) fetch(k0);
+    if (!PREFETCH && k0 > 0) r.load(nl, k0);
     if (NB >= 16 && __ballot(k0 + NB / 2 < c) == 0ull) {
+      uint32_t j[NB / 2];
+      decode<NB / 2>(nl, r, k0, self, j);
+      __builtin_amdgcn_sched_barrier(0);
       T q[NB / 2];
 #pragma unroll
-      for (int b = 0; b < NB / 2; ++b) q[b] = load(jn[b]);
+      for (int b = 0; b < NB / 2; ++b) q[b] = load(j[b]);
 #pragma unroll
       for (int b = 0; b < NB / 2; ++b)
         if (k0 + b < c) body(q[b]);
     } else {
+      uint32_t j[NB];
+      decode<NB>(nl, r, k0, self, j);
+      __builtin_amdgcn_sched_barrier(0);
       T q[NB];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) q[b] = load(jn[b]);
-      // with LAST_SKIP not on the wave's last batch: the decode is VALU work,
-      // but as a block of its own it no longer interleaves with the
-      // arithmetic (faster for the density pass only, measured)
-      if (PREFETCH && (!LAST_SKIP || __ballot(k0 + NB < c) != 0ull)) fetch(k0 + NB);
+      for (int b = 0; b < NB; ++b) q[b] = load(j[b]);
+      if (PREFETCH) r.load(nl, k0 + NB);
       if (__ballot(k0 + NB > c) == 0ull) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) body(q[b]);
@@ -194,14 +211,19 @@ __device__ __forceinline__ void gather_loop(const NbList &nl, uint32_t self, Loa
   }
 }
 
-template <typename T, int NB, bool PREFETCH = true, bool LAST_SKIP = false, typename Load,
-          typename Body>
-__device__ __forceinline__ void for_neighbors(const NbList &nl, uint32_t self, Load load,
-                                              Body body) {
+template <typename T, int NB, bool PREFETCH = true, typename Load, typename Body>
+__device__ __forceinline__ void for_neighbors(const uint32_t *list, const uint4 *head, uint32_t s,
+                                              int *count, Load load, Body body) {
+  uint4 first[NB / 8];
+#pragma unroll
+  for (int u = 0; u < NB / 8; ++u)
+    first[u] = reinterpret_cast<const uint4 *>(list_ptr(list, s))[(size_t)u * kWave];
+  const NbList nl = nb_list(list, head, s);
+  *count = nl.c;
   if (nl.wide)
-    gather_loop<T, NB, PREFETCH, true, LAST_SKIP>(nl, self, load, body);
+    gather_loop<T, NB, PREFETCH, true>(nl, first, s, load, body);
   else
-    gather_loop<T, NB, PREFETCH, false, LAST_SKIP>(nl, self, load, body);
+    gather_loop<T, NB, PREFETCH, false>(nl, first, s, load, body);
 }
 
 struct Pair4 {
@@ -212,10 +234,9 @@ struct Pair4 {
 // (`buffer_load ... idxen`): the texture addresser forms base + 16 j from the
 // index itself, so a gather costs no VALU (a 64-bit address costs two, the
 // zero high word and the shift-add) and needs no address registers.  At 16
-// gathers in flight: colour and confinement 138-140 -> 130-133 VGPRs, delta p
-// spills 20 bytes instead of 52 and density+lambda none instead of 12, XSPH at
-// 8 gathers 112 -> 90 VGPRs (5 waves per SIMD instead of 4), and the autotuner
-// now picks 16 gathers in flight for XSPH and vorticity instead of 8 (measured
+// gathers in flight colour and confinement took 138-140 -> 130-133 VGPRs, XSPH
+// at 8 gathers 112 -> 90 VGPRs (5 waves per SIMD instead of 4), and the autotuner
+// picked 16 gathers in flight for XSPH and vorticity instead of 8 (measured
 // at 8M particles: vorticity 0.70 -> 0.58 ms, XSPH 0.67 -> 0.60, delta p,
 // colour and confinement 3% faster, density+lambda unchanged).  An index at or
 // past `records` reads zeros instead of leaving the array.
@@ -995,12 +1016,12 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
   float err = 0.0f;
   if (active) {
     const float4 p = pos[s];
-    const NbList nl = nb_list(list, head, s);
+    int cnt;
     uint32_t S = 0u;
     float sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, sc = 0.0f;
     const Records16 G(pos, n);
-    for_neighbors<float4, NB, true, true>(nl, s, [&](uint32_t j) { return G[j]; },
-                                          [&](const float4 &q) {
+    for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; },
+                              [&](const float4 &q) {
       const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       const float r2 = sq3(dx, dy, dz);
       if (MODE != 2) S += density_term(r2, P);
@@ -1018,7 +1039,7 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
     });
     float C;
     if (MODE != 2) {
-      C = density_constraint(S, nl.c, P);
+      C = density_constraint(S, cnt, P);
       const float rho = fmaf(C, P.rest_density, P.rest_density);
       rho_out[s] = rho;
       if (c_io) c_io[s] = C;
@@ -1107,10 +1128,12 @@ __device__ __forceinline__ void collide(float &x, float &y, float &z, const SdfD
 // UpdateDPs (particles.c:668-746): returns sum_j (lambda_i + lambda_j) DelW(r)/r d.
 template <int NB>
 __device__ __forceinline__ float3 dp_sum(const float4 &p, const float4 *pos, uint32_t n,
-                                         const NbList &nl, uint32_t self, const DevParams &P) {
+                                         const uint32_t *list, const uint4 *head, uint32_t s,
+                                         const DevParams &P) {
+  int cnt;
   float ax = 0.0f, ay = 0.0f, az = 0.0f;
   const Records16 G(pos, n);
-  for_neighbors<float4, NB>(nl, self, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
     const float ir = fast_rsq(r2c);
@@ -1140,7 +1163,7 @@ __global__ GATHER_BOUNDS(NB) void k_dp(uint32_t n, uint32_t nblocks,
   const uint32_t s = particle_index(nblocks);
   if (s >= n) return;
   const float4 p = pos[s];
-  const float3 a = dp_sum<NB>(p, pos, n, nb_list(list, head, s), s, P);
+  const float3 a = dp_sum<NB>(p, pos, n, list, head, s, P);
   const float4 d = make_float4(scale * a.x, scale * a.y, scale * a.z, 0.0f);
   dp[s] = d;
   if (xnext) {
@@ -1194,7 +1217,7 @@ __global__ GATHER_BOUNDS(NB) void k_dp_update(
     return;
   }
   if (s == 0) stats[STAT_ITERS] += 1u;
-  const float3 a = dp_sum<NB>(p, pin, n, nb_list(list, head, s), s, P);
+  const float3 a = dp_sum<NB>(p, pin, n, list, head, s, P);
   float x = fmaf(scale, a.x, p.x), y = fmaf(scale, a.y, p.y), z = fmaf(scale, a.z, p.z);
   apply_boundary(x, y, z, geo_of<BATCH>(s, P, B), P);
   if (COLLIDE) collide(x, y, z, sdf_of<BATCH>(s, o, B));
@@ -1258,13 +1281,13 @@ __global__ __launch_bounds__(kBlock) void k_warm_lambda(
     const float4 p = pos[s];
     const float4 po = xold[s];
     const float ux = p.x - po.x, uy = p.y - po.y, uz = p.z - po.z;  // dt * v_i
-    const NbList nl = nb_list(list, head, s);
+    int cnt;
     uint32_t S = 0u;
     float sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, sc = 0.0f;
     float mx = 0.0f, my = 0.0f, mz = 0.0f, dv = 0.0f;
     const Records16 Gp(pos, n), Go(xold, n);
     auto load = [&](uint32_t j) { return Pair4{Gp[j], Go[j]}; };
-    for_neighbors<Pair4, NB, false>(nl, s, load, [&](const Pair4 &qq) {
+    for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qq) {
       const float4 &q = qq.a, &qo = qq.b;
       const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       const float r2 = sq3(dx, dy, dz);
@@ -1286,14 +1309,14 @@ __global__ __launch_bounds__(kBlock) void k_warm_lambda(
       const float ex = (q.x - qo.x) - ux, ey = (q.y - qo.y) - uy, ez = (q.z - qo.z) - uz;
       dv = fmaf(g, fmaf(ez, dz, fmaf(ey, dy, ex * dx)), dv);
     });
-    const float cr = density_constraint(S, nl.c, P);
+    const float cr = density_constraint(S, cnt, P);
     rho = fmaf(cr, P.rest_density, P.rest_density);
     rho_io[s] = rho;
     err = fmaxf((rho - P.rest_density) * P.inv_rest_density, 0.0f);  // as k_density_lambda
     const float gc2 = P.lam_k2 * (sc + sq3(sgx, sgy, sgz));
     denom = gc2 + P.lambda_eps;
     lam0 = -fmaxf(cr, 0.0f) / denom;  // as k_density_lambda
-    f[0] = (float)nl.c * (1.0f / 32.0f);
+    f[0] = (float)cnt * (1.0f / 32.0f);
     f[1] = cr;
     f[2] = -lam_prev[id_s[s]] * denom;
     f[3] = gc2 / denom;
@@ -1487,10 +1510,10 @@ __global__ GATHER_BOUNDS(NB) void k_color(uint32_t n, uint32_t nblocks,
   if (s >= n) return;
   const float4 p = pos[s];
   if (WITH_VELOCITY) vel[s] = velocity_of(p, xold[s], P);
-  const NbList nl = nb_list(list, head, s);
+  int cnt;
   float ax = 0.0f, ay = 0.0f, az = 0.0f;
   const Records16 G(pos, n);
-  for_neighbors<float4, NB>(nl, s, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
     const float u = P.h2 - r2c;
@@ -1507,8 +1530,7 @@ __global__ GATHER_BOUNDS(NB) void k_color(uint32_t n, uint32_t nblocks,
 // spline C, particles.c:54-65) + curvature, v += dt F / rho_i in place.  The
 // spline is computed without a branch per neighbour (the branch split the
 // loop body and held 104 VGPRs at 8 gathers in flight, 89 without it); at 16
-// gathers, bounded to 168 VGPRs (3 waves per SIMD, 20 bytes spilled), the
-// pass measured 0.628 -> 0.561 ms at 8M particles.
+// gathers it runs 3 waves per SIMD without spilling.
 template <int NB>
 __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t n, uint32_t nblocks,
                                                     const float4 *__restrict__ pos,
@@ -1520,12 +1542,12 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 ci = color[s];
-  const NbList nl = nb_list(list, head, s);
+  int cnt;
   const float hh = 0.5f * P.h;
   float fx = 0.0f, fy = 0.0f, fz = 0.0f;
   const Records16 Gp(pos, n), Gc(color, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gc[j]}; };
-  for_neighbors<Pair4, NB, false>(nl, s, load, [&](const Pair4 &qc) {
+  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qc) {
     const float4 &q = qc.a, &cq = qc.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1552,10 +1574,6 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t
 
 // ApplyViscosity (particles.c:383-459), reading v_old and writing v_new.  The
 // distance keeps the reference's typo r^2 = dx^2 + dy^2 dz^2 (particles.c:439).
-// The only two-array pass with the list prefetch: at 16 gathers in flight it
-// takes 175 VGPRs (2 waves per SIMD), bounded to 168 (3 waves, 32 bytes
-// spilled) it ran 8% faster than without the prefetch at 8M particles; the
-// surface and vorticity passes were 0-15% slower with it.
 template <int NB>
 __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_xsph(uint32_t n, uint32_t nblocks,
                                                  const float4 *__restrict__ pos,
@@ -1567,11 +1585,11 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_xsph(uint32_t n,
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 vi = vin[s];
-  const NbList nl = nb_list(list, head, s);
+  int cnt;
   float ax = 0.0f, ay = 0.0f, az = 0.0f;
   const Records16 Gp(pos, n), Gv(vin, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  for_neighbors<Pair4, NB, true>(nl, s, load, [&](const Pair4 &qv) {
+  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float u = P.h2 - fmaf(dy * dy * dz, dz, dx * dx);
@@ -1599,11 +1617,11 @@ __global__ __launch_bounds__(kBlock) void k_vorticity(uint32_t n, uint32_t nbloc
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 vi = vel[s];
-  const NbList nl = nb_list(list, head, s);
+  int cnt;
   float ox = 0.0f, oy = 0.0f, oz = 0.0f;
   const Records16 Gp(pos, n), Gv(vel, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  for_neighbors<Pair4, NB, false>(nl, s, load, [&](const Pair4 &qv) {
+  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1641,11 +1659,11 @@ __global__ GATHER_BOUNDS(NB) void k_confine(
   const uint32_t s = particle_index(nblocks);
   if (s >= n) return;
   const float4 p = pw[s];
-  const NbList nl = nb_list(list, head, s);
+  int cnt;
   float ex = 0.0f, ey = 0.0f, ez = 0.0f;
   // only x_j and |omega_j| of the neighbour are needed
   const Records16 G(pw, n);
-  for_neighbors<float4, NB>(nl, s, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
     const float ir = fast_rsq(r2c);
