@@ -5,6 +5,9 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "sph_internal.h"
@@ -192,8 +195,9 @@ static void free_all(sph_ctx *c) {
                   c->warm_net};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
-  if (c->io_dev) (void)hipFree(c->io_dev);
   if (c->io_host) (void)hipHostFree(c->io_host);
+  for (hipEvent_t e : c->io_done)
+    if (e) (void)hipEventDestroy(e);
   for (auto &p : c->prof.pending) {
     (void)hipEventDestroy(p.a);
     (void)hipEventDestroy(p.b);
@@ -586,51 +590,108 @@ extern "C" int sph_set_obstacle(sph_ctx *c, const sph_obstacle_desc *o) {
   return rc;
 }
 
-// SoA <-> the float4 canonical state, on the device (coalesced on both sides).
-__global__ void k_pack_state(uint32_t n, const float *__restrict__ soa,
-                             float4 *__restrict__ x, float4 *__restrict__ v) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  x[i] = make_float4(soa[i], soa[n + i], soa[2 * (size_t)n + i], 0.0f);
-  v[i] = make_float4(soa[3 * (size_t)n + i], soa[4 * (size_t)n + i], soa[5 * (size_t)n + i],
-                     0.0f);
+// State transfers.  The caller's arrays pass through pinned host staging in
+// chunks of `chunk` particles, six arrays of `chunk` floats each, which the GPU
+// reads and writes in place: a pack kernel per chunk takes the staged floats over
+// the bus into the float4 state (an unpack kernel the other way), four particles
+// a thread, 1 KB a wave and array.  Chunks let the bus, at 55 GB/s, run while the
+// host copies the next or the previous one, and several threads copy because one
+// does 27 GB/s.  8.4M particles with velocities: upload 10.2 -> 5.3 ms, download
+// 10.3 -> 4.2 ms; 4096: 23 -> 17 us and 26 -> 17 us (a copy on the device less).
+constexpr int kIoThreads = 4;
+// Below this capacity one chunk and the calling thread (3 MB, 120 us; starting
+// three threads takes 50).
+constexpr int kIoOneChunk = 1 << 17;
+
+static size_t io_chunk(const sph_ctx *c) {
+  const size_t cap = (size_t)std::max(c->cap, 1);
+  if (cap < (size_t)kIoOneChunk) return (cap + 3) & ~(size_t)3;
+  return std::max<size_t>(32768, ((cap + kIoChunks - 1) / kIoChunks + 1023) & ~(size_t)1023);
 }
 
-__global__ void k_unpack_state(uint32_t n, const float4 *__restrict__ x,
-                               const float4 *__restrict__ v, float *__restrict__ soa,
-                               int with_velocity) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kBlock) void k_pack_state(uint32_t n, uint32_t chunk,
+                                                       const float *__restrict__ staged,
+                                                       float4 *__restrict__ x,
+                                                       float4 *__restrict__ v) {
+  const uint32_t i = (blockIdx.x * kBlock + threadIdx.x) * 4u;
   if (i >= n) return;
-  const float4 a = x[i];
-  soa[i] = a.x;
-  soa[n + i] = a.y;
-  soa[2 * (size_t)n + i] = a.z;
-  if (with_velocity) {
-    const float4 b = v[i];
-    soa[3 * (size_t)n + i] = b.x;
-    soa[4 * (size_t)n + i] = b.y;
-    soa[5 * (size_t)n + i] = b.z;
+  float4 a[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+    a[k] = *reinterpret_cast<const float4 *>(staged + (size_t)k * chunk + i);
+#pragma unroll
+  for (uint32_t t = 0; t < 4; ++t) {
+    if (i + t >= n) break;
+    const auto at = [t](const float4 &q) {
+      return t == 0 ? q.x : (t == 1 ? q.y : (t == 2 ? q.z : q.w));
+    };
+    x[i + t] = make_float4(at(a[0]), at(a[1]), at(a[2]), 0.0f);
+    v[i + t] = make_float4(at(a[3]), at(a[4]), at(a[5]), 0.0f);
   }
 }
 
-// Device and pinned host staging for state transfers (6 floats per particle of
-// the capacity), allocated on first use.
+__global__ __launch_bounds__(kBlock) void k_unpack_state(uint32_t n, uint32_t chunk,
+                                                         const float4 *__restrict__ x,
+                                                         const float4 *__restrict__ v,
+                                                         float *__restrict__ staged,
+                                                         int with_velocity) {
+  const uint32_t i = (blockIdx.x * kBlock + threadIdx.x) * 4u;
+  if (i >= n) return;
+  const auto put = [&](const float4 *src, int first) {
+    float4 q[4];
+#pragma unroll
+    for (uint32_t t = 0; t < 4; ++t) q[t] = src[min(i + t, n - 1u)];
+    float4 *d = reinterpret_cast<float4 *>(staged + (size_t)first * chunk + i);
+    d[0] = make_float4(q[0].x, q[1].x, q[2].x, q[3].x);
+    d[chunk / 4u] = make_float4(q[0].y, q[1].y, q[2].y, q[3].y);
+    d[chunk / 2u] = make_float4(q[0].z, q[1].z, q[2].z, q[3].z);
+  };
+  put(x, 0);
+  if (with_velocity) put(v, 3);
+}
+
+// Pinned staging (6 floats per particle of the capacity, in whole chunks) and an
+// event per chunk, on first use.
 static int io_buffers(sph_ctx *c) {
-  if (c->io_dev && c->io_host) return SPH_OK;
-  const size_t bytes = sizeof(float) * 6 * (size_t)std::max(c->cap, 1);
-  if (!c->io_dev) {
-    hipError_t e = hipMalloc(&c->io_dev, bytes);
-    if (e != hipSuccess) {
-      c->io_dev = nullptr;
-      return hip_fail(e, "hipMalloc (state transfer staging)");
-    }
-  }
-  hipError_t e = hipHostMalloc(&c->io_host, bytes, hipHostMallocDefault);
+  if (c->io_host) return SPH_OK;
+  for (hipEvent_t &e : c->io_done)
+    if (!e) SPH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  const size_t chunk = io_chunk(c), cap = (size_t)std::max(c->cap, 1);
+  const size_t bytes = sizeof(float) * 6 * chunk * ((cap + chunk - 1) / chunk);
+  const hipError_t e = hipHostMalloc(&c->io_host, bytes, hipHostMallocDefault);
   if (e != hipSuccess) {
     c->io_host = nullptr;
     return hip_fail(e, "hipHostMalloc (state transfer staging)");
   }
   return SPH_OK;
+}
+
+// Runs work(k) for every chunk k of `chunks`, on this thread and, for more than
+// one chunk, up to kIoThreads - 1 more; without them where none can be started.
+// `mine`, if given, is called on this thread between its own chunks.
+template <class Work, class Mine>
+static void io_chunks(size_t chunks, Work work, Mine mine) {
+  std::atomic<size_t> next{0};
+  auto take = [&]() {
+    const size_t k = next.fetch_add(1);
+    if (k < chunks) work(k);
+    return k < chunks;
+  };
+  std::thread helpers[kIoThreads - 1];
+  for (size_t t = 0; t + 1 < std::min<size_t>(kIoThreads, chunks); ++t) {
+    try {
+      helpers[t] = std::thread([&]() {
+        while (take()) {
+        }
+      });
+    } catch (const std::system_error &) {
+      break;
+    }
+  }
+  while (take()) mine();
+  for (std::thread &h : helpers)
+    if (h.joinable()) h.join();
+  mine();
 }
 
 extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *y,
@@ -651,13 +712,26 @@ extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *
   if (n) {
     int rc = io_buffers(c);
     if (rc) return rc;
-    const size_t un = (size_t)n;
+    const size_t un = (size_t)n, chunk = io_chunk(c), chunks = (un + chunk - 1) / chunk;
     const float *src[6] = {x, y, z, vx, vy, vz};
-    for (int k = 0; k < 6; ++k) memcpy(c->io_host + k * un, src[k], sizeof(float) * un);
-    SPH_HIP(hipMemcpyAsync(c->io_dev, c->io_host, sizeof(float) * 6 * un,
-                           hipMemcpyHostToDevice, c->stream));
-    k_pack_state<<<blocks_for((uint32_t)n), kBlock, 0, c->stream>>>((uint32_t)n, c->io_dev,
-                                                                    c->x_can, c->v_can);
+    std::atomic<bool> staged[kIoChunks] = {};
+    size_t sent = 0;
+    io_chunks(
+        chunks,
+        [&](size_t k) {
+          const size_t first = k * chunk, m = std::min(chunk, un - first);
+          float *to = c->io_host + 6 * first;
+          for (int a = 0; a < 6; ++a) memcpy(to + a * chunk, src[a] + first, sizeof(float) * m);
+          staged[k].store(true, std::memory_order_release);
+        },
+        [&]() {  // the chunks that are staged by now, in order
+          for (; sent < chunks && staged[sent].load(std::memory_order_acquire); ++sent) {
+            const size_t first = sent * chunk, m = std::min(chunk, un - first);
+            k_pack_state<<<blocks_for((uint32_t)m, 4 * kBlock), kBlock, 0, c->stream>>>(
+                (uint32_t)m, (uint32_t)chunk, c->io_host + 6 * first, c->x_can + first,
+                c->v_can + first);
+          }
+        });
     SPH_HIP(hipGetLastError());
   }
   if (c->lam_prev) SPH_HIP(hipMemsetAsync(c->lam_prev, 0, sizeof(float) * c->cap, c->stream));
@@ -679,15 +753,35 @@ extern "C" int sph_download_state(sph_ctx *c, float *x, float *y, float *z, floa
   const bool with_v = vx || vy || vz;
   if (n && (x || y || z || with_v)) {
     if ((rc = io_buffers(c))) return rc;
-    const size_t un = (size_t)n;
-    k_unpack_state<<<blocks_for((uint32_t)n), kBlock, 0, c->stream>>>(
-        (uint32_t)n, c->x_can, c->v_can, c->io_dev, with_v ? 1 : 0);
-    SPH_HIP(hipGetLastError());
-    SPH_HIP(hipMemcpyAsync(c->io_host, c->io_dev, sizeof(float) * (with_v ? 6 : 3) * un,
-                           hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(hipStreamSynchronize(c->stream));
-    for (int k = 0; k < 6; ++k)
-      if (dst[k]) memcpy(dst[k], c->io_host + k * un, sizeof(float) * un);
+    const size_t un = (size_t)n, chunk = io_chunk(c), chunks = (un + chunk - 1) / chunk;
+    for (size_t k = 0; k < chunks; ++k) {
+      const size_t first = k * chunk, m = std::min(chunk, un - first);
+      k_unpack_state<<<blocks_for((uint32_t)m, 4 * kBlock), kBlock, 0, c->stream>>>(
+          (uint32_t)m, (uint32_t)chunk, c->x_can + first, c->v_can + first,
+          c->io_host + 6 * first, with_v ? 1 : 0);
+      SPH_HIP(hipGetLastError());
+      if (chunks > 1) SPH_HIP(hipEventRecord(c->io_done[k], c->stream));
+    }
+    if (chunks == 1) SPH_HIP(hipStreamSynchronize(c->stream));
+    std::atomic<int> failed{hipSuccess};
+    io_chunks(
+        chunks,
+        [&](size_t k) {
+          if (chunks > 1) {
+            const hipError_t e = hipEventSynchronize(c->io_done[k]);
+            if (e != hipSuccess) {
+              failed.store(e);
+              return;
+            }
+          }
+          const size_t first = k * chunk, m = std::min(chunk, un - first);
+          const float *from = c->io_host + 6 * first;
+          for (int a = 0; a < 6; ++a)
+            if (dst[a]) memcpy(dst[a] + first, from + a * chunk, sizeof(float) * m);
+        },
+        []() {});
+    if (failed.load() != hipSuccess)
+      return hip_fail((hipError_t)failed.load(), "hipEventSynchronize (state download)");
     return SPH_OK;
   }
   SPH_HIP(hipStreamSynchronize(c->stream));

@@ -19,6 +19,8 @@ constexpr int kListStride = kWave * kMaxNb;  // list words per 64-particle group
 // 4 GiB, so that gathers address them with 32-bit byte offsets.
 constexpr uint32_t kMaxParticles = SPH_MAX_PARTICLES;
 static_assert((kMaxParticles + 64ull) * 16ull <= (1ull << 32), "32-bit byte offsets");
+// Chunks of a state transfer, at most.
+constexpr int kIoChunks = 16;
 // Particles per block of the per-scene error reduction of a batch.
 constexpr uint32_t kSceneChunk = 4096;
 // Neighbour-list head per particle: the first candidate index of each of the
@@ -200,9 +202,10 @@ struct sph_ctx {
   float *cstage = nullptr, *lam_stage = nullptr;
   uint32_t *list = nullptr;     // sorted neighbour indices, quads of slots per 64 particles
   uint4 *list_head = nullptr;   // per sorted particle: layer bases and counts
-  // state transfers: SoA x, y, z, vx, vy, vz of up to cap particles, on the
-  // device and in pinned host memory (allocated on first use)
-  float *io_dev = nullptr, *io_host = nullptr;
+  // state transfers: x, y, z, vx, vy, vz of up to cap particles in pinned host
+  // memory, by chunks, and each chunk's end of unpacking (on first use)
+  float *io_host = nullptr;
+  hipEvent_t io_done[sph::kIoChunks] = {};
   uint32_t *stats = nullptr;  // sph::STAT_WORDS words
   uint32_t *pair_partial = nullptr;  // per-block list-length sums of the last search
   uint32_t pair_blocks = 0;

@@ -77,6 +77,30 @@ def test_cell_bounds_at_the_edges_of_the_scan(cells):
     test_cell_bounds_bit_exact(20_000, cells)
 
 
+@pytest.mark.parametrize("n,cap", [(1, 1), (3, 7), (4, 4), (1021, 2000), ((1 << 17) - 1,) * 2,
+                                   (1 << 17,) * 2, (5, 1 << 17), (32769, 1 << 17),
+                                   ((1 << 19) + 1,) * 2,
+                                   ((1 << 21) + 5,) * 2])
+def test_state_transfer_round_trip(n, cap):
+    """One chunk below 2^17 particles of capacity, up to 16 above, ragged ends,
+    and a download of some of the arrays only."""
+    sc = Scene(0.02, (1.0, 1.0, 1.0))
+    rng = np.random.default_rng(n)
+    pos, vel = rng.random((n, 3), np.float32), rng.standard_normal((n, 3), np.float32)
+    with sc.context(cap) as ctx:
+        for _ in range(2):
+            ctx.upload(pos, vel)
+            p, v = ctx.download()
+            assert np.array_equal(p, pos) and np.array_equal(v, vel)
+            pos, vel = vel, pos
+        y, vz = np.full(n, 7.0, np.float32), np.full(n, 7.0, np.float32)
+        for some in ((y, None), (y, vz)):
+            a = [None, some[0], None, None, None, some[1]]
+            sa.check(sa.lib().sph_download_state(
+                ctx.handle, *[sa._fptr(v) if v is not None else None for v in a]))
+        assert np.array_equal(y, vel[:, 1]) and np.array_equal(vz, pos[:, 2])
+
+
 # ---------------------------------------------------------------------------
 # Neighbour search in the staged pipeline (neighbors.c:68-298)
 # ---------------------------------------------------------------------------
