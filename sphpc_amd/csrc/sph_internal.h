@@ -290,10 +290,11 @@ inline size_t scan_tiles(size_t len) { return (len + kScanTile - 1) / kScanTile 
 // write_total also sets out[len].
 int scan(const uint32_t *in, uint32_t *out, uint32_t len, bool inclusive, bool write_total,
          ScanScratch *scratch, hipStream_t s, sph_ctx *prof);
+// hist: radix_words(n, key_bits) words.
+size_t radix_words(uint32_t n, int key_bits);
 int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uint32_t *v0,
-                     uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t **hist,
-                     size_t *hist_cap, ScanScratch *scratch, hipStream_t s,
-                     const uint32_t **kout, const uint32_t **vout);
+                     uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t *hist,
+                     hipStream_t s, const uint32_t **kout, const uint32_t **vout);
 int count_keys(const uint32_t *keys, uint32_t n, uint32_t *count, uint32_t cells,
                hipStream_t s);
 

@@ -1,15 +1,14 @@
 // Stable key/value radix sort, exclusive scan and cell bounds for gfx950.
 //
 // Replaces the Thrust wrappers of the reference (thrust_c.cu:86-120):
-//  - SortByKey: LSD radix sort, 8-bit digits.  Each pass is an upsweep
-//    (per-tile digit histogram), a scan of the histogram in digit-major
-//    order, and a downsweep that ranks keys inside the tile with wavefront
-//    ballots (peers with the same digit), stages the tile in LDS in digit
-//    order and writes each digit run out contiguously.  Ranks follow input
-//    position (wave, round, lane), so the sort is stable.
-//  - FindLowerBounds/FindUpperBounds: a key histogram followed by an
-//    exclusive scan gives lower_bound(c) for every cell; upper_bound(c) is
-//    lower_bound(c+1).
+//  - SortByKey: LSD radix sort, digits of 8 or 10 bits.  Each pass is an
+//    upsweep (per-tile digit histogram), a scan of each digit's row of it, and a
+//    downsweep that ranks keys inside the tile with wavefront ballots (peers with
+//    the same digit), stages the tile in LDS in digit order and writes each digit
+//    run out contiguously.  Ranks follow input position (wave, round, lane), so
+//    the sort is stable.
+//  - FindLowerBounds/FindUpperBounds: a key histogram followed by a scan:
+//    exclusive it is lower_bound(c) for every cell, inclusive upper_bound(c).
 #include <mutex>
 
 #include "sph_internal.h"
@@ -55,11 +54,12 @@ __device__ __forceinline__ uint32_t block_excl_scan_256(uint32_t x, uint32_t *wt
   return pre + (lane ? before : 0u);
 }
 
-// Lanes of the wave holding the same 8-bit digit (valid lanes only).
+// Lanes of the wave holding the same digit (valid lanes only).
+template <int BITS>
 __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid) {
   uint64_t peers = __ballot(valid);
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
+  for (int b = 0; b < BITS; ++b) {
     const bool bit = (d >> b) & 1u;
     const uint64_t bb = __ballot(bit);
     peers &= bit ? bb : ~bb;
@@ -237,12 +237,15 @@ int scan(const uint32_t *in, uint32_t *out, uint32_t len, bool inclusive, bool w
 // --------------------------------------------------------------------------
 // Radix sort
 // --------------------------------------------------------------------------
+// hist[digit * tiles + tile]: the tile's count of the digit.
+template <int BITS>
 __global__ __launch_bounds__(RS_THREADS) void k_radix_upsweep(const uint32_t *__restrict__ keys,
                                                               uint32_t n, int shift,
                                                               uint32_t *__restrict__ hist,
                                                               uint32_t tiles) {
-  __shared__ uint32_t h[RS_WAVES][256];
-  for (int i = threadIdx.x; i < RS_WAVES * 256; i += RS_THREADS) (&h[0][0])[i] = 0u;
+  constexpr int D = 1 << BITS;
+  __shared__ uint32_t h[RS_WAVES][D];
+  for (int i = threadIdx.x; i < RS_WAVES * D; i += RS_THREADS) (&h[0][0])[i] = 0u;
   __syncthreads();
   const int w = threadIdx.x >> 6;
   const uint64_t lt = lanemask_lt();
@@ -257,31 +260,56 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_upsweep(const uint32_t *__
   for (int r = 0; r < RS_ITEMS; ++r) {
     const uint32_t i = base + r * RS_THREADS + threadIdx.x;
     const bool valid = i < n;
-    const uint32_t d = (kk[r] >> shift) & 255u;
-    const uint64_t peers = match_digit(d, valid);
+    const uint32_t d = (kk[r] >> shift) & (D - 1u);
+    const uint64_t peers = match_digit<BITS>(d, valid);
     // one leader per digit per wave adds the digit's count (a non-returning
     // LDS add: no wait between rounds)
     if (valid && (peers & lt) == 0) atomicAdd(&h[w][d], (uint32_t)__popcll(peers));
   }
   __syncthreads();
-  uint32_t s = 0;
+  for (int d = threadIdx.x; d < D; d += RS_THREADS) {
+    uint32_t s = 0;
 #pragma unroll
-  for (int ww = 0; ww < RS_WAVES; ++ww) s += h[ww][threadIdx.x];
-  hist[(size_t)threadIdx.x * tiles + blockIdx.x] = s;
+    for (int ww = 0; ww < RS_WAVES; ++ww) s += h[ww][d];
+    hist[(size_t)d * tiles + blockIdx.x] = s;
+  }
 }
 
+// Exclusive scan of each digit's row of the histogram and its total, a block per
+// digit.  With the digits' own scan left to the downsweep (a block scan of the
+// totals) this is one launch, where a scan of the whole histogram takes three.
+__global__ __launch_bounds__(RS_THREADS) void k_radix_rows(uint32_t *__restrict__ hist,
+                                                           uint32_t tiles,
+                                                           uint32_t *__restrict__ totals) {
+  __shared__ uint32_t wtot[4];
+  uint32_t *row = hist + (size_t)blockIdx.x * tiles;
+  uint32_t carry = 0;
+  for (uint32_t t0 = 0; t0 < tiles; t0 += RS_THREADS) {
+    const uint32_t t = t0 + threadIdx.x;
+    uint32_t tot;
+    const uint32_t e = block_excl_scan_256(t < tiles ? row[t] : 0u, wtot, &tot);
+    if (t < tiles) row[t] = carry + e;
+    carry += tot;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+// ROWS: the histogram's rows are scanned and `totals` holds their sums;
+// otherwise each block sums the rows itself (few tiles: no launch between).
+template <int BITS, bool ROWS>
 __global__ __launch_bounds__(RS_THREADS) void k_radix_downsweep(
     const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
     uint32_t *__restrict__ kout, uint32_t *__restrict__ vout, uint32_t n, int shift,
-    const uint32_t *__restrict__ offs, uint32_t tiles) {
-  __shared__ uint32_t wcnt[RS_WAVES][256];
-  __shared__ uint32_t dstart[256];
-  __shared__ uint32_t goff[256];
+    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, uint32_t tiles) {
+  constexpr int D = 1 << BITS, DPT = D / RS_THREADS;  // digits per thread, consecutive
+  __shared__ uint32_t wcnt[RS_WAVES][D];
+  __shared__ uint32_t dstart[D];
+  __shared__ uint32_t goff[D];
   __shared__ uint32_t wtot[4];
   __shared__ uint32_t sk[RS_TILE];
   __shared__ uint32_t sv[RS_TILE];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  for (int i = tid; i < RS_WAVES * 256; i += RS_THREADS) (&wcnt[0][0])[i] = 0u;
+  for (int i = tid; i < RS_WAVES * D; i += RS_THREADS) (&wcnt[0][0])[i] = 0u;
   __syncthreads();
   const uint64_t lt = lanemask_lt();
   const uint32_t tile0 = blockIdx.x * RS_TILE;
@@ -298,8 +326,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_downsweep(
   for (int r = 0; r < RS_ITEMS; ++r) {
     const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
     const bool valid = i < n;
-    const uint32_t d = (k[r] >> shift) & 255u;
-    const uint64_t peers = match_digit(d, valid);
+    const uint32_t d = (k[r] >> shift) & (D - 1u);
+    const uint64_t peers = match_digit<BITS>(d, valid);
     const uint32_t below = (uint32_t)__popcll(peers & lt);
     // the digit's leader (lowest peer) takes the wave's running count and adds
     // the peers; LDS operations of a wave complete in order, so later rounds
@@ -309,25 +337,59 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_downsweep(
     const int leader = peers ? (int)__builtin_ctzll(peers) : lane;
     rk[r] = __shfl(old, leader, 64) + below;
   }
-  __syncthreads();
-  // Digit `tid`: prefix over waves, then tile-level digit starts.
-  uint32_t run = 0;
+  // where the digits of this thread begin in the output, over all tiles and in
+  // this one's share
+  uint32_t all[DPT], before[DPT], sum = 0u;
 #pragma unroll
-  for (int ww = 0; ww < RS_WAVES; ++ww) {
-    const uint32_t c = wcnt[ww][tid];
-    wcnt[ww][tid] = run;
-    run += c;
+  for (int q = 0; q < DPT; ++q) {
+    const int d = tid * DPT + q;
+    const uint32_t *row = hist + (size_t)d * tiles;
+    if (ROWS) {
+      all[q] = totals[d];
+      before[q] = row[blockIdx.x];
+    } else {
+      all[q] = before[q] = 0u;
+      for (uint32_t t = 0; t < tiles; ++t) {
+        const uint32_t x = row[t];
+        all[q] += x;
+        before[q] += t < blockIdx.x ? x : 0u;
+      }
+    }
+    sum += all[q];
   }
-  uint32_t tot;
-  const uint32_t ex = block_excl_scan_256(run, wtot, &tot);
-  dstart[tid] = ex;
-  goff[tid] = offs[(size_t)tid * tiles + blockIdx.x];
+  uint32_t tot, run = block_excl_scan_256(sum, wtot, &tot);  // its barriers end the counting
+#pragma unroll
+  for (int q = 0; q < DPT; ++q) {
+    goff[tid * DPT + q] = run + before[q];
+    run += all[q];
+  }
+  // prefix over the waves, then tile-level digit starts
+  uint32_t mine[DPT];
+  sum = 0u;
+#pragma unroll
+  for (int q = 0; q < DPT; ++q) {
+    uint32_t c = 0u;
+#pragma unroll
+    for (int ww = 0; ww < RS_WAVES; ++ww) {
+      const uint32_t x = wcnt[ww][tid * DPT + q];
+      wcnt[ww][tid * DPT + q] = c;
+      c += x;
+    }
+    mine[q] = c;
+    sum += c;
+  }
+  run = block_excl_scan_256(sum, wtot, &tot);
+#pragma unroll
+  for (int q = 0; q < DPT; ++q) {
+    dstart[tid * DPT + q] = run;
+    run += mine[q];
+  }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < RS_ITEMS; ++r) {
     const uint32_t i = wbase + (uint32_t)r * 64u + (uint32_t)lane;
     if (i < n) {
-      const uint32_t d = (k[r] >> shift) & 255u;
+      const uint32_t d = (k[r] >> shift) & (D - 1u);
       const uint32_t lp = dstart[d] + wcnt[w][d] + rk[r];
       sk[lp] = k[r];
       sv[lp] = v[r];
@@ -337,39 +399,61 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_downsweep(
   const uint32_t tile_n = min((uint32_t)RS_TILE, n - tile0);
   for (uint32_t i = tid; i < tile_n; i += RS_THREADS) {
     const uint32_t kk = sk[i];
-    const uint32_t d = (kk >> shift) & 255u;
+    const uint32_t d = (kk >> shift) & (D - 1u);
     const uint32_t o = goff[d] + (i - dstart[d]);
     kout[o] = kk;
     vout[o] = sv[i];
   }
 }
 
-int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uint32_t *v0,
-                     uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t **hist,
-                     size_t *hist_cap, ScanScratch *sc, hipStream_t s,
-                     const uint32_t **kout, const uint32_t **vout) {
-  *kout = kin;
-  *vout = vin;
-  if (n == 0) return SPH_OK;
-  const int passes = key_bits <= 0 ? 1 : (key_bits + 7) / 8;
-  const uint32_t tiles = (n + RS_TILE - 1) / RS_TILE;
-  const size_t need = (size_t)256 * tiles;
-  if (*hist_cap < need) {
-    if (*hist) SPH_HIP(hipFree(*hist));
-    *hist = nullptr;
-    SPH_HIP(hipMalloc(hist, sizeof(uint32_t) * need));
-    *hist_cap = need;
+// Digits of 8 bits, or of 10 where that saves a pass and the launches of a pass
+// weigh: a wider digit ranks with more ballots, holds more LDS (57 KB a block
+// against 39) and leaves shorter runs to write.  Measured for 20-bit keys, two
+// passes of 10 against three of 8, with the copy in and the wait: 1,000 pairs 45 /
+// 58 us, 30k 60 / 66, 300k 65 / 76, 1M 76 / 87, 4M 172 / 150.  Three of 10 for
+// 30-bit keys give nothing over four of 8 (1M: 107 / 100), nor do 11 bits for 22
+// (1M: 95 / 87).
+static void radix_digits(uint32_t n, int key_bits, int *bits, int *passes) {
+  *bits = 8;
+  *passes = key_bits <= 0 ? 1 : (key_bits + 7) / 8;
+  const int wide = (key_bits + 9) / 10;
+  if (n <= (1u << 21) && wide < *passes && wide <= 2) {
+    *bits = 10;
+    *passes = wide;
   }
-  const uint32_t *ck = kin, *cv = vin;
+}
+
+// A block sums the rows itself up to so many words per thread.
+constexpr uint32_t kRadixSelfWords = 32;
+
+size_t radix_words(uint32_t n, int key_bits) {
+  int bits = 8, passes = 1;
+  radix_digits(n, key_bits, &bits, &passes);
+  const size_t tiles = (n + RS_TILE - 1) / RS_TILE;
+  return ((size_t)1 << bits) * (tiles + 1);
+}
+
+template <int BITS>
+static int radix_passes(int passes, const uint32_t *ck, const uint32_t *cv, uint32_t *k0,
+                        uint32_t *v0, uint32_t *k1, uint32_t *v1, uint32_t n, uint32_t *hist,
+                        hipStream_t s, const uint32_t **kout, const uint32_t **vout) {
+  constexpr uint32_t D = 1u << BITS;
+  const uint32_t tiles = (n + RS_TILE - 1) / RS_TILE;
+  uint32_t *totals = hist + (size_t)D * tiles;
+  const bool self = D / RS_THREADS * tiles <= kRadixSelfWords;
   for (int p = 0; p < passes; ++p) {
     uint32_t *ok = (p & 1) ? k1 : k0;
     uint32_t *ov = (p & 1) ? v1 : v0;
-    const int shift = 8 * p;
-    k_radix_upsweep<<<tiles, RS_THREADS, 0, s>>>(ck, n, shift, *hist, tiles);
-    SPH_HIP(hipGetLastError());
-    int rc = scan(*hist, *hist, (uint32_t)need, false, false, sc, s, nullptr);
-    if (rc) return rc;
-    k_radix_downsweep<<<tiles, RS_THREADS, 0, s>>>(ck, cv, ok, ov, n, shift, *hist, tiles);
+    const int shift = BITS * p;
+    k_radix_upsweep<BITS><<<tiles, RS_THREADS, 0, s>>>(ck, n, shift, hist, tiles);
+    if (self) {
+      k_radix_downsweep<BITS, false><<<tiles, RS_THREADS, 0, s>>>(ck, cv, ok, ov, n, shift, hist,
+                                                                  nullptr, tiles);
+    } else {
+      k_radix_rows<<<D, RS_THREADS, 0, s>>>(hist, tiles, totals);
+      k_radix_downsweep<BITS, true><<<tiles, RS_THREADS, 0, s>>>(ck, cv, ok, ov, n, shift, hist,
+                                                                 totals, tiles);
+    }
     SPH_HIP(hipGetLastError());
     ck = ok;
     cv = ov;
@@ -379,19 +463,39 @@ int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uin
   return SPH_OK;
 }
 
+int radix_sort_pairs(const uint32_t *kin, const uint32_t *vin, uint32_t *k0, uint32_t *v0,
+                     uint32_t *k1, uint32_t *v1, uint32_t n, int key_bits, uint32_t *hist,
+                     hipStream_t s, const uint32_t **kout, const uint32_t **vout) {
+  *kout = kin;
+  *vout = vin;
+  if (n == 0) return SPH_OK;
+  int bits = 8, passes = 1;
+  radix_digits(n, key_bits, &bits, &passes);
+  const auto go = bits == 8 ? radix_passes<8> : radix_passes<10>;
+  return go(passes, kin, vin, k0, v0, k1, v1, n, hist, s, kout, vout);
+}
+
+// Counts of the keys below `cells`.  A run of equal keys in a wave (sorted keys
+// are nothing else) adds with one atomic: lanes of a run serialise on its word,
+// and a lower bound of a million sorted pairs took 46 us, now 24.
 __global__ void k_count_keys(const uint32_t *__restrict__ keys, uint32_t n,
                              uint32_t *__restrict__ count, uint32_t cells) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const uint32_t k = keys[i];
-    if (k < cells) atomicAdd(&count[k], 1u);
-  }
+  const int lane = threadIdx.x & 63;
+  const uint32_t k = i < n ? keys[i] : 0xFFFFFFFFu;
+  const uint32_t left = __shfl_up(k, 1, 64);
+  const bool first = lane == 0 || left != k;
+  const uint64_t firsts = __ballot(first);
+  const uint64_t after = lane == 63 ? 0ull : firsts >> (lane + 1);
+  const int next = after ? lane + 1 + __builtin_ctzll(after) : 64;
+  // the lanes of the last wave that lie past n end the last run, or are one
+  const uint32_t in = i < n ? min((uint32_t)(next - lane), n - i) : 0u;
+  if (first && i < n && k < cells) atomicAdd(&count[k], in);
 }
 
 int count_keys(const uint32_t *keys, uint32_t n, uint32_t *count, uint32_t cells,
                hipStream_t s) {
-  const uint32_t len = cells + 1;
-  k_fill_u32<<<blocks_for(len), kBlock, 0, s>>>(count, 0u, len);
+  k_fill_u32<<<blocks_for(cells), kBlock, 0, s>>>(count, 0u, cells);
   if (n) k_count_keys<<<blocks_for(n), kBlock, 0, s>>>(keys, n, count, cells);
   SPH_HIP(hipGetLastError());
   return SPH_OK;
@@ -416,7 +520,8 @@ struct AbiScratch {
   uint32_t *hist = nullptr;
   size_t hist_cap = 0;
   ScanScratch sc;
-  uint32_t *word = nullptr;  // one word for the key OR-reduction
+  uint32_t *word = nullptr;   // the keys' OR and the count of finished blocks
+  uint32_t *found = nullptr;  // the OR again, in pinned host memory
 };
 constexpr int kAbiDevices = 64;
 AbiScratch g_abi[kAbiDevices];
@@ -447,16 +552,63 @@ int abi_words(AbiScratch *w, size_t words) {
 }
 }  // namespace
 
-// OR of all keys (one device-scope atomic per wave): the highest set bit gives
-// the radix passes a 32-bit sort needs.
+// OR of all keys: the highest set bit gives the radix passes a 32-bit sort
+// needs.  One device-scope atomic per block (with one per wave, 4096 of them on
+// one word took 50 us); the last block to finish puts the result into pinned
+// host memory and both words back to zero for the next call.
+constexpr uint32_t kOrBlocks = 256;
 __global__ __launch_bounds__(kBlock) void k_or_keys(const uint32_t *__restrict__ keys,
-                                                    uint32_t n, uint32_t *__restrict__ out) {
+                                                    uint32_t n, uint32_t *words,
+                                                    uint32_t *found) {
+  __shared__ uint32_t part[kBlock / kWave];
   uint32_t v = 0;
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
     v |= keys[i];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v |= __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0 && v) atomicOr(out, v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kBlock / kWave; ++w) v |= part[w];
+    atomicOr(&words[0], v);
+    __threadfence();
+    if (atomicAdd(&words[1], 1u) == gridDim.x - 1u) {
+      *found = atomicExch(&words[0], 0u);
+      atomicExch(&words[1], 0u);
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_copy_pairs(uint32_t n, const uint32_t *__restrict__ k,
+                                                       const uint32_t *__restrict__ v,
+                                                       uint32_t *__restrict__ kout,
+                                                       uint32_t *__restrict__ vout) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  kout[i] = k[i];
+  vout[i] = v[i];
+}
+
+// The word pair and the pinned word of k_or_keys, on first use.
+static int or_words(AbiScratch *w, hipStream_t s) {
+  if (w->word && w->found) return SPH_OK;
+  hipError_t e = hipSuccess;
+  if (!w->word) {
+    e = hipMalloc(&w->word, 2 * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemsetAsync(w->word, 0, 2 * sizeof(uint32_t), s);
+    if (e != hipSuccess) {
+      if (w->word) (void)hipFree(w->word);
+      w->word = nullptr;
+      return hip_fail(e, "hipMalloc (key range)");
+    }
+  }
+  e = hipHostMalloc((void **)&w->found, sizeof(uint32_t), hipHostMallocDefault);
+  if (e != hipSuccess) {
+    w->found = nullptr;
+    return hip_fail(e, "hipHostMalloc (key range)");
+  }
+  return SPH_OK;
 }
 
 static int sort_impl(uint32_t *keys, uint32_t *values, int n, int key_bits, void *stream) {
@@ -472,31 +624,29 @@ static int sort_impl(uint32_t *keys, uint32_t *values, int n, int key_bits, void
   std::lock_guard<std::mutex> lock(w->m);
   if ((rc = abi_words(w, (size_t)n))) return rc;
   if (key_bits == 0) {  // unknown key range: from the keys' OR
-    if (!w->word) {
-      hipError_t e = hipMalloc(&w->word, sizeof(uint32_t));
-      if (e != hipSuccess) {
-        w->word = nullptr;
-        return hip_fail(e, "hipMalloc (key range)");
-      }
-    }
-    k_fill_u32<<<1, 64, 0, s>>>(w->word, 0u, 1u);
-    k_or_keys<<<std::min(blocks_for((uint32_t)n), 1024u), kBlock, 0, s>>>(keys, (uint32_t)n,
-                                                                          w->word);
+    if ((rc = or_words(w, s))) return rc;
+    k_or_keys<<<std::min(blocks_for((uint32_t)n), kOrBlocks), kBlock, 0, s>>>(
+        keys, (uint32_t)n, w->word, w->found);
     SPH_HIP(hipGetLastError());
-    uint32_t all = 0;
-    SPH_HIP(hipMemcpyAsync(&all, w->word, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     SPH_HIP(hipStreamSynchronize(s));
+    const uint32_t all = *(volatile uint32_t *)w->found;
     key_bits = all ? 32 - __builtin_clz(all) : 1;
   }
+  const size_t need = radix_words((uint32_t)n, key_bits);
+  if (w->hist_cap < need) {
+    if (w->hist) SPH_HIP(hipFree(w->hist));
+    w->hist = nullptr;
+    w->hist_cap = 0;
+    SPH_HIP(hipMalloc(&w->hist, sizeof(uint32_t) * need));
+    w->hist_cap = need;
+  }
   const uint32_t *kout = nullptr, *vout = nullptr;
-  rc = radix_sort_pairs(keys, values, w->a, w->b, keys, values, (uint32_t)n, key_bits, &w->hist,
-                        &w->hist_cap, &w->sc, s, &kout, &vout);
+  rc = radix_sort_pairs(keys, values, w->a, w->b, keys, values, (uint32_t)n, key_bits, w->hist, s,
+                        &kout, &vout);
   if (rc == SPH_OK && kout != keys) {
-    hipError_t e =
-        hipMemcpyAsync(keys, kout, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(values, vout, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) rc = hip_fail(e, "hipMemcpyAsync (sort result)");
+    k_copy_pairs<<<blocks_for((uint32_t)n), kBlock, 0, s>>>((uint32_t)n, kout, vout, keys, values);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = hip_fail(e, "k_copy_pairs");
   }
   const hipError_t e = hipStreamSynchronize(s);
   if (rc == SPH_OK && e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize (sort)");
@@ -522,19 +672,18 @@ extern "C" int sph_sort_by_key(uint32_t *keys, uint32_t *values, int n, void *st
 // --------------------------------------------------------------------------
 // For callers that cannot allocate device memory (code under stream capture,
 // serving loops, harnesses that forbid hipMalloc).  Layout, in words: the two
-// ping-pong buffers (kStaticPairs each), the digit histogram (256 per 4096-key
-// tile) and the scan's tile sums; each part starts on a 16-byte boundary.
+// ping-pong buffers (kStaticPairs each) and the digit histogram with its totals
+// (for the widest digits); each part starts on a 16-byte boundary.
 namespace {
 constexpr size_t kStaticPairs = size_t(1) << 21;
 constexpr size_t kStaticTiles = (kStaticPairs + RS_TILE - 1) / RS_TILE;
-constexpr size_t kStaticHist = 256 * kStaticTiles;
-constexpr size_t kStaticScanTiles = (kStaticHist + SC_TILE - 1) / SC_TILE;
-constexpr size_t kStaticWords = 2 * kStaticPairs + kStaticHist + ((kStaticScanTiles + 3) & ~3ull);
+constexpr size_t kStaticHist = 1024 * (kStaticTiles + 1);
+constexpr size_t kStaticWords = 2 * kStaticPairs + kStaticHist;
 static_assert(kStaticPairs % 4 == 0 && kStaticHist % 4 == 0, "16-byte aligned parts");
 static_assert(kStaticPairs == SPH_SORT_NOALLOC_MAX_PAIRS, "header limit");
 }  // namespace
 
-// Each GPU holds its own copy until the process ends (about 17 MB).
+// Each GPU holds its own copy until the process ends (about 19 MB).
 static __device__ __align__(256) uint32_t scratch[kStaticWords];
 
 namespace {
@@ -577,21 +726,14 @@ extern "C" int sph_sort_by_key_bits_noalloc(uint32_t *keys, uint32_t *values, in
   int rc = static_scratch(&base);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  uint32_t *a = base, *b = base + kStaticPairs;
-  uint32_t *hist = base + 2 * kStaticPairs;
-  size_t hist_cap = kStaticHist;  // large enough: radix_sort_pairs allocates nothing
-  ScanScratch sc;
-  sc.tile_sums = hist + kStaticHist;
-  sc.tile_cap = kStaticScanTiles;
+  uint32_t *a = base, *b = base + kStaticPairs, *hist = base + 2 * kStaticPairs;
   const uint32_t *kout = nullptr, *vout = nullptr;
-  rc = radix_sort_pairs(keys, values, a, b, keys, values, (uint32_t)n, key_bits, &hist,
-                        &hist_cap, &sc, s, &kout, &vout);
+  rc = radix_sort_pairs(keys, values, a, b, keys, values, (uint32_t)n, key_bits, hist, s, &kout,
+                        &vout);
   if (rc) return rc;
   if (kout != keys) {  // an odd number of passes ends in the scratch buffers
-    SPH_HIP(hipMemcpyAsync(keys, kout, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice,
-                           s));
-    SPH_HIP(hipMemcpyAsync(values, vout, sizeof(uint32_t) * (size_t)n,
-                           hipMemcpyDeviceToDevice, s));
+    k_copy_pairs<<<blocks_for((uint32_t)n), kBlock, 0, s>>>((uint32_t)n, kout, vout, keys, values);
+    SPH_HIP(hipGetLastError());
   }
   return SPH_OK;
 }
@@ -608,17 +750,9 @@ static int bounds_impl(const uint32_t *keys, int n, int cells, uint32_t *out, vo
   int rc = abi_scratch(&w);
   if (rc) return rc;
   std::lock_guard<std::mutex> lock(w->m);
-  if ((rc = abi_words(w, (size_t)cells + 1))) return rc;
-  uint32_t *count = w->a, *start = w->b;
-  rc = count_keys(keys, (uint32_t)n, count, (uint32_t)cells, s);
-  if (rc == SPH_OK)
-    rc = scan(count, start, (uint32_t)cells, false, true, &w->sc, s, nullptr);
-  if (rc == SPH_OK) {
-    const hipError_t e = hipMemcpyAsync(out, start + (upper ? 1 : 0),
-                                        sizeof(uint32_t) * (size_t)cells,
-                                        hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) rc = hip_fail(e, "hipMemcpyAsync (bounds)");
-  }
+  if ((rc = abi_words(w, (size_t)cells))) return rc;
+  rc = count_keys(keys, (uint32_t)n, w->a, (uint32_t)cells, s);
+  if (rc == SPH_OK) rc = scan(w->a, out, (uint32_t)cells, upper, false, &w->sc, s, nullptr);
   const hipError_t e = hipStreamSynchronize(s);
   if (rc == SPH_OK && e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize (bounds)");
   return rc;

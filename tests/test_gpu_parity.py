@@ -59,6 +59,32 @@ def test_sort_by_key_bit_exact(n, bits, hi, adaptive):
         assert np.array_equal(k, k2) and np.array_equal(v, v2)
 
 
+@pytest.mark.parametrize("bits", [1, 9, 10, 11, 17, 20, 21, 30, 31])
+@pytest.mark.parametrize("n", [2, 8 * 4096, 8 * 4096 + 1, 32 * 4096 + 1, (1 << 21) + 1])
+def test_sort_at_the_limits_of_its_digits(n, bits):
+    """10-bit digits where they save a pass, up to 2^21 pairs; rows of the
+    histogram summed by the blocks themselves up to 8 (10 bits) or 32 tiles."""
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n, dtype=np.uint64).astype(np.uint32)
+    vals = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    order = np.argsort(keys, kind="stable")
+    for kb in (bits, None):
+        k, v = sa.sort_by_key(keys, vals, kb)
+        assert np.array_equal(k, keys[order]) and np.array_equal(v, vals[order])
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 100_001])
+def test_cell_bounds_of_unsorted_keys(n):
+    """The bounds count, so keys in any order give the same table; runs of equal
+    keys across wavefronts and at the ragged end."""
+    keys = np.random.default_rng(n).integers(0, 7, n).astype(np.uint32)
+    keys[-3:] = 6
+    lo, hi = sa.cell_bounds(keys, 6)
+    c, k = np.arange(6, dtype=np.uint32), np.sort(keys)
+    assert np.array_equal(lo, np.searchsorted(k, c, "left"))
+    assert np.array_equal(hi, np.searchsorted(k, c, "right"))
+
+
 @pytest.mark.parametrize("n,cells", [(0, 10), (1, 1), (5000, 997), (300_000, 1_000_000)])
 def test_cell_bounds_bit_exact(n, cells):
     rng = np.random.default_rng(cells)
