@@ -345,8 +345,8 @@ typedef struct sph_tuning {
 } sph_tuning;
 int sph_autotune(sph_ctx *ctx, int substeps, sph_tuning *result);
 /* The context's current launch choices (timings zero), and applying a saved
- * set: block 0 / depth 0 keep the default (256 threads, 16 gathers); other
- * values must be 64, 128 or 256 and 8, 16 or 32.  Entries of kernels that
+ * set: block 0 / depth 0 keep the default (by kernel and particle count);
+ * other values must be 64, 128 or 256 and 8, 16 or 32.  Entries of kernels that
  * are not tuned are ignored. */
 int sph_get_tuning(sph_ctx *ctx, sph_tuning *out);
 int sph_set_tuning(sph_ctx *ctx, const sph_tuning *tuning);

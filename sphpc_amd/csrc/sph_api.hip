@@ -1429,12 +1429,15 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
   uint16_t best_bs[K_COUNT] = {};
   for (int k = 0; k < K_COUNT; ++k) best[k] = 1e300;
   const uint16_t sizes[3] = {64, 128, 256};
+  if (e == hipSuccess) {
+    graph_reset(c);
+    rc = trial(cur, &before);  // as the context was
+  }
   for (int b = 0; b < 3 && e == hipSuccess && !rc; ++b) {
     for (int k : kTunable) c->tune.block[k] = sizes[b];
     graph_reset(c);
     rc = trial(cur, &total);
     if (rc) break;
-    if (sizes[b] == 256) before = total;
     for (int k : kTunable)
       if (cur[k] > 0.0 && cur[k] < best[k]) {
         best[k] = cur[k];

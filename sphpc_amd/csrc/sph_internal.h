@@ -234,9 +234,12 @@ struct sph_ctx {
   sph::BatchDev batch() const { return sph::BatchDev{scenes_dev, scene_of}; }
   // launch choices (sph_autotune)
   struct {
-    bool split_collide = true;  // obstacle push as its own pass after k_dp_update
-    uint16_t block[sph::K_COUNT] = {};  // threads per block of gather kernels (0: 256)
-    uint8_t depth[sph::K_COUNT] = {};   // gathers in flight per wave: 8, 16, 32 (0: 16)
+    // obstacle push as its own pass after k_dp_update: slower at every size (with
+    // the push fused a frame's kernels take 3.7 ms instead of 4.3 at 131k
+    // particles, 7.9 instead of 8.1 at 1M, 60.2 instead of 60.8 at 8.4M)
+    bool split_collide = false;
+    uint16_t block[sph::K_COUNT] = {};  // threads per block of gather kernels (0: by rule)
+    uint8_t depth[sph::K_COUNT] = {};   // gathers in flight per wave: 8, 16, 32 (0: by rule)
     bool wide_lists = false;  // 32-bit list entries for every wave
   } tune;
   // whole-substep HIP graph (sph_set_graph)

@@ -1191,10 +1191,9 @@ __global__ __launch_bounds__(kBlock) void k_position_stars(uint32_t n, float4 *_
 }
 
 // Fused UpdateDPs + UpdatePositionStars: reads pin (x*, lambda), writes pout
-// (x*', rho).  COLLIDE false leaves the obstacle to k_collide_sorted: the
-// inlined trilinear gradient doubles the kernel's registers (109 vs 58 VGPRs)
-// and halves its occupancy, for a push that only particles inside the SDF box
-// need.  In tolerance mode, once the density pass of this iteration is
+// (x*', rho).  COLLIDE false leaves the obstacle to k_collide_sorted (a launch
+// choice; the trilinear gradient needs no more registers than the gathers).  In
+// tolerance mode, once the density pass of this iteration is
 // within tolerance, the particles are copied unchanged instead.  With lam_acc,
 // adds stiff * lambda_i to the particle's accumulated multiplier.
 template <bool COLLIDE, bool BATCH, int NB>
@@ -1829,10 +1828,22 @@ __global__ __launch_bounds__(kBlock) void k_kinetic_energy(uint32_t n,
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-// Gathers in flight per wave of a gather kernel: the autotuner's choice or 16.
+// Kernels that end in a block's maximum and its atomic, in place of none.
+static inline bool reduces_error(int kernel) {
+  return kernel == K_DENSITY_LAMBDA || kernel == K_DENSITY || kernel == K_LAMBDA ||
+         kernel == K_WARM_LAMBDA;
+}
+
+// Gathers in flight per wave of a gather kernel where neither the autotuner nor
+// the caller chose: 16, and 8 where the chip holds all waves at once anyway and
+// 8 let more of them in per SIMD (70 VGPRs).  Measured (us, events included), 16 /
+// 8: 133k particles delta p 11.1 / 10.7, XSPH 14.7 / 13.8, vorticity 15.8 / 14.9;
+// 439k 22.4 / 21.1, 33.8 / 33.3, 35.8 / 35.2; but surface at 681k 48.8 / 50.6, 1M
+// 70.1 / 76.8, and the density pass at every size (439k: 36 / 40).
 static inline int tuned_depth(const sph_ctx *c, int kernel) {
   const int d = c->tune.depth[kernel];
-  return d ? d : 16;
+  if (d) return d;
+  return c->n <= (1 << 19) && !reduces_error(kernel) ? 8 : 16;
 }
 
 template <typename F>
@@ -1845,10 +1856,23 @@ static inline void with_depth(int depth, F &&f) {
     f(std::integral_constant<int, 16>{});
 }
 
-// Threads per block of a gather kernel: the autotuner's choice or kBlock.
+// Threads per block of a gather kernel where neither the autotuner nor the
+// caller chose.  A block of one wave frees its place as soon as that wave ends
+// and, of few particles, spreads the waves over the CUs (a wave's gathers keep a
+// vector L1 busy): surface 10.8 -> 8.8 us at 4k particles, 79.2 -> 70.1 at 1M
+// (256 / 64 threads, events included), XSPH 10.2 -> 7.9 and 75.3 -> 69.9, delta p
+// 8.5 -> 7.7 and 46.1 -> 42.5.  At 8.4M the neighbouring waves of a larger block
+// share more lines: colour 363 / 370, confinement 394 / 400, delta p 327 (128) /
+// 329, but surface 616 / 597.  The density passes pay an atomic per block: 256
+// threads are fastest up to 64k (11.9 against 13.3 and 12.6), 128 from 90k up (1M:
+// 52.5 against 55.0 and 56.3).
 static inline uint32_t tuned_block(const sph_ctx *c, int kernel) {
   const uint32_t b = c->tune.block[kernel];
-  return b ? b : (uint32_t)kBlock;
+  if (b) return b;
+  if (kernel == K_BUILD_LISTS) return (uint32_t)kBlock;
+  if (reduces_error(kernel)) return c->n <= (1 << 16) ? (uint32_t)kBlock : 128u;
+  if (c->n <= (1 << 21) || kernel == K_SURFACE) return 64u;
+  return kernel == K_DP || kernel == K_DP_UPDATE ? 128u : (uint32_t)kBlock;
 }
 
 #define LAUNCH_TIMED(ctx, kid, grid, ...)                               \
