@@ -187,7 +187,7 @@ static void free_all(sph_ctx *c) {
   graph_reset(c);
   void *bufs[] = {c->x_can, c->v_can, c->xs_can, c->keys, c->cell_rank, c->slots,
                   c->key_s, c->id_s, c->cell_count, c->cell_start, c->pos_a, c->pos_b, c->xold,
-                  c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage, c->lam_stage,
+                  c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage,
                   c->list, c->list_head,
                   c->stats, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
                   c->pw, c->sx, c->lam_acc, c->lam_prev, c->feat, c->scenes_dev, c->scene_of,
@@ -297,7 +297,6 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       {(void **)&c->vel_b, f4},       {(void **)&c->aux, f4},
       {(void **)&c->dpbuf, f4},       {(void **)&c->rho, sizeof(float) * cap},
       {(void **)&c->cstage, sizeof(float) * cap},
-      {(void **)&c->lam_stage, sizeof(float) * cap},
       {(void **)&c->list, sizeof(uint32_t) * groups * kListStride},
       {(void **)&c->list_head, sizeof(uint4) * cap},
       {(void **)&c->pw, f4},
@@ -821,8 +820,9 @@ extern "C" int sph_compute_densities(sph_ctx *c) {
   c->staged_slot++;
   c->last_err_slot = slot;
   // density_to_w keeps rho in pos.w for the velocity passes.  With a fixed
-  // iteration count the same gather also computes lambda and keeps it aside
-  // for an immediately following sph_compute_lambda.
+  // iteration count the same gather also computes lambda and writes (x*, lambda)
+  // to the other position buffer, for an immediately following
+  // sph_compute_lambda to switch to.
   if (c->P.density_tolerance > 0.0) return launch_density(c, 3, slot);
   if ((rc = launch_density(c, 4, slot))) return rc;
   c->lam_gen = c->gen;
@@ -835,7 +835,9 @@ extern "C" int sph_compute_lambda(sph_ctx *c) {
   const bool fresh = c && c->lam_gen == c->gen;
   int rc = require_lists(c);
   if (rc) return rc;
-  return fresh ? launch_lambda_from_density(c) : launch_density(c, 2, -1);
+  if (!fresh) return launch_density(c, 2, -1);
+  c->pos = c->pos == c->pos_a ? c->pos_b : c->pos_a;
+  return SPH_OK;
 }
 
 extern "C" int sph_update_dps(sph_ctx *c, int substep) {

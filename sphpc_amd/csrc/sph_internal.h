@@ -137,8 +137,8 @@ struct MlpPacked {
   float b3;
 };
 
-// The order is that of sph_profile_kernel_name and of saved tunings; the two
-// radix entries stay for it (the search has counted by cell since).
+// The order is that of sph_profile_kernel_name and of saved tunings; the radix
+// and lambda_copy entries stay for it (nothing launches them in a context).
 enum KernelId {
   K_PREDICT_HASH = 0, K_HASH, K_GRAVITY, K_PREDICT, K_RADIX_UP, K_RADIX_DOWN, K_SCAN,
   K_REORDER, K_BUILD_LISTS, K_DENSITY_LAMBDA, K_DENSITY, K_LAMBDA, K_DP, K_DP_UPDATE,
@@ -198,8 +198,8 @@ struct sph_ctx {
   float4 *dpbuf = nullptr;  // staged delta p
   float *rho = nullptr;
   // stage path: C = rho/rho0 - 1 of the last density stage (read by a lambda
-  // stage that runs its own gather) and the lambda that density pass computed
-  float *cstage = nullptr, *lam_stage = nullptr;
+  // stage that runs its own gather)
+  float *cstage = nullptr;
   uint32_t *list = nullptr;     // sorted neighbour indices, quads of slots per 64 particles
   uint4 *list_head = nullptr;   // per sorted particle: layer bases and counts
   // state transfers: x, y, z, vx, vy, vz of up to cap particles in pinned host
@@ -256,8 +256,8 @@ struct sph_ctx {
   int last_err_slot = -1;
   int staged_slot = 0;
   // state generation: bumped by every call that may change the state; the
-  // stage path's density pass records it, and the lambda stage reuses that
-  // pass's lambda when nothing ran in between
+  // stage path's density pass records it, and the lambda stage switches to the
+  // buffer with that pass's lambda when nothing ran in between
   unsigned long long gen = 0, lam_gen = ~0ull;
   unsigned long long dp_gen = ~0ull;  // likewise the delta-p stage's updated x*
   float4 *dp_next = nullptr;
@@ -307,9 +307,8 @@ int launch_predict(sph_ctx *c);
 int launch_neighbor_search(sph_ctx *c, bool fused);
 // mode 0: density + lambda (fused substep), 1: density, 2: lambda, 3: density
 // with rho into pos.w (tolerance loop), 4: density + lambda with rho into pos.w
-// and lambda into dpbuf (the stage path; launch_lambda_from_density moves it)
+// and (x*, lambda) into the other position buffer (the stage path)
 int launch_density(sph_ctx *c, int mode, int err_slot);
-int launch_lambda_from_density(sph_ctx *c);
 // xnext: also the position update of launch_position_stars, into xnext
 int launch_dp(sph_ctx *c, int substep, float4 *xnext = nullptr);
 int launch_position_stars(sph_ctx *c);

@@ -1002,14 +1002,14 @@ __device__ __forceinline__ float density_constraint(uint32_t S, int cnt, const D
 // in one gather: rho_i needs only r^2, lambda_i needs C_i (own) and the
 // spiky gradients.  Writes rho and pos.w = lambda.
 // MODE 0: both, 1: density only, 2: lambda only (C from c_io).  With c_io,
-// MODE 0/1 also store C there; with lam_out, lambda goes there and pos.w
-// keeps rho (density_to_w).
+// MODE 0/1 also store C there; with with_lambda, (x*, lambda) goes to that
+// buffer and pos.w keeps rho (density_to_w).
 template <int MODE, int NB>
 __global__ GATHER_BOUNDS(NB) void k_density_lambda(
     uint32_t n, uint32_t nblocks, float4 *pos, const uint32_t *__restrict__ list,
     const uint4 *__restrict__ head, DevParams P, float *__restrict__ rho_out, float *c_io,
     uint32_t *stats, int err_slot, int check_converged, int density_to_w,
-    float *__restrict__ lam_out) {
+    float4 *__restrict__ with_lambda) {
   if (check_converged && converged(stats)) return;
   const uint32_t s = particle_index(nblocks);
   const bool active = s < n;
@@ -1054,8 +1054,8 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
       const float Ci = fmaxf(C, 0.0f);
       const float sum_c = P.lam_k2 * (sc + sq3(sgx, sgy, sgz));
       const float lam = -Ci / (sum_c + P.lambda_eps);
-      if (lam_out)
-        lam_out[s] = lam;  // pos.w keeps rho (density_to_w)
+      if (with_lambda)
+        with_lambda[s] = make_float4(p.x, p.y, p.z, lam);
       else
         pos[s].w = lam;
     }
@@ -2021,13 +2021,13 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        n, nb, c->pos, c->list, c->list_head, c->dev, c->rho, c->cstage, c->stats,
                        err_slot, 0, 0, nullptr));
     });
-  else if (mode == 4)  // density and lambda in one gather: rho into w, lambda aside
+  else if (mode == 4)  // density and lambda in one gather: rho into w, (x*, lambda) aside
     with_depth(tuned_depth(c, K_DENSITY_LAMBDA), [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_DENSITY_LAMBDA, 0,
                    k_density_lambda<0, NBv><<<nb, bs, 0, s>>>(
                        n, nb, c->pos, c->list, c->list_head, c->dev, c->rho, c->cstage, c->stats,
-                       err_slot, 0, 1, c->lam_stage));
+                       err_slot, 0, 1, c->pos == c->pos_a ? c->pos_b : c->pos_a));
     });
   else if (mode == 3)  // final density of a capped tolerance loop: rho also into w
     with_depth(tuned_depth(c, K_DENSITY), [&](auto D_) {
@@ -2045,22 +2045,6 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        n, nb, c->pos, c->list, c->list_head, c->dev, c->rho, c->cstage, c->stats,
                        -1, 0, 0, nullptr));
     });
-  SPH_HIP(hipGetLastError());
-  return SPH_OK;
-}
-
-// pos.w = the lambda a mode-4 density pass put aside.
-__global__ __launch_bounds__(kBlock) void k_lambda_to_w(uint32_t n, const float *__restrict__ lam,
-                                                        float4 *__restrict__ pos) {
-  const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-  if (s < n) pos[s].w = lam[s];
-}
-
-int launch_lambda_from_density(sph_ctx *c) {
-  const uint32_t n = c->n;
-  if (!n) return SPH_OK;
-  LAUNCH_TIMED(c, K_LAMBDA_COPY, 0,
-               k_lambda_to_w<<<blocks_for(n), kBlock, 0, c->stream>>>(n, c->lam_stage, c->pos));
   SPH_HIP(hipGetLastError());
   return SPH_OK;
 }
