@@ -1863,14 +1863,12 @@ static inline void with_depth(int depth, F &&f) {
 // (256 / 64 threads, events included), XSPH 10.2 -> 7.9 and 75.3 -> 69.9, delta p
 // 8.5 -> 7.7 and 46.1 -> 42.5.  At 8.4M the neighbouring waves of a larger block
 // share more lines: colour 363 / 370, confinement 394 / 400, delta p 327 (128) /
-// 329, but surface 616 / 597.  The density passes pay an atomic per block: 256
-// threads are fastest up to 64k (11.9 against 13.3 and 12.6), 128 from 90k up (1M:
-// 52.5 against 55.0 and 56.3).
+// 329, but surface 616 / 597.  The density passes pay an atomic per block on one
+// word and keep 256 (442k: 26.5 us against 30.0 at 128 and 36 at 64).
 static inline uint32_t tuned_block(const sph_ctx *c, int kernel) {
   const uint32_t b = c->tune.block[kernel];
   if (b) return b;
-  if (kernel == K_BUILD_LISTS) return (uint32_t)kBlock;
-  if (reduces_error(kernel)) return c->n <= (1 << 16) ? (uint32_t)kBlock : 128u;
+  if (kernel == K_BUILD_LISTS || reduces_error(kernel)) return (uint32_t)kBlock;
   if (c->n <= (1 << 21) || kernel == K_SURFACE) return 64u;
   return kernel == K_DP || kernel == K_DP_UPDATE ? 128u : (uint32_t)kBlock;
 }
