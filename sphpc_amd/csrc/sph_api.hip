@@ -189,7 +189,7 @@ static void free_all(sph_ctx *c) {
                   c->key_s, c->id_s, c->cell_count, c->cell_start, c->pos_a, c->pos_b, c->xold,
                   c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage,
                   c->list, c->list_head,
-                  c->stats, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
+                  c->stats, c->stats_read, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
                   c->pw, c->sx, c->lam_acc, c->lam_prev, c->feat, c->scenes_dev, c->scene_of,
                   c->batch_sdf, c->scene_err, c->scene_err0, c->scene_chunks,
                   c->warm_net};
@@ -305,6 +305,7 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       // their placing, which zeroes them
       {(void **)&c->scan.tile_sums, sizeof(uint32_t) * scan_tiles(c->cells)},
       {(void **)&c->stats, sizeof(uint32_t) * STAT_WORDS},
+      {(void **)&c->stats_read, sizeof(uint32_t) * STAT_READ_WORDS},
       {(void **)&c->pair_partial, sizeof(uint32_t) * blocks_for((uint32_t)cap, kWave)},
       {(void **)&c->red, sizeof(double) * std::max<size_t>(4, blocks_for((uint32_t)cap))},
   };
@@ -1111,11 +1112,25 @@ extern "C" int sph_synchronize(sph_ctx *c) {
   return SPH_OK;
 }
 
+static int fetch_stats(sph_ctx *c, std::vector<uint32_t> *w) {
+  const int rc = launch_collect_stats(c);
+  return rc ? rc : fetch(c, (const uint32_t *)c->stats_read, STAT_READ_WORDS, w);
+}
+
+// Maximum density error of iteration `it` of fetched statistics; a single scene
+// that fell back from its warm start went on from the error before it.
+static float fetched_error(const sph_ctx *c, const std::vector<uint32_t> &w, int it) {
+  if (it == 1 && !c->nscenes && w[STAT_FALLBACK]) it = 0;
+  float f;
+  memcpy(&f, &w[STAT_ERR0 + it], sizeof(f));
+  return f;
+}
+
 extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
   if (!c || !st) return arg_error("NULL argument");
-  uint32_t w[STAT_WORDS];
-  SPH_HIP(hipMemcpyAsync(w, c->stats, sizeof(w), hipMemcpyDeviceToHost, c->stream));
-  SPH_HIP(hipStreamSynchronize(c->stream));
+  std::vector<uint32_t> w;
+  int rc = fetch_stats(c, &w);
+  if (rc) return rc;
   memset(st, 0, sizeof(*st));
   st->particles = c->n;
   st->iterations = (int)w[STAT_ITERS];
@@ -1123,11 +1138,7 @@ extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
   st->warm_fallback = (int)w[STAT_FALLBACK];
   int slot = c->last_err_slot;
   if (c->P.density_tolerance > 0.0 && st->converged) slot = st->iterations;
-  if (slot >= 0 && slot <= kMaxIters) {
-    float f;
-    memcpy(&f, &w[STAT_ERR0 + slot], sizeof(f));
-    st->max_density_error = f;
-  }
+  if (slot >= 0 && slot <= kMaxIters) st->max_density_error = fetched_error(c, w, slot);
   st->neighbor_overflow = (unsigned long long)w[STAT_DROPPED] |
                           ((unsigned long long)w[STAT_DROPPED + 1] << 32);
   st->cell_clamps =
@@ -1135,7 +1146,7 @@ extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
   st->substeps = c->substeps;
   if (c->pair_blocks) {
     std::vector<uint32_t> part;
-    int rc = fetch(c, (const uint32_t *)c->pair_partial, c->pair_blocks, &part);
+    rc = fetch(c, (const uint32_t *)c->pair_partial, c->pair_blocks, &part);
     if (rc) return rc;
     unsigned long long sum = 0;
     for (uint32_t v : part) sum += v;
@@ -1146,15 +1157,15 @@ extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
 
 extern "C" int sph_get_residuals(sph_ctx *c, float *err, int cap, int *count) {
   if (!c || !err || !count) return arg_error("NULL argument");
-  uint32_t w[STAT_WORDS];
-  SPH_HIP(hipMemcpyAsync(w, c->stats, sizeof(w), hipMemcpyDeviceToHost, c->stream));
-  SPH_HIP(hipStreamSynchronize(c->stream));
+  std::vector<uint32_t> w;
+  int rc = fetch_stats(c, &w);
+  if (rc) return rc;
   // one density pass before each applied update; with a tolerance, one more
   // (the pass that met it, or the final pass after the capped loop)
   const int applied = (int)w[STAT_ITERS];
   int passes = c->P.density_tolerance > 0.0 ? applied + 1 : applied;
   passes = std::max(0, std::min(passes, std::min(cap, kMaxIters + 1)));
-  for (int k = 0; k < passes; ++k) memcpy(&err[k], &w[STAT_ERR0 + k], sizeof(float));
+  for (int k = 0; k < passes; ++k) err[k] = fetched_error(c, w, k);
   *count = passes;
   return SPH_OK;
 }

@@ -108,10 +108,19 @@ enum StatSlot {
   STAT_ITERS = 4,
   STAT_CONVERGED = 5,
   STAT_FALLBACK = 6,     // warm start reverted to the plain first iteration
-  STAT_ERR0 = 8,         // per-iteration max error bits (kMaxIters + 1 slots)
-  STAT_WORDS = 256
+  STAT_ERR0 = 64         // max error bits, kErrSlots lines for each iteration
 };
 constexpr int kMaxIters = 128;
+// A density pass spreads its error maximum over 64 words (a wave reads them in
+// one load), each on a 128-byte line of its own: atomics to one line take about
+// 4 ns each, whichever of its words.
+constexpr uint32_t kErrSlots = 64, kErrStride = 32;
+constexpr uint32_t err_word(uint32_t it, uint32_t slot) {
+  return STAT_ERR0 + (it * kErrSlots + slot) * kErrStride;
+}
+constexpr uint32_t STAT_WORDS = err_word(kMaxIters + 1u, 0u);
+// The statistics as the host reads them: the flags, then a word per iteration.
+constexpr uint32_t STAT_READ_WORDS = STAT_ERR0 + kMaxIters + 1;
 
 // Lambda warm-start network: 12 features (padded to 16) -> 64 SiLU -> 64 SiLU -> 1.
 // FP32 master parameters in one vector: W1[16][64] (row = input), b1[64],
@@ -207,6 +216,7 @@ struct sph_ctx {
   float *io_host = nullptr;
   hipEvent_t io_done[sph::kIoChunks] = {};
   uint32_t *stats = nullptr;  // sph::STAT_WORDS words
+  uint32_t *stats_read = nullptr;  // sph::STAT_READ_WORDS words
   uint32_t *pair_partial = nullptr;  // per-block list-length sums of the last search
   uint32_t pair_blocks = 0;
   double *red = nullptr;      // FP64 reduction scratch
@@ -320,6 +330,7 @@ int launch_xsph(sph_ctx *c);
 int launch_vorticity(sph_ctx *c);
 int launch_confine(sph_ctx *c, bool commit);
 int launch_commit(sph_ctx *c);
+int launch_collect_stats(sph_ctx *c);
 int launch_collide_soa(float *x, float *y, float *z, uint32_t n, const SdfDev &o,
                        hipStream_t s);
 int launch_collide_soa_f64(double *x, double *y, double *z, uint32_t n, const SdfDev &o,

@@ -435,13 +435,14 @@ __device__ __forceinline__ uint32_t count_into_cell(uint32_t *__restrict__ cell_
   return __shfl(old, head, 64) + (uint32_t)(lane - head);
 }
 
-// Substep bookkeeping: clears the per-iteration error slots and flags, from the
-// search's first kernel (nothing of it uses them).  No hipMemsetAsync, so that
-// the substep can be captured in a graph.
-__device__ __forceinline__ void clear_substep_stats(uint32_t *stats) {
-  static_assert(STAT_WORDS <= kBlock, "one block clears the statistics");
-  if (blockIdx.x == 0 && threadIdx.x >= STAT_ITERS && threadIdx.x < STAT_WORDS)
-    stats[threadIdx.x] = 0u;
+// Substep bookkeeping: clears the flags and the error words of iterations up to
+// `last`, from the search's first kernel (nothing of it uses them).  No
+// hipMemsetAsync, so that the substep can be captured in a graph.
+__device__ __forceinline__ void clear_substep_stats(uint32_t *stats, uint32_t last) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= STAT_ITERS && i < STAT_ERR0) stats[i] = 0u;
+  for (uint32_t e = i; e < (last + 1u) * kErrSlots; e += gridDim.x * kBlock)
+    stats[err_word(0u, e)] = 0u;
 }
 
 // HashParticles (neighbors.c:101-125).
@@ -450,8 +451,9 @@ __global__ __launch_bounds__(kBlock) void k_hash(uint32_t n, const float4 *__res
                                                  uint32_t *__restrict__ keys,
                                                  uint32_t *__restrict__ cell_rank,
                                                  uint32_t *__restrict__ cell_count, DevParams P,
-                                                 uint32_t *__restrict__ stats, BatchDev B) {
-  clear_substep_stats(stats);
+                                                 uint32_t *__restrict__ stats,
+                                                 uint32_t last_error, BatchDev B) {
+  clear_substep_stats(stats, last_error);
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   const bool valid = i < n;
   uint32_t clamped = 0, key = 0;
@@ -479,8 +481,8 @@ __global__ __launch_bounds__(kBlock) void k_predict_hash(uint32_t n,
                                                          uint32_t *__restrict__ cell_count,
                                                          DevParams P,
                                                          uint32_t *__restrict__ stats,
-                                                         BatchDev B) {
-  clear_substep_stats(stats);
+                                                         uint32_t last_error, BatchDev B) {
+  clear_substep_stats(stats, last_error);
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   const bool valid = i < n;
   uint32_t clamped = 0, key = 0;
@@ -945,27 +947,29 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
 // ---------------------------------------------------------------------------
 // Jacobi constraint loop
 // ---------------------------------------------------------------------------
-// Max of a non-negative float over a block, then at most one atomic on the
-// float's bit pattern (monotonic for non-negative floats).  The slot only
-// grows during a launch, so a block whose maximum does not exceed the value it
-// reads skips the atomic; without this every block would issue a device-scope
-// atomic to one address.  Every thread of the block must call it.  With one
-// read and atomic per wave instead, each wave waited for that round trip at
-// its end: per block, the density pass measured 1.6% faster at 8M particles.
-__device__ __forceinline__ void block_max_to(uint32_t *slot, float v, bool active) {
-  __shared__ float bm[kBlock / kWave];
+// The error maximum of a density pass: a wave's maximum of a non-negative float,
+// then one atomic on its bit pattern (monotonic for non-negative floats) on the
+// iteration's word for the wave's number, which nothing waits for.  Without the
+// error the density pass takes 39.8 us at 1M particles and 6.0 at 32k.  With one
+// word, read and if need be raised by each block at its end, it took 45.2 and 7.9
+// (a barrier and a memory round trip a block); an atomic per
+// wave costs 40.8 and 6.9.
+// Every lane of the wave must call it.
+__device__ __forceinline__ void raise_error(uint32_t *stats, int it, float v, bool active) {
   float m = active ? v : 0.0f;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0) bm[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (uint32_t w = 1; w < blockDim.x / kWave; ++w) m = fmaxf(m, bm[w]);
-    if (m > 0.0f) {
-      const uint32_t bits = __float_as_uint(m);
-      if (bits > *(volatile uint32_t *)slot) atomicMax(slot, bits);
-    }
-  }
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  if ((threadIdx.x & 63) == 0 && m > 0.0f)
+    atomicMax(&stats[err_word((uint32_t)it, wave & (kErrSlots - 1u))], __float_as_uint(m));
+}
+
+// The maximum an iteration's waves left (bits), in every lane of the wave.
+__device__ __forceinline__ uint32_t max_error(const uint32_t *stats, int it) {
+  uint32_t m = stats[err_word((uint32_t)it, threadIdx.x & (kErrSlots - 1u))];
+#pragma unroll
+  for (int o = kErrSlots / 2; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+  return m;
 }
 
 __device__ __forceinline__ bool converged(const uint32_t *stats) {
@@ -1060,8 +1064,8 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
         pos[s].w = lam;
     }
   }
-  // every thread gets here: the only early return above is uniform
-  if (MODE != 2 && err_slot >= 0) block_max_to(&stats[STAT_ERR0 + err_slot], err, active);
+  // every lane gets here: the only early return above is uniform
+  if (MODE != 2 && err_slot >= 0) raise_error(stats, err_slot, err, active);
 }
 
 // Trilinear sample with normalised coordinates, texel centres at (i+0.5)/dim
@@ -1201,11 +1205,13 @@ __global__ GATHER_BOUNDS(NB) void k_dp_update(
     uint32_t n, uint32_t nblocks, const float4 *__restrict__ pin, float4 *__restrict__ pout,
     const float *__restrict__ rho, const uint32_t *__restrict__ list,
     const uint4 *__restrict__ head, DevParams P, float scale, SdfDev o, uint32_t *stats,
-    int err_slot, float tol, float *__restrict__ lam_acc, float stiff, BatchDev B) {
+    int err_slot, int fallback_slot, float tol, float *__restrict__ lam_acc, float stiff,
+    BatchDev B) {
   bool done = false;
   if (tol > 0.0f) {
-    done = converged(stats) ||
-           __uint_as_float(stats[STAT_ERR0 + err_slot]) <= tol;
+    // a substep that fell back goes on from the error before its warm start
+    const int slot = stats[STAT_FALLBACK] ? fallback_slot : err_slot;
+    done = converged(stats) || __uint_as_float(max_error(stats, slot)) <= tol;
   }
   const uint32_t s = particle_index(nblocks);
   if (s >= n) return;
@@ -1326,7 +1332,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_lambda(
     f[10] = mk * my;
     f[11] = mk * mz;
   }
-  block_max_to(&stats[STAT_ERR0], err, active);  // every thread gets here
+  raise_error(stats, 0, err, active);  // every lane gets here
   float lam = lam0;
   if (LOG) {
     if (active) {
@@ -1369,8 +1375,9 @@ __global__ __launch_bounds__(kBlock) void k_warm_prev(uint32_t n, float4 *__rest
 // Plain fallback of a warm start, after the density pass of iteration 1: if
 // the predicted step left the maximum density error above the error before it,
 // the particles return to their positions before the step with the plain
-// first-iteration lambda and density, and iteration 1 proceeds from there
-// (its error slot then holds the pre-step error).
+// first-iteration lambda and density, and iteration 1 proceeds from there.  The
+// errors themselves stay as they are (blocks that start late decide by them too);
+// STAT_FALLBACK tells their readers that iteration 1 has the pre-step error.
 __global__ __launch_bounds__(kBlock) void k_warm_fallback(uint32_t n, uint32_t *stats,
                                                           const float4 *__restrict__ pre,
                                                           float4 *__restrict__ pos,
@@ -1378,8 +1385,8 @@ __global__ __launch_bounds__(kBlock) void k_warm_fallback(uint32_t n, uint32_t *
                                                           float *__restrict__ rho,
                                                           float *__restrict__ lam_acc) {
   if (stats[STAT_CONVERGED]) return;
-  const uint32_t e0 = stats[STAT_ERR0], e1 = stats[STAT_ERR0 + 1];
-  if (e1 <= e0) return;  // non-negative floats compare as their bit patterns
+  // non-negative floats compare as their bit patterns
+  if (max_error(stats, 1) <= max_error(stats, 0)) return;
   const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
   if (s < n) {
     const float4 p = pre[s];
@@ -1388,10 +1395,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_fallback(uint32_t n, uint32_t *
     rho[s] = q.y;
     lam_acc[s] = 0.0f;
   }
-  if (s == 0) {
-    stats[STAT_FALLBACK] = 1u;
-    stats[STAT_ERR0 + 1] = e0;
-  }
+  if (s == 0) stats[STAT_FALLBACK] = 1u;
 }
 
 // The same for a batch of scenes, scene by scene: a scene whose maximum error
@@ -1437,10 +1441,8 @@ __global__ __launch_bounds__(kBlock) void k_warm_fallback_stats(uint32_t nscenes
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    stats[STAT_ERR0 + 1] = sm[0];
-    stats[STAT_FALLBACK] = sr[0];
-  }
+  if (threadIdx.x < kErrSlots) stats[err_word(1u, threadIdx.x)] = threadIdx.x == 0 ? sm[0] : 0u;
+  if (threadIdx.x == 0) stats[STAT_FALLBACK] = sr[0];
 }
 
 // Keeps each particle's accumulated multiplier in particle-id order.
@@ -1708,10 +1710,20 @@ __global__ __launch_bounds__(kBlock) void k_commit(uint32_t n, const float4 *__r
   v_can[id] = make_float4(v.x, v.y, v.z, 0.0f);
 }
 
+// The statistics for the host: the flags and, a wave per iteration, its maximum.
+__global__ __launch_bounds__(kBlock) void k_collect_stats(const uint32_t *__restrict__ stats,
+                                                          uint32_t iterations,
+                                                          uint32_t *__restrict__ out) {
+  const uint32_t it = (blockIdx.x * kBlock + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
+  if (it == 0) out[lane] = stats[lane];
+  if (it >= iterations) return;
+  const uint32_t m = max_error(stats, (int)it);
+  if (lane == 0) out[STAT_ERR0 + it] = m;
+}
+
 // clear_substep_stats for a context without particles.
-__global__ void k_substep_init(uint32_t *stats) {
-  const int i = threadIdx.x;
-  if (i >= STAT_ITERS && i < STAT_WORDS) stats[i] = 0u;
+__global__ __launch_bounds__(kBlock) void k_substep_init(uint32_t *stats) {
+  clear_substep_stats(stats, kMaxIters);
 }
 
 // Standalone CalculateParticleCollisions on SoA float arrays.
@@ -1828,22 +1840,20 @@ __global__ __launch_bounds__(kBlock) void k_kinetic_energy(uint32_t n,
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-// Kernels that end in a block's maximum and its atomic, in place of none.
-static inline bool reduces_error(int kernel) {
-  return kernel == K_DENSITY_LAMBDA || kernel == K_DENSITY || kernel == K_LAMBDA ||
-         kernel == K_WARM_LAMBDA;
-}
-
 // Gathers in flight per wave of a gather kernel where neither the autotuner nor
-// the caller chose: 16, and 8 where the chip holds all waves at once anyway and
-// 8 let more of them in per SIMD (70 VGPRs).  Measured (us, events included), 16 /
-// 8: 133k particles delta p 11.1 / 10.7, XSPH 14.7 / 13.8, vorticity 15.8 / 14.9;
-// 439k 22.4 / 21.1, 33.8 / 33.3, 35.8 / 35.2; but surface at 681k 48.8 / 50.6, 1M
-// 70.1 / 76.8, and the density pass at every size (439k: 36 / 40).
+// the caller chose: 8 where the chip holds all or most waves at once anyway, which
+// lets more of them in per SIMD (70 VGPRs), 16 beyond.  Measured (us, 64 threads a
+// block, events included), 16 / 8: density 439k particles 25.6 / 23.0, 2.1M 87.4 /
+// 85.8, 3.4M 145.9 / 154.9; delta p 439k 22.4 / 21.1, 1M 42.6 / 41.3, 1.6M 58.5 /
+// 58.8; XSPH 133k 14.7 / 13.8, 439k 33.8 / 33.3, 1M 69.9 / 72.0; surface 681k 48.8
+// / 50.6, 1M 70.1 / 76.8.
 static inline int tuned_depth(const sph_ctx *c, int kernel) {
   const int d = c->tune.depth[kernel];
   if (d) return d;
-  return c->n <= (1 << 19) && !reduces_error(kernel) ? 8 : 16;
+  int most = 1 << 19;
+  if (kernel == K_DENSITY_LAMBDA || kernel == K_DENSITY || kernel == K_LAMBDA) most = 1 << 21;
+  if (kernel == K_DP || kernel == K_DP_UPDATE) most = 1 << 20;
+  return c->n <= most ? 8 : 16;
 }
 
 template <typename F>
@@ -1861,16 +1871,20 @@ static inline void with_depth(int depth, F &&f) {
 // and, of few particles, spreads the waves over the CUs (a wave's gathers keep a
 // vector L1 busy): surface 10.8 -> 8.8 us at 4k particles, 79.2 -> 70.1 at 1M
 // (256 / 64 threads, events included), XSPH 10.2 -> 7.9 and 75.3 -> 69.9, delta p
-// 8.5 -> 7.7 and 46.1 -> 42.5.  At 8.4M the neighbouring waves of a larger block
-// share more lines: colour 363 / 370, confinement 394 / 400, delta p 327 (128) /
-// 329, but surface 616 / 597.  The density passes pay an atomic per block on one
-// word and keep 256 (442k: 26.5 us against 30.0 at 128 and 36 at 64).
+// 8.5 -> 7.7 and 46.1 -> 42.5, density 9.3 -> 8.4 and 50.4 -> 46.9.  At 8.4M the
+// neighbouring waves of a larger block share more lines: colour 363 / 370,
+// confinement 394 / 400, delta p 327 (128) / 329, but surface 616 / 597 and density
+// 352 / 343.
 static inline uint32_t tuned_block(const sph_ctx *c, int kernel) {
   const uint32_t b = c->tune.block[kernel];
   if (b) return b;
-  if (kernel == K_BUILD_LISTS || reduces_error(kernel)) return (uint32_t)kBlock;
-  if (c->n <= (1 << 21) || kernel == K_SURFACE) return 64u;
-  return kernel == K_DP || kernel == K_DP_UPDATE ? 128u : (uint32_t)kBlock;
+  switch (kernel) {
+    case K_BUILD_LISTS: return kBlock;
+    case K_COLOR: case K_XSPH: case K_VORTICITY: case K_CONFINE:
+      return c->n <= (1 << 21) ? 64 : kBlock;
+    case K_DP: case K_DP_UPDATE: return c->n <= (1 << 21) ? 64 : 128;
+    default: return 64;  // density, surface, warm start
+  }
 }
 
 #define LAUNCH_TIMED(ctx, kid, grid, ...)                               \
@@ -1912,28 +1926,30 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
   const uint32_t n = c->n;
   hipStream_t s = c->stream;
   const BatchDev B = c->batch();
+  // the stage calls may run any number of density passes
+  const uint32_t last = (uint32_t)(fused ? c->P.solve_iterations : kMaxIters);
   if (n) {
     if (fused && c->nscenes) {
       LAUNCH_TIMED(c, K_PREDICT_HASH, 0,
                    k_predict_hash<true><<<blocks_for(n), kBlock, 0, s>>>(
                        n, c->x_can, c->v_can, c->xs_can, c->keys, c->cell_rank, c->cell_count,
-                       c->dev, c->stats, B));
+                       c->dev, c->stats, last, B));
     } else if (fused) {
       LAUNCH_TIMED(c, K_PREDICT_HASH, 0,
                    k_predict_hash<false><<<blocks_for(n), kBlock, 0, s>>>(
                        n, c->x_can, c->v_can, c->xs_can, c->keys, c->cell_rank, c->cell_count,
-                       c->dev, c->stats, B));
+                       c->dev, c->stats, last, B));
     } else if (c->nscenes) {
       LAUNCH_TIMED(c, K_HASH, 0,
                    k_hash<true><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, B));
+                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last, B));
     } else {
       LAUNCH_TIMED(c, K_HASH, 0,
                    k_hash<false><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, B));
+                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last, B));
     }
   } else {
-    k_substep_init<<<1, STAT_WORDS, 0, s>>>(c->stats);
+    k_substep_init<<<1, kBlock, 0, s>>>(c->stats);
   }
   SPH_HIP(hipGetLastError());
   // cell_start[c] = #keys < c (lower bound), cell_start[cells] = n
@@ -2100,6 +2116,7 @@ int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate) {
   float *acc = accumulate ? c->lam_acc : nullptr;
   const float scale = stiffness_scale(c, substep), stiff = stiffness_unitless(c, substep);
   const float tol = (float)c->P.density_tolerance;
+  const int fallback_slot = err_slot == 1 && !c->nscenes ? 0 : err_slot;
   const BatchDev B = c->batch();
   const bool obstacle = c->nscenes ? c->batch_sdf != nullptr : c->sdf.data != nullptr;
   const bool split = obstacle && c->tune.split_collide;
@@ -2109,7 +2126,7 @@ int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate) {
     LAUNCH_TIMED(c, K_DP_UPDATE, 0,                                                         \
                  (k_dp_update<COL, BAT, NBv><<<nb, bs, 0, c->stream>>>(                      \
                      n, nb, c->pos, out, c->rho, c->list, c->list_head, c->dev, scale, c->sdf, \
-                     c->stats, err_slot, tol, acc, stiff, B)));                             \
+                     c->stats, err_slot, fallback_slot, tol, acc, stiff, B)));              \
   })
   if (c->nscenes) {
     if (split) DP_UPDATE(false, true); else DP_UPDATE(true, true);
@@ -2345,6 +2362,15 @@ int launch_commit(sph_ctx *c) {
   LAUNCH_TIMED(c, K_COMMIT, 0,
                k_commit<<<blocks_for(n), kBlock, 0, c->stream>>>(n, c->pos, c->vel, c->id_s,
                                                                  c->x_can, c->v_can));
+  SPH_HIP(hipGetLastError());
+  return SPH_OK;
+}
+
+int launch_collect_stats(sph_ctx *c) {
+  static_assert(STAT_ERR0 == kWave, "a wave copies the flags");
+  constexpr uint32_t its = kMaxIters + 1;
+  k_collect_stats<<<blocks_for(its, kBlock / kWave), kBlock, 0, c->stream>>>(c->stats, its,
+                                                                            c->stats_read);
   SPH_HIP(hipGetLastError());
   return SPH_OK;
 }

@@ -357,3 +357,52 @@ def test_residuals_report_every_density_pass():
     st = ctx.stats()
     assert len(r) == st.iterations + 1 == 5   # capped: 4 updates + the final pass
     assert r[-1] == st.max_density_error
+
+
+def test_fallback_reverts_every_particle_of_a_large_scene():
+    """More blocks than the chip holds at once: those that start after the first
+    have ended revert their particles too.  After the revert one plain iteration
+    (stiffness index 1) is left, which the stages run from the same state."""
+    s = 0.02
+    sc = Scene(s, (3.0, 2.4, 2.4), iters=2, lambda_eps=600.0)
+    pos, vel = block_scene((106, 104, 104), s * 0.97, (0.3, 0.0, 0.2), jitter=0.01, seed=4,
+                           vel_sigma=0.2)
+    n = len(pos)
+    warm = sc.context(n)
+    warm.upload(pos, vel)
+    warm.set_warm_start(_face_net(40.0))
+    warm.step(1)
+    assert warm.stats().warm_fallback == 1
+    got, _ = warm.download()
+    plain = sc.context(n)
+    plain.upload(pos, vel)
+    plain.apply_gravity()
+    plain.predict_positions()
+    plain.find_all_neighbors()
+    plain.compute_densities()
+    plain.compute_lambda()
+    plain.update_dps(1)
+    plain.update_position_stars()
+    want = plain.field(sa.FIELD_POSITION_STAR)
+    # fused multiply-add in one path, product and sum in the other: an ulp or two
+    assert np.max(np.abs(got - want)) <= 4 * np.spacing(np.float32(3.0))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 64 * 64 + 1])
+def test_error_maximum_over_the_waves_words(n):
+    """The maximum is spread over 64 words by wavefront: one wave, a ragged one,
+    and more waves than words, with the largest density anywhere."""
+    s = 0.02
+    sc = Scene(s, (2.0, 1.0, 1.0), iters=1, lambda_eps=600.0)
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0.2, 0.2 + 0.8 * s * n ** (1.0 / 3.0), (n, 3)).astype(np.float32)
+    with sc.context(n) as ctx:
+        for _ in range(2):  # the second finds the words cleared
+            ctx.upload(pos)
+            ctx.predict_positions()
+            ctx.find_all_neighbors()
+            ctx.compute_densities()
+            rho = ctx.field(sa.FIELD_DENSITY)
+            want = max(float(np.max(rho) - np.float32(1000.0)) / 1000.0, 0.0)
+            assert abs(ctx.stats().max_density_error - want) <= 1e-6 * max(want, 1.0)
+            pos = (pos[::-1] + np.float32(0.001)).astype(np.float32)
