@@ -332,8 +332,10 @@ int sph_profile_kernel_count(void);
  * and 8/16/32 neighbour gathers in flight per wavefront for every
  * neighbour-gather kernel, with an obstacle the push fused into the
  * position update or as a separate pass, and compact (16-bit offsets) versus
- * wide (32-bit indices) neighbour lists.  Keeps the fastest choice per
- * kernel.  Results do not depend on the choice. */
+ * wide (32-bit indices) neighbour lists; in a small scene also four lanes a
+ * particle, which no field of sph_tuning names (the context keeps that until
+ * the next sph_set_tuning).  Keeps the fastest choice per kernel.  Results do not
+ * depend on the choice. */
 #define SPH_TUNE_KERNELS 32
 typedef struct sph_tuning {
   int split_collide;              /* obstacle push as a separate pass */

@@ -1446,6 +1446,7 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
     graph_reset(c);
     rc = trial(cur, &before);  // as the context was
   }
+  for (int k : kTunable) c->tune.quad[k] = false;
   for (int b = 0; b < 3 && e == hipSuccess && !rc; ++b) {
     for (int k : kTunable) c->tune.block[k] = sizes[b];
     graph_reset(c);
@@ -1474,6 +1475,13 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
       }
   }
   for (int k : kTunable) c->tune.depth[k] = best_depth[k] ? best_depth[k] : (uint8_t)16;
+  // four lanes a particle, where the scene is small enough for them
+  if (e == hipSuccess && !rc && c->n <= (uint32_t)sph::kQuadMax) {
+    for (int k : kTunable) c->tune.quad[k] = true;
+    graph_reset(c);
+    rc = trial(cur, &total);
+    for (int k : kTunable) c->tune.quad[k] = cur[k] > 0.0 && cur[k] < best[k];
+  }
   bool split_best = c->tune.split_collide;
   double after = 0.0;
   if (!rc && e == hipSuccess) {
@@ -1542,6 +1550,7 @@ extern "C" int sph_set_tuning(sph_ctx *c, const sph_tuning *t) {
       return arg_error("gathers in flight must be 0, 8, 16 or 32");
     tune.block[k] = (uint16_t)b;
     tune.depth[k] = (uint8_t)d;
+    tune.quad[k] = false;
   }
   tune.split_collide = t->split_collide != 0;
   tune.wide_lists = t->wide_lists != 0;

@@ -21,6 +21,18 @@ constexpr uint32_t kMaxParticles = SPH_MAX_PARTICLES;
 static_assert((kMaxParticles + 64ull) * 16ull <= (1ull << 32), "32-bit byte offsets");
 // Chunks of a state transfer, at most.
 constexpr int kIoChunks = 16;
+// Most particles of the gather kernels with four lanes a particle (sum_neighbors),
+// if nobody chose a launch or the autotuner measured them fastest.  A wave of 64
+// particles leaves most SIMDs without one up to here, and each lane's gathers come
+// in four or more rounds one after the other; four lanes need one or two.  Measured
+// (us, events included: about 3.5 of each; one lane a particle / four): density 8.9
+// / 6.9 at 4k particles, 8.8 / 7.6 at 16k, 9.3 / 8.7 at 33k, 9.6 / 10.0 at 47k;
+// delta p 8.2 / 6.5, 8.1 / 6.7, 8.5 / 7.4, 8.8 / 8.4; colour 7.8 / 6.3, 7.9 / 6.6,
+// 8.3 / 7.6, 8.4 / 8.6; surface 8.9 / 6.5, 9.2 / 7.8, 9.8 / 8.9, 10.4 / 10.9; XSPH
+// 7.7 / 6.2, 8.0 / 6.9, 8.5 / 8.7, 9.2 / 10.3; vorticity 8.2 / 6.5, 8.3 / 7.5, 9.2 /
+// 9.3, 10.0 / 11.4; confinement 7.9 / 6.3, 7.9 / 6.8, 8.6 / 7.8, 8.7 / 9.0.  Two
+// lanes a particle were slower than either from 1k to 133k.
+constexpr int kQuadMax = 1 << 15;
 // Particles per block of the per-scene error reduction of a batch.
 constexpr uint32_t kSceneChunk = 4096;
 // Neighbour-list head per particle: the first candidate index of each of the
@@ -251,6 +263,8 @@ struct sph_ctx {
     uint16_t block[sph::K_COUNT] = {};  // threads per block of gather kernels (0: by rule)
     uint8_t depth[sph::K_COUNT] = {};   // gathers in flight per wave: 8, 16, 32 (0: by rule)
     bool wide_lists = false;  // 32-bit list entries for every wave
+    // four lanes a particle measured fastest (the autotuner; not part of sph_tuning)
+    bool quad[sph::K_COUNT] = {};
   } tune;
   // whole-substep HIP graph (sph_set_graph)
   bool graph_on = false;

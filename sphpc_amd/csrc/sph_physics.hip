@@ -38,6 +38,20 @@ __device__ __forceinline__ uint32_t particle_index(uint32_t n_blocks) {
   return xcd_block(blockIdx.x, n_blocks) * blockDim.x + threadIdx.x;
 }
 
+// Depth of the gather kernels that give a particle four lanes (sum_neighbors).
+constexpr int kQuad = 4;
+
+// The particle of a gather kernel's lane, and whether the lane stores its results.
+template <int NB>
+__device__ __forceinline__ uint32_t gather_index(uint32_t n_blocks) {
+  return NB == kQuad ? particle_index(n_blocks) >> 2 : particle_index(n_blocks);
+}
+
+template <int NB>
+__device__ __forceinline__ bool gather_lead() {
+  return NB != kQuad || (threadIdx.x & 3u) == 0u;
+}
+
 __device__ __forceinline__ const uint32_t *list_ptr(const uint32_t *list, uint32_t s) {
   return list + (size_t)(s >> 6) * kListStride + (s & 63u) * 4u;
 }
@@ -229,6 +243,104 @@ __device__ __forceinline__ void for_neighbors(const uint32_t *list, const uint4 
 struct Pair4 {
   float4 a, b;
 };
+
+// What a neighbour adds to a particle's NA sums: acc[a] = fma(w, d, acc[a]) for the
+// P pairs (w, d) of each, in order.
+template <int NA, int P = 1>
+struct Terms {
+  float w[NA * P], d[NA * P];
+};
+
+// Value of lane K of each four lanes, in all of them.
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+
+// Sum over each four lanes, in all of them.
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // 1 0 3 2
+  return v + (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);  // 2 3 0 1
+}
+
+// The sums over a particle's neighbours with four lanes for each particle: lane q
+// of the four gathers and evaluates entries 8 q .. 8 q + 7 of each 32, and the sums
+// pass from lane to lane, so that they are the ones a single lane makes in list
+// order, bit for bit.  An entry past the list adds 0 * 0.
+template <typename T, int NA, int P, bool WIDE, typename Load, typename Term>
+__device__ __forceinline__ void quad_loop(const NbList &nl, const uint4 &first, uint32_t self,
+                                          Load &load, Term &term, float (&acc)[NA]) {
+  constexpr int E = 8;  // entries per lane and round
+  const int sub = threadIdx.x & 3;
+  Quads<E, WIDE> r;
+  if (WIDE)
+    r.load(nl, E * sub);
+  else
+    r.q[0] = first;
+  for (int base = 0; base < nl.c; base += 4 * E) {
+    const int k0 = base + E * sub;
+    uint32_t j[E];
+    decode<E>(nl, r, k0, self, j);
+    __builtin_amdgcn_sched_barrier(0);
+    T q[E];
+    if (k0 < nl.c) {
+#pragma unroll
+      for (int b = 0; b < E; ++b) q[b] = load(j[b]);
+    }
+    r.load(nl, k0 + 4 * E);
+    Terms<NA, P> t[E];
+#pragma unroll
+    for (int b = 0; b < E; ++b) {
+      t[b] = {};
+      if (k0 + b < nl.c) t[b] = term(q[b]);
+    }
+    const auto pass = [&](auto lane) {
+#pragma unroll
+      for (int b = 0; b < E; ++b)
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+          for (int i = 0; i < P; ++i)
+            acc[a] = fmaf(t[b].w[a * P + i], t[b].d[a * P + i], acc[a]);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = quad_lane<decltype(lane)::value>(acc[a]);
+      // whether the next lane has an entry in any particle of the wave
+      return __ballot(base + E * (decltype(lane)::value + 1) < nl.c) != 0ull;
+    };
+    if (pass(std::integral_constant<int, 0>{}) && pass(std::integral_constant<int, 1>{}) &&
+        pass(std::integral_constant<int, 2>{}))
+      pass(std::integral_constant<int, 3>{});
+  }
+}
+
+// acc = the sums of term(load(j)) over the neighbours j of particle s, in list
+// order, with NB gathers in flight or (kQuad) four lanes a particle.
+template <typename T, int NB, bool PREFETCH, int NA, int P, typename Load, typename Term>
+__device__ __forceinline__ void sum_neighbors(const uint32_t *list, const uint4 *head, uint32_t s,
+                                              int *count, float (&acc)[NA], Load load,
+                                              Term term) {
+#pragma unroll
+  for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+  if constexpr (NB == kQuad) {
+    const uint4 first =
+        reinterpret_cast<const uint4 *>(list_ptr(list, s))[(size_t)(threadIdx.x & 3u) * kWave];
+    const NbList nl = nb_list(list, head, s);
+    *count = nl.c;
+    if (nl.wide)
+      quad_loop<T, NA, P, true>(nl, first, s, load, term, acc);
+    else
+      quad_loop<T, NA, P, false>(nl, first, s, load, term, acc);
+  } else {
+    for_neighbors<T, NB, PREFETCH>(list, head, s, count, load, [&](const T &q) {
+      const Terms<NA, P> t = term(q);
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int i = 0; i < P; ++i) acc[a] = fmaf(t.w[a * P + i], t.d[a * P + i], acc[a]);
+    });
+  }
+}
 
 // Gathers of 16-byte records through a buffer resource with a 16-byte stride
 // (`buffer_load ... idxen`): the texture addresser forms base + 16 j from the
@@ -1015,53 +1127,62 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
     uint32_t *stats, int err_slot, int check_converged, int density_to_w,
     float4 *__restrict__ with_lambda) {
   if (check_converged && converged(stats)) return;
-  const uint32_t s = particle_index(nblocks);
-  const bool active = s < n;
+  const uint32_t s = gather_index<NB>(nblocks);
+  const bool active = s < n, lead = gather_lead<NB>();
   float err = 0.0f;
   if (active) {
     const float4 p = pos[s];
     int cnt;
     uint32_t S = 0u;
-    float sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, sc = 0.0f;
     const Records16 G(pos, n);
-    for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; },
-                              [&](const float4 &q) {
+    const auto load = [&](uint32_t j) { return G[j]; };
+    // sum of g d (three), and of g^2 r^2
+    float sg[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const auto term = [&](const float4 &q) {
       const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       const float r2 = sq3(dx, dy, dz);
       if (MODE != 2) S += density_term(r2, P);
-      if (MODE != 1) {
-        const float r2c = fmaxf(r2, P.rmin2);
-        const float ir = fast_rsq(r2c);
-        const float hr = fmaf(-r2c, ir, P.h);  // h - r, r floored at 1e-4 h
-        const float hp = fmaxf(hr, 0.0f);  // a listed pair can be past h after an update
-        const float g = hp * hp * ir;  // DelW(r)/r / norm
-        sgx = fmaf(g, dx, sgx);
-        sgy = fmaf(g, dy, sgy);
-        sgz = fmaf(g, dz, sgz);
-        sc = fmaf(g * g, r2, sc);
-      }
-    });
+      const float r2c = fmaxf(r2, P.rmin2);
+      const float ir = fast_rsq(r2c);
+      const float hr = fmaf(-r2c, ir, P.h);  // h - r, r floored at 1e-4 h
+      const float hp = fmaxf(hr, 0.0f);  // a listed pair can be past h after an update
+      const float g = hp * hp * ir;  // DelW(r)/r / norm
+      return Terms<4>{{g, g, g, g * g}, {dx, dy, dz, r2}};
+    };
+    if constexpr (MODE == 1) {
+      float none[1];
+      sum_neighbors<float4, NB, true, 1, 1>(list, head, s, &cnt, none, load,
+                                            [&](const float4 &q) {
+        S += density_term(sq3(p.x - q.x, p.y - q.y, p.z - q.z), P);
+        return Terms<1>{{0.0f}, {0.0f}};
+      });
+    } else {
+      sum_neighbors<float4, NB, true, 4, 1>(list, head, s, &cnt, sg, load, term);
+    }
+    if constexpr (NB == kQuad) S = quad_sum(S);
     float C;
     if (MODE != 2) {
       C = density_constraint(S, cnt, P);
       const float rho = fmaf(C, P.rest_density, P.rest_density);
-      rho_out[s] = rho;
-      if (c_io) c_io[s] = C;
+      if (lead) rho_out[s] = rho;
+      if (c_io && lead) c_io[s] = C;
       // the reported error is that of the stored density, as every later
       // reader of rho (per-scene errors, the warm fallback) computes it
       err = fmaxf((rho - P.rest_density) * P.inv_rest_density, 0.0f);
-      if (density_to_w) pos[s].w = rho;
+      if (density_to_w && lead) pos[s].w = rho;
     } else {
       C = c_io[s];
     }
     if (MODE != 1) {
       const float Ci = fmaxf(C, 0.0f);
-      const float sum_c = P.lam_k2 * (sc + sq3(sgx, sgy, sgz));
+      const float sum_c = P.lam_k2 * (sg[3] + sq3(sg[0], sg[1], sg[2]));
       const float lam = -Ci / (sum_c + P.lambda_eps);
-      if (with_lambda)
+      if (!lead) {
+      } else if (with_lambda) {
         with_lambda[s] = make_float4(p.x, p.y, p.z, lam);
-      else
+      } else {
         pos[s].w = lam;
+      }
     }
   }
   // every lane gets here: the only early return above is uniform
@@ -1135,21 +1256,20 @@ __device__ __forceinline__ float3 dp_sum(const float4 &p, const float4 *pos, uin
                                          const uint32_t *list, const uint4 *head, uint32_t s,
                                          const DevParams &P) {
   int cnt;
-  float ax = 0.0f, ay = 0.0f, az = 0.0f;
+  float a[3];
   const Records16 G(pos, n);
-  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
-    const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
-    const float ir = fast_rsq(r2c);
-    const float hr = fmaf(-r2c, ir, P.h);
-    const float hp = fmaxf(hr, 0.0f);
-    const float g = hp * hp * ir;
-    const float f = (p.w + q.w) * g;
-    ax = fmaf(f, dx, ax);
-    ay = fmaf(f, dy, ay);
-    az = fmaf(f, dz, az);
-  });
-  return make_float3(ax, ay, az);
+  sum_neighbors<float4, NB, true, 3, 1>(
+      list, head, s, &cnt, a, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
+        const float ir = fast_rsq(r2c);
+        const float hr = fmaf(-r2c, ir, P.h);
+        const float hp = fmaxf(hr, 0.0f);
+        const float g = hp * hp * ir;
+        const float f = (p.w + q.w) * g;
+        return Terms<3>{{f, f, f}, {dx, dy, dz}};
+      });
+  return make_float3(a[0], a[1], a[2]);
 }
 
 // Staged UpdateDPs: dp = stiffness * m * DelW_norm / rho0 * sum.
@@ -1164,17 +1284,18 @@ __global__ GATHER_BOUNDS(NB) void k_dp(uint32_t n, uint32_t nblocks,
                                                float4 *__restrict__ xnext,
                                                const float *__restrict__ rho, SdfDev o,
                                                BatchDev B) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
   const float4 p = pos[s];
   const float3 a = dp_sum<NB>(p, pos, n, list, head, s, P);
   const float4 d = make_float4(scale * a.x, scale * a.y, scale * a.z, 0.0f);
-  dp[s] = d;
+  const bool lead = gather_lead<NB>();
+  if (lead) dp[s] = d;
   if (xnext) {
     float x = p.x + d.x, y = p.y + d.y, z = p.z + d.z;
     apply_boundary(x, y, z, geo_of<BATCH>(s, P, B), P);
     collide(x, y, z, sdf_of<BATCH>(s, o, B));
-    xnext[s] = make_float4(x, y, z, rho[s]);
+    if (lead) xnext[s] = make_float4(x, y, z, rho[s]);
   }
 }
 
@@ -1213,19 +1334,21 @@ __global__ GATHER_BOUNDS(NB) void k_dp_update(
     const int slot = stats[STAT_FALLBACK] ? fallback_slot : err_slot;
     done = converged(stats) || __uint_as_float(max_error(stats, slot)) <= tol;
   }
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
+  const bool lead = gather_lead<NB>();
   const float4 p = pin[s];
   if (done) {
     if (s == 0) stats[STAT_CONVERGED] = 1u;
-    pout[s] = make_float4(p.x, p.y, p.z, rho[s]);
+    if (lead) pout[s] = make_float4(p.x, p.y, p.z, rho[s]);
     return;
   }
-  if (s == 0) stats[STAT_ITERS] += 1u;
+  if (s == 0 && lead) stats[STAT_ITERS] += 1u;
   const float3 a = dp_sum<NB>(p, pin, n, list, head, s, P);
   float x = fmaf(scale, a.x, p.x), y = fmaf(scale, a.y, p.y), z = fmaf(scale, a.z, p.z);
   apply_boundary(x, y, z, geo_of<BATCH>(s, P, B), P);
   if (COLLIDE) collide(x, y, z, sdf_of<BATCH>(s, o, B));
+  if (!lead) return;
   pout[s] = make_float4(x, y, z, rho[s]);
   if (lam_acc) lam_acc[s] = fmaf(stiff, p.w, lam_acc[s]);
 }
@@ -1507,24 +1630,25 @@ __global__ GATHER_BOUNDS(NB) void k_color(uint32_t n, uint32_t nblocks,
                                                   const uint4 *__restrict__ head, DevParams P,
                                                   float4 *__restrict__ vel,
                                                   float4 *__restrict__ color) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
+  const bool lead = gather_lead<NB>();
   const float4 p = pos[s];
-  if (WITH_VELOCITY) vel[s] = velocity_of(p, xold[s], P);
+  if (WITH_VELOCITY && lead) vel[s] = velocity_of(p, xold[s], P);
   int cnt;
-  float ax = 0.0f, ay = 0.0f, az = 0.0f;
+  float a[3];
   const Records16 G(pos, n);
-  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
-    const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
-    const float u = P.h2 - r2c;
-    const float up = fmaxf(u, 0.0f);
-    const float g = up * up * fast_rcp(q.w);
-    ax = fmaf(g, dx, ax);
-    ay = fmaf(g, dy, ay);
-    az = fmaf(g, dz, az);
-  });
-  color[s] = make_float4(P.color_k * ax, P.color_k * ay, P.color_k * az, 0.0f);
+  sum_neighbors<float4, NB, true, 3, 1>(
+      list, head, s, &cnt, a, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
+        const float u = P.h2 - r2c;
+        const float up = fmaxf(u, 0.0f);
+        const float g = up * up * fast_rcp(q.w);
+        return Terms<3>{{g, g, g}, {dx, dy, dz}};
+      });
+  if (lead)
+    color[s] = make_float4(P.color_k * a[0], P.color_k * a[1], P.color_k * a[2], 0.0f);
 }
 
 // ComputeSurfaceTension force pass (particles.c:142-204): cohesion (Akinci
@@ -1539,16 +1663,16 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t
                                                     const uint32_t *__restrict__ list,
                                                     const uint4 *__restrict__ head, DevParams P,
                                                     float4 *__restrict__ vel) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 ci = color[s];
   int cnt;
   const float hh = 0.5f * P.h;
-  float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+  float f[3];
   const Records16 Gp(pos, n), Gc(color, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gc[j]}; };
-  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qc) {
+  sum_neighbors<Pair4, NB, false, 3, 1>(list, head, s, &cnt, f, load, [&](const Pair4 &qc) {
     const float4 &q = qc.a, &cq = qc.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1561,15 +1685,17 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t
     const float spline = r <= hh ? fmaf(2.0f, t3, -P.h6_64) : t3;
     const float coh = P.coh_k * spline * ir;
     const float K = 2.0f * P.rest_density * fast_rcp(p.w + q.w);
-    fx = fmaf(K, fmaf(coh, dx, P.curv_k * (ci.x - cq.x)), fx);
-    fy = fmaf(K, fmaf(coh, dy, P.curv_k * (ci.y - cq.y)), fy);
-    fz = fmaf(K, fmaf(coh, dz, P.curv_k * (ci.z - cq.z)), fz);
+    return Terms<3>{{K, K, K},
+                    {fmaf(coh, dx, P.curv_k * (ci.x - cq.x)),
+                     fmaf(coh, dy, P.curv_k * (ci.y - cq.y)),
+                     fmaf(coh, dz, P.curv_k * (ci.z - cq.z))}};
   });
+  if (!gather_lead<NB>()) return;
   const float k = P.dt / p.w;
   float4 v = vel[s];
-  v.x = fmaf(k, fx, v.x);
-  v.y = fmaf(k, fy, v.y);
-  v.z = fmaf(k, fz, v.z);
+  v.x = fmaf(k, f[0], v.x);
+  v.y = fmaf(k, f[1], v.y);
+  v.z = fmaf(k, f[2], v.z);
   vel[s] = v;
 }
 
@@ -1582,26 +1708,25 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_xsph(uint32_t n,
                                                  const uint32_t *__restrict__ list,
                                                  const uint4 *__restrict__ head, DevParams P,
                                                  float4 *__restrict__ vout) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 vi = vin[s];
   int cnt;
-  float ax = 0.0f, ay = 0.0f, az = 0.0f;
+  float a[3];
   const Records16 Gp(pos, n), Gv(vin, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qv) {
+  sum_neighbors<Pair4, NB, false, 3, 1>(list, head, s, &cnt, a, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float u = P.h2 - fmaf(dy * dy * dz, dz, dx * dx);
     const float up = fmaxf(u, 0.0f);
     const float w = up * up * up * fast_rcp(q.w);
-    ax = fmaf(vq.x - vi.x, w, ax);
-    ay = fmaf(vq.y - vi.y, w, ay);
-    az = fmaf(vq.z - vi.z, w, az);
+    return Terms<3>{{vq.x - vi.x, vq.y - vi.y, vq.z - vi.z}, {w, w, w}};
   });
   const float k = P.xsph_c * P.mWn;
-  vout[s] = make_float4(fmaf(k, ax, vi.x), fmaf(k, ay, vi.y), fmaf(k, az, vi.z), 0.0f);
+  if (gather_lead<NB>())
+    vout[s] = make_float4(fmaf(k, a[0], vi.x), fmaf(k, a[1], vi.y), fmaf(k, a[2], vi.z), 0.0f);
 }
 
 // ComputeVorticity (particles.c:207-283); aux = (omega, |omega|), and
@@ -1614,15 +1739,15 @@ __global__ __launch_bounds__(kBlock) void k_vorticity(uint32_t n, uint32_t nbloc
                                                       const uint4 *__restrict__ head, DevParams P,
                                                       float4 *__restrict__ omega,
                                                       float4 *__restrict__ pw) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
   const float4 p = pos[s];
   const float4 vi = vel[s];
   int cnt;
-  float ox = 0.0f, oy = 0.0f, oz = 0.0f;
+  float o[3];
   const Records16 Gp(pos, n), Gv(vel, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qv) {
+  sum_neighbors<Pair4, NB, false, 3, 2>(list, head, s, &cnt, o, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1633,14 +1758,11 @@ __global__ __launch_bounds__(kBlock) void k_vorticity(uint32_t n, uint32_t nbloc
     if (P.vort_model == 1) g *= fast_rcp(q.w);
     const float wx = g * dx, wy = g * dy, wz = g * dz;
     const float vx = vq.x - vi.x, vy = vq.y - vi.y, vz = vq.z - vi.z;
-    ox = fmaf(vy, wz, fmaf(-vz, wy, ox));
-    oy = fmaf(vz, wx, fmaf(-vx, wz, oy));
-    oz = fmaf(vx, wy, fmaf(-vy, wx, oz));
+    return Terms<3, 2>{{-vz, vy, -vx, vz, -vy, vx}, {wy, wz, wz, wx, wx, wy}};
   });
+  if (!gather_lead<NB>()) return;
   const float k = P.vort_model == 1 ? P.DelW_norm * P.mass : P.DelW_norm;
-  ox *= k;
-  oy *= k;
-  oz *= k;
+  const float ox = o[0] * k, oy = o[1] * k, oz = o[2] * k;
   const float wn = sqrtf(sq3(ox, oy, oz));
   omega[s] = make_float4(ox, oy, oz, wn);
   pw[s] = make_float4(p.x, p.y, p.z, wn);
@@ -1657,27 +1779,25 @@ __global__ GATHER_BOUNDS(NB) void k_confine(
     const uint4 *__restrict__ head, DevParams P, const float4 *__restrict__ vin,
     float4 *__restrict__ vout, const uint32_t *__restrict__ id_s, float4 *__restrict__ x_can,
     float4 *__restrict__ v_can) {
-  const uint32_t s = particle_index(nblocks);
+  const uint32_t s = gather_index<NB>(nblocks);
   if (s >= n) return;
   const float4 p = pw[s];
   int cnt;
-  float ex = 0.0f, ey = 0.0f, ez = 0.0f;
+  float e[3];
   // only x_j and |omega_j| of the neighbour are needed
   const Records16 G(pw, n);
-  for_neighbors<float4, NB>(list, head, s, &cnt, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
-    const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
-    const float ir = fast_rsq(r2c);
-    const float hr = fmaf(-r2c, ir, P.h);
-    const float hp = fmaxf(hr, 0.0f);
-    const float g = q.w * hp * hp * ir;
-    ex = fmaf(g, dx, ex);
-    ey = fmaf(g, dy, ey);
-    ez = fmaf(g, dz, ez);
-  });
-  ex *= P.DelW_norm;
-  ey *= P.DelW_norm;
-  ez *= P.DelW_norm;
+  sum_neighbors<float4, NB, true, 3, 1>(
+      list, head, s, &cnt, e, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
+        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
+        const float ir = fast_rsq(r2c);
+        const float hr = fmaf(-r2c, ir, P.h);
+        const float hp = fmaxf(hr, 0.0f);
+        const float g = q.w * hp * hp * ir;
+        return Terms<3>{{g, g, g}, {dx, dy, dz}};
+      });
+  if (!gather_lead<NB>()) return;
+  const float ex = e[0] * P.DelW_norm, ey = e[1] * P.DelW_norm, ez = e[2] * P.DelW_norm;
   const float em = fmaxf(sqrtf(sq3(ex, ey, ez)), P.rmin);
   const float Nx = ex / em, Ny = ey / em, Nz = ez / em;
   const float4 wi = omega[s];
@@ -1841,14 +1961,15 @@ __global__ __launch_bounds__(kBlock) void k_kinetic_energy(uint32_t n,
 // Launchers
 // ---------------------------------------------------------------------------
 // Gathers in flight per wave of a gather kernel where neither the autotuner nor
-// the caller chose: 8 where the chip holds all or most waves at once anyway, which
-// lets more of them in per SIMD (70 VGPRs), 16 beyond.  Measured (us, 64 threads a
-// block, events included), 16 / 8: density 439k particles 25.6 / 23.0, 2.1M 87.4 /
-// 85.8, 3.4M 145.9 / 154.9; delta p 439k 22.4 / 21.1, 1M 42.6 / 41.3, 1.6M 58.5 /
-// 58.8; XSPH 133k 14.7 / 13.8, 439k 33.8 / 33.3, 1M 69.9 / 72.0; surface 681k 48.8
-// / 50.6, 1M 70.1 / 76.8.
+// the caller chose: four lanes a particle up to kQuadMax; 8 where the chip holds all
+// or most waves at once anyway, which lets more of them in per SIMD (70 VGPRs); 16
+// beyond.  Measured (us, 64 threads a block, events included), 16 / 8: density 439k
+// particles 25.6 / 23.0, 2.1M 87.4 / 85.8, 3.4M 145.9 / 154.9; delta p 439k 22.4 /
+// 21.1, 1M 42.6 / 41.3, 1.6M 58.5 / 58.8; XSPH 133k 14.7 / 13.8, 439k 33.8 / 33.3,
+// 1M 69.9 / 72.0; surface 681k 48.8 / 50.6, 1M 70.1 / 76.8.
 static inline int tuned_depth(const sph_ctx *c, int kernel) {
   const int d = c->tune.depth[kernel];
+  if (c->n <= kQuadMax && (c->tune.quad[kernel] || (!d && !c->tune.block[kernel]))) return kQuad;
   if (d) return d;
   int most = 1 << 19;
   if (kernel == K_DENSITY_LAMBDA || kernel == K_DENSITY || kernel == K_LAMBDA) most = 1 << 21;
@@ -1862,6 +1983,8 @@ static inline void with_depth(int depth, F &&f) {
     f(std::integral_constant<int, 32>{});
   else if (depth == 8)
     f(std::integral_constant<int, 8>{});
+  else if (depth == kQuad)
+    f(std::integral_constant<int, kQuad>{});
   else
     f(std::integral_constant<int, 16>{});
 }
@@ -1885,6 +2008,19 @@ static inline uint32_t tuned_block(const sph_ctx *c, int kernel) {
     case K_DP: case K_DP_UPDATE: return c->n <= (1 << 21) ? 64 : 128;
     default: return 64;  // density, surface, warm start
   }
+}
+
+// Depth, threads per block and blocks of a gather kernel's launch; the threads as
+// chosen for block_of.
+struct Gather {
+  int depth;
+  uint32_t threads, blocks;
+};
+static inline Gather gather_launch(const sph_ctx *c, int kernel, int block_of) {
+  const int depth = tuned_depth(c, kernel);
+  if (depth == kQuad) return {depth, kWave, blocks_for(c->n, kWave / 4)};
+  const uint32_t t = tuned_block(c, block_of);
+  return {depth, t, blocks_for(c->n, t)};
 }
 
 #define LAUNCH_TIMED(ctx, kid, grid, ...)                               \
@@ -2016,11 +2152,12 @@ static float stiffness_scale(const sph_ctx *c, int substep) {
 int launch_density(sph_ctx *c, int mode, int err_slot) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_DENSITY_LAMBDA);
-  const uint32_t nb = blocks_for(n, bs);
+  const int kernel = mode == 0 || mode == 4 ? K_DENSITY_LAMBDA : mode == 2 ? K_LAMBDA : K_DENSITY;
+  const Gather g = gather_launch(c, kernel, K_DENSITY_LAMBDA);
+  const uint32_t bs = g.threads, nb = g.blocks;
   hipStream_t s = c->stream;
   if (mode == 0)
-    with_depth(tuned_depth(c, K_DENSITY_LAMBDA), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_DENSITY_LAMBDA, 0,
                    k_density_lambda<0, NBv><<<nb, bs, 0, s>>>(
@@ -2028,7 +2165,7 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        err_slot, c->P.density_tolerance > 0, 0, nullptr));
     });
   else if (mode == 1)
-    with_depth(tuned_depth(c, K_DENSITY), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_DENSITY, 0,
                    k_density_lambda<1, NBv><<<nb, bs, 0, s>>>(
@@ -2036,7 +2173,7 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        err_slot, 0, 0, nullptr));
     });
   else if (mode == 4)  // density and lambda in one gather: rho into w, (x*, lambda) aside
-    with_depth(tuned_depth(c, K_DENSITY_LAMBDA), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_DENSITY_LAMBDA, 0,
                    k_density_lambda<0, NBv><<<nb, bs, 0, s>>>(
@@ -2044,7 +2181,7 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        err_slot, 0, 1, c->pos == c->pos_a ? c->pos_b : c->pos_a));
     });
   else if (mode == 3)  // final density of a capped tolerance loop: rho also into w
-    with_depth(tuned_depth(c, K_DENSITY), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_DENSITY, 0,
                    k_density_lambda<1, NBv><<<nb, bs, 0, s>>>(
@@ -2052,7 +2189,7 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                        err_slot, 1, 1, nullptr));
     });
   else
-    with_depth(tuned_depth(c, K_LAMBDA), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_LAMBDA, 0,
                    k_density_lambda<2, NBv><<<nb, bs, 0, s>>>(
@@ -2066,11 +2203,11 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
 int launch_dp(sph_ctx *c, int substep, float4 *xnext) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_DP);
-  const uint32_t nb = blocks_for(n, bs);
+  const Gather g = gather_launch(c, K_DP, K_DP);
+  const uint32_t bs = g.threads, nb = g.blocks;
   const float scale = stiffness_scale(c, substep);
   const BatchDev B = c->batch();
-  with_depth(tuned_depth(c, K_DP), [&](auto D_) {
+  with_depth(g.depth, [&](auto D_) {
     constexpr int NBv = decltype(D_)::value;
     if (c->nscenes)
       LAUNCH_TIMED(c, K_DP, 0,
@@ -2110,8 +2247,8 @@ static float stiffness_unitless(const sph_ctx *c, int substep) {
 int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_DP_UPDATE);
-  const uint32_t nb = blocks_for(n, bs);
+  const Gather g = gather_launch(c, K_DP_UPDATE, K_DP_UPDATE);
+  const uint32_t bs = g.threads, nb = g.blocks;
   float4 *out = (c->pos == c->pos_a) ? c->pos_b : c->pos_a;
   float *acc = accumulate ? c->lam_acc : nullptr;
   const float scale = stiffness_scale(c, substep), stiff = stiffness_unitless(c, substep);
@@ -2121,7 +2258,7 @@ int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate) {
   const bool obstacle = c->nscenes ? c->batch_sdf != nullptr : c->sdf.data != nullptr;
   const bool split = obstacle && c->tune.split_collide;
 #define DP_UPDATE(COL, BAT)                                                                 \
-  with_depth(tuned_depth(c, K_DP_UPDATE), [&](auto D_) {                                    \
+  with_depth(g.depth, [&](auto D_) {                                    \
     constexpr int NBv = decltype(D_)::value;                                                \
     LAUNCH_TIMED(c, K_DP_UPDATE, 0,                                                         \
                  (k_dp_update<COL, BAT, NBv><<<nb, bs, 0, c->stream>>>(                      \
@@ -2257,10 +2394,10 @@ int launch_color(sph_ctx *c, bool with_velocity) {
   const uint32_t n = c->n;
   if (with_velocity) c->vel = c->vel_a;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_COLOR);
-  const uint32_t nb = blocks_for(n, bs);
+  const Gather g = gather_launch(c, K_COLOR, K_COLOR);
+  const uint32_t bs = g.threads, nb = g.blocks;
   if (with_velocity)
-    with_depth(tuned_depth(c, K_COLOR), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_COLOR, 0,
                    k_color<true, NBv><<<nb, bs, 0, c->stream>>>(n, nb, c->pos, c->xold, c->list,
@@ -2268,7 +2405,7 @@ int launch_color(sph_ctx *c, bool with_velocity) {
                                                                c->aux));
     });
   else
-    with_depth(tuned_depth(c, K_COLOR), [&](auto D_) {
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_COLOR, 0,
                    k_color<false, NBv><<<nb, bs, 0, c->stream>>>(n, nb, c->pos, c->xold, c->list,
@@ -2282,9 +2419,9 @@ int launch_color(sph_ctx *c, bool with_velocity) {
 int launch_surface(sph_ctx *c) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_SURFACE);
-  const uint32_t nb = blocks_for(n, bs);
-  with_depth(tuned_depth(c, K_SURFACE), [&](auto D_) {
+  const Gather g = gather_launch(c, K_SURFACE, K_SURFACE);
+  const uint32_t bs = g.threads, nb = g.blocks;
+  with_depth(g.depth, [&](auto D_) {
     constexpr int NBv = decltype(D_)::value;
     LAUNCH_TIMED(c, K_SURFACE, 0,
                  k_surface<NBv><<<nb, bs, 0, c->stream>>>(n, nb, c->pos, c->aux, c->list,
@@ -2298,9 +2435,9 @@ int launch_xsph(sph_ctx *c) {
   const uint32_t n = c->n;
   float4 *out = (c->vel == c->vel_a) ? c->vel_b : c->vel_a;
   if (n) {
-    const uint32_t bs = tuned_block(c, K_XSPH);
-    const uint32_t nb = blocks_for(n, bs);
-    with_depth(tuned_depth(c, K_XSPH), [&](auto D_) {
+    const Gather g = gather_launch(c, K_XSPH, K_XSPH);
+    const uint32_t bs = g.threads, nb = g.blocks;
+    with_depth(g.depth, [&](auto D_) {
       constexpr int NBv = decltype(D_)::value;
       LAUNCH_TIMED(c, K_XSPH, 0,
                    k_xsph<NBv><<<nb, bs, 0, c->stream>>>(n, nb, c->pos, c->vel, c->list,
@@ -2315,9 +2452,9 @@ int launch_xsph(sph_ctx *c) {
 int launch_vorticity(sph_ctx *c) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const uint32_t bs = tuned_block(c, K_VORTICITY);
-  const uint32_t nb = blocks_for(n, bs);
-  with_depth(tuned_depth(c, K_VORTICITY), [&](auto D_) {
+  const Gather g = gather_launch(c, K_VORTICITY, K_VORTICITY);
+  const uint32_t bs = g.threads, nb = g.blocks;
+  with_depth(g.depth, [&](auto D_) {
     constexpr int NBv = decltype(D_)::value;
     LAUNCH_TIMED(c, K_VORTICITY, 0,
                  k_vorticity<NBv><<<nb, bs, 0, c->stream>>>(n, nb, c->pos, c->vel, c->list,
@@ -2332,10 +2469,10 @@ int launch_confine(sph_ctx *c, bool commit) {
   const uint32_t n = c->n;
   float4 *out = (c->vel == c->vel_a) ? c->vel_b : c->vel_a;
   if (n) {
-    const uint32_t bs = tuned_block(c, K_CONFINE);
-    const uint32_t nb = blocks_for(n, bs);
+    const Gather g = gather_launch(c, K_CONFINE, K_CONFINE);
+    const uint32_t bs = g.threads, nb = g.blocks;
     if (commit)
-      with_depth(tuned_depth(c, K_CONFINE), [&](auto D_) {
+      with_depth(g.depth, [&](auto D_) {
         constexpr int NBv = decltype(D_)::value;
         LAUNCH_TIMED(c, K_CONFINE, 0,
                        k_confine<true, NBv><<<nb, bs, 0, c->stream>>>(
@@ -2343,7 +2480,7 @@ int launch_confine(sph_ctx *c, bool commit) {
                            c->id_s, c->x_can, c->v_can));
       });
     else
-      with_depth(tuned_depth(c, K_CONFINE), [&](auto D_) {
+      with_depth(g.depth, [&](auto D_) {
         constexpr int NBv = decltype(D_)::value;
         LAUNCH_TIMED(c, K_CONFINE, 0,
                        k_confine<false, NBv><<<nb, bs, 0, c->stream>>>(

@@ -149,3 +149,49 @@ def test_launch_choices_do_not_change_results(depth, block, wide):
         ref.step(1)
         other.step(1)
         _same(ref, other, step)
+
+
+@pytest.mark.parametrize("n,squeeze,wide,calls", [
+    (1, 1.0, False, "fused"), (17, 1.0, False, "staged"), (1000, 0.85, False, "fused"),
+    (1003, 0.85, True, "fused"), (4099, 0.85, True, "staged"), (32768, 1.0, False, "fused"),
+    (32769, 1.0, False, "fused")])
+def test_four_lanes_a_particle_equal_one(n, squeeze, wide, calls):
+    """The gather kernels that small scenes take (four lanes a particle) give the
+    bits of those with one lane, which an explicit depth asks for: both sides of
+    the limit, part-filled waves, lists past 32 entries (lattice spacing times
+    ``squeeze``), both list formats, the fused and the staged calls."""
+    s, side = 0.02, int(np.ceil(np.cbrt(n) - 1e-9))
+    sc = Scene(s, (2.0, 1.0, 1.0), iters=4, tol=1e-3 if calls == "fused" else 0.0, k=0.5, c=0.01,
+               vort_eps=0.01, vort_model=1, lambda_eps=600.0)
+    pos, vel = block_scene((side, side, side), s * squeeze, (0.1, 0.05, 0.1), jitter=0.05, seed=5,
+                           vel_sigma=0.1, swirl=0.3)
+    pos, vel = pos[:n], vel[:n]
+    names = ("density_lambda", "density", "lambda", "dp", "dp_update", "color", "surface", "xsph",
+             "vorticity", "confine")
+    four, one = sc.context(n), sc.context(n)
+    four.set_tuning(wide_lists=wide)
+    one.set_tuning(depth={k: 16 for k in names}, wide_lists=wide)
+    for c in (four, one):
+        c.upload(pos, vel)
+    for step in range(2):
+        for c in (four, one):
+            if calls == "fused":
+                c.step(1)
+                continue
+            c.apply_gravity()
+            c.predict_positions()
+            c.find_all_neighbors()
+            for it in range(3):
+                c.compute_densities()
+                c.compute_lambda()
+                c.update_dps(it)
+                c.update_position_stars()
+            c.update_velocities()
+            c.compute_surface_tension()
+            c.apply_viscosity()
+            c.compute_vorticity()
+            c.apply_vorticity_confinement()
+            c.update_positions()
+        if squeeze < 1.0 and step == 0:  # the solver spreads them
+            assert four.neighbors()[1].max() > 32
+        _same(four, one, step)
