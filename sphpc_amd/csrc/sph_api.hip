@@ -916,6 +916,7 @@ static int substep_launch(sph_ctx *c, bool *warm_out) {
   const bool prev = c->warm_prev_scale > 0.0f && !c->log_on;
   const bool warm = iters > 0 && (c->log_on || c->warm_on || prev);
   *warm_out = warm;
+  const bool finish = iters > 0 && finishes_in_update(c);
   int it0 = 0;
   const float4 *pre_warm = nullptr;
   const bool fallback = warm && !c->log_on && iters > 1;
@@ -924,7 +925,7 @@ static int substep_launch(sph_ctx *c, bool *warm_out) {
     // a batch decides the fallback per scene: errors before the step
     if (fallback && c->nscenes && (rc = launch_scene_errors(c, c->scene_err0))) return rc;
     pre_warm = c->pos;
-    if ((rc = launch_dp_update(c, 0, 0, true))) return rc;
+    if ((rc = launch_dp_update(c, 0, 0, true, finish && iters == 1))) return rc;
     it0 = 1;
   }
   for (int it = it0; it < iters; ++it) {
@@ -933,7 +934,7 @@ static int substep_launch(sph_ctx *c, bool *warm_out) {
       if (c->nscenes && (rc = launch_scene_errors(c))) return rc;
       if ((rc = launch_warm_fallback(c, pre_warm))) return rc;
     }
-    if ((rc = launch_dp_update(c, it, it, warm))) return rc;
+    if ((rc = launch_dp_update(c, it, it, warm, finish && it == iters - 1))) return rc;
   }
   c->last_err_slot = iters > 0 ? iters - 1 : -1;
   if (c->P.density_tolerance > 0.0) {
@@ -944,14 +945,14 @@ static int substep_launch(sph_ctx *c, bool *warm_out) {
   if (c->P.surface_tension) {
     if ((rc = launch_color(c, true))) return rc;
     if ((rc = launch_surface(c))) return rc;
-  } else {
+  } else if (!finish) {
     if ((rc = launch_velocity(c))) return rc;
   }
   if (c->P.viscosity && (rc = launch_xsph(c))) return rc;
   if (c->P.vorticity) {
     if ((rc = launch_vorticity(c))) return rc;
     if ((rc = launch_confine(c, true))) return rc;
-  } else {
+  } else if (!finish) {
     if ((rc = launch_commit(c))) return rc;
   }
   if (warm && (rc = launch_scatter_lambda(c))) return rc;

@@ -336,7 +336,11 @@ int launch_density(sph_ctx *c, int mode, int err_slot);
 // xnext: also the position update of launch_position_stars, into xnext
 int launch_dp(sph_ctx *c, int substep, float4 *xnext = nullptr);
 int launch_position_stars(sph_ctx *c);
-int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate = false);
+// Whether the last launch_dp_update of a substep can also finish it (no velocity
+// terms; the obstacle push not a pass of its own), and the update.
+bool finishes_in_update(const sph_ctx *c);
+int launch_dp_update(sph_ctx *c, int substep, int err_slot, bool accumulate = false,
+                     bool finish = false);
 int launch_velocity(sph_ctx *c);
 int launch_color(sph_ctx *c, bool with_velocity);
 int launch_surface(sph_ctx *c);

@@ -195,3 +195,26 @@ def test_four_lanes_a_particle_equal_one(n, squeeze, wide, calls):
         if squeeze < 1.0 and step == 0:  # the solver spreads them
             assert four.neighbors()[1].max() > 32
         _same(four, one, step)
+
+
+@pytest.mark.parametrize("iters", [0, 1, 4])
+@pytest.mark.parametrize("tol", [0.0, 1e-3, 10.0])
+@pytest.mark.parametrize("depth", [0, 16])
+def test_update_that_ends_the_substep_equals_separate_passes(iters, tol, depth):
+    """Without velocity terms the last position update also makes the velocities
+    and the results by id; with the obstacle push as its own pass (split) those are
+    separate kernels.  Same bits, also where the loop ends within tolerance at once
+    (10), in the middle or never, and without iterations."""
+    sc, ctxs = _pair(tol, iters)
+    p = sc.gpu_params()
+    p.surface_tension = p.viscosity = p.vorticity = 0
+    for c, split in zip(ctxs, (True, False)):
+        c.set_params(p)
+        c.set_tuning(split_collide=split, depth={"dp_update": depth})
+    for step in range(3):
+        for c in ctxs:
+            c.step(1)
+        _same(*ctxs, step)
+        # no iteration, no density pass: the field holds nothing
+        for f in (sa.FIELD_VELOCITY,) + ((sa.FIELD_DENSITY,) if iters else ()):
+            assert np.array_equal(ctxs[0].field(f), ctxs[1].field(f)), (step, f)
