@@ -24,13 +24,21 @@ constexpr int SC_ITEMS = 16;
 constexpr int SC_TILE = SC_THREADS * SC_ITEMS;
 static_assert(SC_TILE == kScanTile, "scratch sized by scan_tiles");
 
+// Every lane of the wave calls it.  Data-parallel moves (shifts within 16 lanes,
+// then lane 15 of each row and lane 31 passed on) in place of six LDS round trips.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  const auto from = [&x](auto ctrl, auto rows) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value,
+                                                 decltype(rows)::value, 0xF, false);
+  };
+  using std::integral_constant;
+  const integral_constant<int, 0xF> all;
+  x += from(integral_constant<int, 0x111>{}, all);
+  x += from(integral_constant<int, 0x112>{}, all);
+  x += from(integral_constant<int, 0x114>{}, all);
+  x += from(integral_constant<int, 0x118>{}, all);
+  x += from(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});
+  x += from(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});
   return x;
 }
 
@@ -75,23 +83,27 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 // --------------------------------------------------------------------------
 // Scan
 // --------------------------------------------------------------------------
-// Thread t of a tile owns entries [t*SC_ITEMS, (t+1)*SC_ITEMS): four 16-byte
-// loads and stores per thread, one block scan per tile.
-__device__ __forceinline__ void load_items(const uint32_t *in, uint32_t i0, uint32_t len,
-                                           uint32_t (&x)[SC_ITEMS]) {
-  if (i0 + SC_ITEMS <= len) {
-    const uint4 *v = reinterpret_cast<const uint4 *>(in + i0);
+// A wave owns 1024 consecutive entries of a tile, a lane four of each 256 of
+// them: one 16-byte load and store a quarter, side by side over the lanes.
+constexpr int SC_QUARTERS = SC_ITEMS / 4;
+__device__ __forceinline__ uint32_t first_item(int q) {
+  return blockIdx.x * SC_TILE + (threadIdx.x >> 6) * (64 * SC_ITEMS) + q * 256 +
+         (threadIdx.x & 63) * 4;
+}
+
+__device__ __forceinline__ void load_items(const uint32_t *in, uint32_t len,
+                                           uint4 (&x)[SC_QUARTERS]) {
 #pragma unroll
-    for (int q = 0; q < SC_ITEMS / 4; ++q) {
-      const uint4 a = v[q];
-      x[4 * q] = a.x;
-      x[4 * q + 1] = a.y;
-      x[4 * q + 2] = a.z;
-      x[4 * q + 3] = a.w;
+  for (int q = 0; q < SC_QUARTERS; ++q) {
+    const uint32_t i = first_item(q);
+    if (i + 4 <= len) {
+      x[q] = *reinterpret_cast<const uint4 *>(in + i);
+    } else {
+      x[q].x = i < len ? in[i] : 0u;
+      x[q].y = i + 1 < len ? in[i + 1] : 0u;
+      x[q].z = i + 2 < len ? in[i + 2] : 0u;
+      x[q].w = 0u;
     }
-  } else {
-#pragma unroll
-    for (int r = 0; r < SC_ITEMS; ++r) x[r] = i0 + r < len ? in[i0 + r] : 0u;
   }
 }
 
@@ -99,11 +111,11 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_tile_sums(const uint32_t *_
                                                                uint32_t len,
                                                                uint32_t *__restrict__ sums) {
   __shared__ uint32_t wtot[4];
-  uint32_t x[SC_ITEMS];
-  load_items(in, blockIdx.x * SC_TILE + threadIdx.x * SC_ITEMS, len, x);
+  uint4 x[SC_QUARTERS];
+  load_items(in, len, x);
   uint32_t s = 0;
 #pragma unroll
-  for (int r = 0; r < SC_ITEMS; ++r) s += x[r];
+  for (int q = 0; q < SC_QUARTERS; ++q) s += (x[q].x + x[q].y) + (x[q].z + x[q].w);
   uint32_t tot;
   block_excl_scan_256(s, wtot, &tot);
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
@@ -131,30 +143,36 @@ enum ScanFrom {
 // One launch costs 4-5 us of a small substep (kernel and gap), and reading up
 // to 7 tiles (28,672 words, all of L2) again costs less; a block reads 2048
 // sums in 8 loads per thread, less than the spine's launch.
-constexpr uint32_t kScanSelfTiles = 8, kScanSumTiles = 2048;
+constexpr uint32_t kScanSelfTiles = 8, kScanLateTiles = 256, kScanSumTiles = 2048;
 
 // in and out may alias with SCAN_SUMS and SCAN_SPINE (in-place scan).
+// Bounded by the writes of a large table (5.9M cells, 23 MB, of which particles are
+// in a tenth): with 16 consecutive entries a thread, each store left in 64 pieces of
+// 16 bytes, 13.4 us; side by side and without reading the empty tiles 6.9.
 template <ScanFrom FROM>
 __global__ __launch_bounds__(SC_THREADS) void k_scan_apply(const uint32_t *in, uint32_t *out,
                                                            uint32_t len,
                                                            const uint32_t *__restrict__ sums,
                                                            int inclusive, int write_total) {
   __shared__ uint32_t wtot[4];
-  const uint32_t i0 = blockIdx.x * SC_TILE + threadIdx.x * SC_ITEMS;
-  uint32_t x[SC_ITEMS];
-  load_items(in, i0, len, x);
+  uint4 x[SC_QUARTERS] = {};
+  // of many tiles, one without a count is not read (a table of cells is mostly
+  // empty); of few, its loads go out before its sum is known
+  const bool late = FROM == SCAN_SUMS && gridDim.x > kScanLateTiles;
+  if (!late) load_items(in, len, x);
   uint32_t before = 0;
   if (FROM == SCAN_SPINE) {
     before = sums[blockIdx.x];
   } else {
     uint32_t own = 0;
     if (FROM == SCAN_SUMS) {
+      if (late && sums[blockIdx.x] != 0u) load_items(in, len, x);
       for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SC_THREADS) own += sums[t];
     } else {
       for (uint32_t t = 0; t < blockIdx.x; ++t) {
         const uint4 *v = reinterpret_cast<const uint4 *>(in + t * SC_TILE) + threadIdx.x;
 #pragma unroll
-        for (int q = 0; q < SC_ITEMS / 4; ++q) {
+        for (int q = 0; q < SC_QUARTERS; ++q) {
           const uint4 a = v[q * SC_THREADS];
           own += (a.x + a.y) + (a.z + a.w);
         }
@@ -162,29 +180,37 @@ __global__ __launch_bounds__(SC_THREADS) void k_scan_apply(const uint32_t *in, u
     }
     block_excl_scan_256(own, wtot, &before);
   }
-  uint32_t own = 0;
+  // scan within the quarters, the quarters' sums before them, the waves' before those
+  uint32_t pre[SC_QUARTERS], run = 0;
 #pragma unroll
-  for (int r = 0; r < SC_ITEMS; ++r) own += x[r];
-  uint32_t tot;
-  uint32_t run = before + block_excl_scan_256(own, wtot, &tot);
-#pragma unroll
-  for (int r = 0; r < SC_ITEMS; ++r) {
-    const uint32_t e = run;
-    run += x[r];
-    x[r] = inclusive ? run : e;
+  for (int q = 0; q < SC_QUARTERS; ++q) {
+    const uint32_t own = (x[q].x + x[q].y) + (x[q].z + x[q].w), inc = wave_incl_scan(own);
+    pre[q] = run + inc - own;
+    run += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
   }
-  if (i0 + SC_ITEMS <= len && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
-    uint4 *o = reinterpret_cast<uint4 *>(out + i0);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) wtot[w] = run;
+  __syncthreads();
 #pragma unroll
-    for (int q = 0; q < SC_ITEMS / 4; ++q)
-      o[q] = make_uint4(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
-  } else {
+  for (int i = 0; i < 3; ++i)
+    if (i < w) before += wtot[i];
+  const bool aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
 #pragma unroll
-    for (int r = 0; r < SC_ITEMS; ++r)
-      if (i0 + r < len) out[i0 + r] = x[r];
+  for (int q = 0; q < SC_QUARTERS; ++q) {
+    const uint32_t i = first_item(q), e0 = before + pre[q], e1 = e0 + x[q].x, e2 = e1 + x[q].y,
+                   e3 = e2 + x[q].z, e4 = e3 + x[q].w;
+    const uint4 o = inclusive ? make_uint4(e1, e2, e3, e4) : make_uint4(e0, e1, e2, e3);
+    if (i + 4 <= len && aligned) {
+      *reinterpret_cast<uint4 *>(out + i) = o;
+    } else {
+      if (i < len) out[i] = o.x;
+      if (i + 1 < len) out[i + 1] = o.y;
+      if (i + 2 < len) out[i + 2] = o.z;
+      if (i + 3 < len) out[i + 3] = o.w;
+    }
+    // the thread holding entry len-1 writes the total after it
+    if (write_total && i < len && len <= i + 4) out[len] = e4;
   }
-  // the thread holding entry len-1 writes the total after it
-  if (write_total && i0 < len && len <= i0 + SC_ITEMS) out[len] = run;
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, uint32_t len) {

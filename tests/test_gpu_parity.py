@@ -103,6 +103,20 @@ def test_cell_bounds_at_the_edges_of_the_scan(cells):
     test_cell_bounds_bit_exact(20_000, cells)
 
 
+@pytest.mark.parametrize("cells", [256 * 4096, 256 * 4096 + 1, 257 * 4096 + 2, 700 * 4096 + 3])
+def test_cell_bounds_of_mostly_empty_tables(cells):
+    """Past 256 tiles of 4096 cells a tile without keys is not read; ends that are
+    no multiple of four, keys in a few tiles, the first and the last cell."""
+    rng = np.random.default_rng(cells)
+    keys = np.concatenate([np.zeros(3), rng.integers(4095, 4098, 50),
+                           rng.integers(130 * 4096, 131 * 4096, 5000), np.full(7, cells - 1)])
+    keys = np.sort(keys).astype(np.uint32)
+    lo, hi = sa.cell_bounds(keys, cells)
+    c = np.arange(cells, dtype=np.uint32)
+    assert np.array_equal(lo, np.searchsorted(keys, c, "left"))
+    assert np.array_equal(hi, np.searchsorted(keys, c, "right"))
+
+
 @pytest.mark.parametrize("n,cap", [(1, 1), (3, 7), (4, 4), (1021, 2000), ((1 << 17) - 1,) * 2,
                                    (1 << 17,) * 2, (5, 1 << 17), (32769, 1 << 17),
                                    ((1 << 19) + 1,) * 2,
