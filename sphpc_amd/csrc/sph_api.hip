@@ -108,8 +108,7 @@ static void derive(sph_ctx *c) {
   d.h = (float)h;
   d.h2 = (float)(h * h);
   d.inv_h = (float)(1.0 / h);
-  d.h2_lo = (float)(h * h * (1.0 - 1e-5));
-  d.h2_hi = (float)(h * h * (1.0 + 1e-5));
+  d.h2_band = (float)(h * h * 1e-5);
   d.h2d = h * h;
   d.rmin = (float)(h * 0.0001);
   d.rmin2 = (float)(h * 0.0001 * h * 0.0001);

@@ -52,7 +52,7 @@ constexpr size_t kPosPad = 8;
 // Device-side constants of one run, all FP32 except the exact-predicate h^2.
 struct DevParams {
   float h, h2, inv_h;
-  float h2_lo, h2_hi;        // guard band around h^2 for the list predicate
+  float h2_band;             // guard band around h^2 of the list predicate
   double h2d;                // (double)h * (double)h, exact
   float rmin, rmin2;         // r floor 1e-4 h (particles.c:125,265,344,636,725)
   float W_norm, DelW_norm, DelW_poly_norm, C_norm;

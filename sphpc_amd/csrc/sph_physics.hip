@@ -111,7 +111,6 @@ __device__ __forceinline__ NbList nb_list(const uint32_t *list, const uint4 *hea
 // to the particle itself when that layer has no candidates), which costs less
 // than it seems: an index past the records instead, which touches no line, made
 // no pass faster.
-constexpr int kBatch = 8;  // candidate batch of the list build
 constexpr uint32_t kQuadStride = kWave * 4;  // list words between a lane's quads
 // Hits the list build buffers in LDS per thread (16 bits each) for the
 // coalesced write-out; later hits of a compact list are stored directly.  At
@@ -687,20 +686,60 @@ __device__ __noinline__ bool inside_exact(float px, float py, float pz, float qx
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ f4u ld4u(const float *p) { return *reinterpret_cast<const f4u *>(p); }
 
-// One candidate of the list build: each mask takes its compare as the next
-// bit, m = 2 m + [r2 < bound], one add-with-carry with the compare in VCC as
-// the carry (two VALU per mask, where the compiler's select, shift and or take
-// two and a half).  Candidates are fed last to first, so candidate t ends at
-// bit t.
-__device__ __forceinline__ void candidate_bits(uint32_t &lo, uint32_t &hi, float r2,
-                                               float h2_lo, float h2_hi) {
-  asm("v_cmp_gt_f32_e32 vcc, %[hl], %[r]\n\t"
-      "v_addc_co_u32_e32 %[lo], vcc, %[lo], %[lo], vcc\n\t"
-      "v_cmp_gt_f32_e32 vcc, %[hh], %[r]\n\t"
-      "v_addc_co_u32_e32 %[hi], vcc, %[hi], %[hi], vcc"
-      : [lo] "+v"(lo), [hi] "+v"(hi)
-      : [r] "v"(r2), [hl] "s"(h2_lo), [hh] "s"(h2_hi)
-      : "vcc");
+// Appends the bits of N candidates, from the coordinate arrays at X, to the masks
+// of hits (r^2 < h^2) and of those to be decided exactly (within the guard band of
+// h^2, wider than any rounding of r^2 - h^2); candidate t ends at bit t, so the last
+// are fed first.  Two 16-byte loads per coordinate: a wave's lanes (about 8 cells)
+// then touch 2-3 cache lines per load instead of about 8 for 16-byte records.  Reads
+// up to 7 entries past a range: each array is padded by kPosPad readable entries.
+// Bounded by the vector L1 (12 bytes a candidate and lane) and, close behind, by the
+// VALU.  A candidate's bit is the sign of r^2 - h^2, shifted in by one instruction, and
+// one minimum3 for two candidates tells whether the wave has any to decide (a NaN,
+// whose sign says nothing, is one), whose bits are then made from the same
+// differences: 7.8 instructions a candidate, against 10 with a compare and an add for
+// each of two thresholds.  k_build_lists with that and the halves of test32 (us):
+// 8.4M particles 876 -> 840, 1M 103 -> 98, 442k 50.3 -> 48.0.
+template <int N>
+__device__ __forceinline__ void test(const float4 &p, const float *X, uint32_t stride,
+                                     const DevParams &P, uint32_t &hits, uint32_t &exact) {
+  f4u x[N / 4], y[N / 4], z[N / 4];
+#pragma unroll
+  for (int v = 0; v < N / 4; ++v) {
+    x[v] = ld4u(X + 4 * v);
+    y[v] = ld4u(X + stride + 4 * v);
+    z[v] = ld4u(X + 2u * stride + 4 * v);
+  }
+  float u[N], nearest = P.h2;
+#pragma unroll
+  for (int t = N - 1; t >= 0; --t) {
+    const float dx = p.x - x[t / 4][t & 3], dy = p.y - y[t / 4][t & 3],
+                dz = p.z - z[t / 4][t & 3];
+    u[t] = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -P.h2)));
+    hits = __builtin_amdgcn_alignbit(hits, __float_as_uint(u[t]), 31);
+  }
+#pragma unroll
+  for (int t = 0; t < N; t += 2)
+    nearest = __builtin_elementwise_minimum(
+        __builtin_elementwise_minimum(nearest, fabsf(u[t])), fabsf(u[t + 1]));
+  exact <<= N;
+  if (__ballot(!(nearest >= P.h2_band)) != 0ull) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) exact |= fabsf(u[t]) >= P.h2_band ? 0u : 1u << t;
+  }
+}
+
+// The masks of up to 32 candidates.  Groups last to first: a lane skips a suffix of
+// the groups, which then come first, while its masks are still 0.  A row of three
+// cells holds 24 particles or a few more, so the last 8 go in two halves.
+__device__ __forceinline__ void test32(const float4 &p, const float *X, uint32_t stride,
+                                       uint32_t len, const DevParams &P, uint32_t &hits,
+                                       uint32_t &exact) {
+#pragma unroll
+  for (int g = 28; g >= 24; g -= 4)
+    if ((uint32_t)g < len) test<4>(p, X + g, stride, P, hits, exact);
+#pragma unroll
+  for (int g = 16; g >= 0; g -= 8)
+    if ((uint32_t)g < len) test<8>(p, X + g, stride, P, hits, exact);
 }
 
 // One thread per sorted particle.  The 3 cells (dx = -1..1) of each (dz, dy)
@@ -782,35 +821,12 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
           // then append the hits of the chunk in j order
           for (uint32_t cb = j0; cb < j1; cb += 32) {
             const uint32_t len = j1 - cb;
-            uint32_t lo = 0u, hi = 0u;  // bits: r2 < h2_lo, r2 < h2_hi
-            // groups last to first: a lane skips a suffix of the groups, which
-            // then come first, while its masks are still 0
-#pragma unroll
-            for (int g = 3; g >= 0; --g) {
-              if (8u * g < len) {
-                // 8 candidates as two 16-byte loads per coordinate array:
-                // a wave's lanes (about 8 cells) then touch 2-3 cache lines per
-                // load instead of about 8 for 16-byte records.  Reads up to 7
-                // entries past j1: each array is padded by kPosPad readable
-                // entries beyond the capacity.
-                const float *X = sx + cb + 8 * g;
-                const f4u x0 = ld4u(X), x1 = ld4u(X + 4);
-                const f4u y0 = ld4u(X + stride), y1 = ld4u(X + stride + 4);
-                const f4u z0 = ld4u(X + 2u * stride), z1 = ld4u(X + 2u * stride + 4);
-                const float qx[kBatch] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-                const float qy[kBatch] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
-                const float qz[kBatch] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
-#pragma unroll
-                for (int t = kBatch - 1; t >= 0; --t) {
-                  const float r2 = sq3(p.x - qx[t], p.y - qy[t], p.z - qz[t]);
-                  candidate_bits(lo, hi, r2, P.h2_lo, P.h2_hi);
-                }
-              }
-            }
+            uint32_t lo = 0u, band = 0u;  // hits, and candidates within the guard band
+            test32(p, sx + cb, stride, len, P, lo, band);
             uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
             if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
-            lo &= keep;
-            uint32_t band = hi & keep & ~lo;  // within the guard band of h^2
+            band &= keep;
+            lo &= keep & ~band;
             while (band) {
               const int t = __builtin_ctz(band);
               band &= band - 1u;
@@ -957,28 +973,12 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
   // hits of the up to 32 candidates [cb, end) as a mask
   auto test = [&](uint32_t cb, uint32_t end) {
     const uint32_t len = end - cb;
-    uint32_t lo = 0u, hi = 0u;  // bits: r2 < h2_lo, r2 < h2_hi (as in k_build_lists)
-#pragma unroll
-    for (int g = 3; g >= 0; --g) {
-      if (8u * g < len) {
-        const float *X = sx + cb + 8 * g;
-        const f4u x0 = ld4u(X), x1 = ld4u(X + 4);
-        const f4u y0 = ld4u(X + stride), y1 = ld4u(X + stride + 4);
-        const f4u z0 = ld4u(X + 2u * stride), z1 = ld4u(X + 2u * stride + 4);
-        const float qx[kBatch] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        const float qy[kBatch] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
-        const float qz[kBatch] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
-#pragma unroll
-        for (int t = kBatch - 1; t >= 0; --t) {
-          const float r2 = sq3(p.x - qx[t], p.y - qy[t], p.z - qz[t]);
-          candidate_bits(lo, hi, r2, P.h2_lo, P.h2_hi);
-        }
-      }
-    }
+    uint32_t lo = 0u, band = 0u;  // as in k_build_lists
+    test32(p, sx + cb, stride, len, P, lo, band);
     uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
     if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
-    lo &= keep;
-    uint32_t band = hi & keep & ~lo;
+    band &= keep;
+    lo &= keep & ~band;
     while (band) {
       const int t = __builtin_ctz(band);
       band &= band - 1u;
