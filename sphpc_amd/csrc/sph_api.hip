@@ -109,6 +109,7 @@ static void derive(sph_ctx *c) {
   d.h2 = (float)(h * h);
   d.inv_h = (float)(1.0 / h);
   d.h2_band = (float)(h * h * 1e-5);
+  d.fixed_scale = kFixedH / h;
   d.h2d = h * h;
   d.rmin = (float)(h * 0.0001);
   d.rmin2 = (float)(h * 0.0001 * h * 0.0001);

@@ -33,6 +33,14 @@ constexpr int kIoChunks = 16;
 // 9.3, 10.0 / 11.4; confinement 7.9 / 6.3, 7.9 / 6.8, 8.6 / 7.8, 8.7 / 9.0.  Two
 // lanes a particle were slower than either from 1k to 133k.
 constexpr int kQuadMax = 1 << 15;
+// k_build_lists tests candidates by 16-bit fixed-point coordinates of kFixedH steps
+// per h, modulo 65536 (8 h; the cells searched lie within 2 h): rounded down, a
+// difference is off by less than 1, and r^2 near h^2 by less than 2 sqrt(3) kFixedH +
+// 3, which kFixedBand covers.  kFixedNaN lies more than h and up to 25 / 8 h from what
+// has its coordinate in the first two cells (a NaN's cell is the first): three such
+// squares fit 31 bits.
+constexpr int kFixedH = 8192, kFixedBand = 28672;
+constexpr uint32_t kFixedNaN = 25 * kFixedH / 8;
 // Particles per block of the per-scene error reduction of a batch.
 constexpr uint32_t kSceneChunk = 4096;
 // Neighbour-list head per particle: the first candidate index of each of the
@@ -53,6 +61,7 @@ constexpr size_t kPosPad = 8;
 struct DevParams {
   float h, h2, inv_h;
   float h2_band;             // guard band around h^2 of the list predicate
+  double fixed_scale;        // kFixedH / h
   double h2d;                // (double)h * (double)h, exact
   float rmin, rmin2;         // r floor 1e-4 h (particles.c:125,265,344,636,725)
   float W_norm, DelW_norm, DelW_poly_norm, C_norm;
@@ -212,8 +221,8 @@ struct sph_ctx {
   float4 *vel_a = nullptr, *vel_b = nullptr, *vel = nullptr;  // vel: current v
   float4 *aux = nullptr;  // colour normal, then vorticity (w = |omega|)
   float4 *pw = nullptr;   // (x*, |omega|) for the confinement gather
-  // sorted x* again as three float arrays (x, then y, then z, soa_stride
-  // apart), written by the reorder pass for the list build's candidate loads
+  // sorted x* again for the list build: three float arrays (x, then y, then z,
+  // soa_stride entries each), or the 16-bit coordinates in the same memory
   float *sx = nullptr;
   uint32_t soa_stride = 0;
   float4 *dpbuf = nullptr;  // staged delta p

@@ -636,6 +636,14 @@ __global__ __launch_bounds__(kBlock) void k_place(uint32_t n, const uint32_t *__
 // Each particle's place in (cell key, id) order, from the ids of its cell that
 // are below its own (8 or so, read by the cell's lanes together), and x*, x,
 // key and id gathered there.
+// Also x* as the list build reads it: three float arrays, or (FIXED) 16-bit
+// coordinates, x and y in one word and z in an array of its own, in the same memory.
+__device__ __forceinline__ uint32_t fixed16(float x, double scale) {
+  const double t = (double)x * scale;
+  return x == x ? (uint32_t)(t - 65536.0 * floor(t * (1.0 / 65536.0))) & 0xFFFFu : kFixedNaN;
+}
+
+template <bool FIXED>
 __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__restrict__ slots,
                                                     const uint32_t *__restrict__ cell_start,
                                                     const float4 *__restrict__ xs_can,
@@ -644,7 +652,8 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__r
                                                     uint32_t *__restrict__ id_s,
                                                     float4 *__restrict__ pos,
                                                     float4 *__restrict__ xold,
-                                                    float *__restrict__ sx, uint32_t stride) {
+                                                    float *__restrict__ sx, uint32_t stride,
+                                                    double fixed_scale) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= n) return;
   const uint2 me = slots[t];
@@ -661,9 +670,15 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__r
   key_s[s] = me.y;
   id_s[s] = me.x;
   pos[s] = q;
-  sx[s] = q.x;
-  sx[stride + s] = q.y;
-  sx[2u * stride + s] = q.z;
+  if (FIXED) {
+    reinterpret_cast<uint32_t *>(sx)[s] =
+        fixed16(q.x, fixed_scale) | fixed16(q.y, fixed_scale) << 16;
+    reinterpret_cast<uint16_t *>(sx + stride)[s] = (uint16_t)fixed16(q.z, fixed_scale);
+  } else {
+    sx[s] = q.x;
+    sx[stride + s] = q.y;
+    sx[2u * stride + s] = q.z;
+  }
   xold[s] = o;
 }
 
@@ -697,8 +712,7 @@ __device__ __forceinline__ f4u ld4u(const float *p) { return *reinterpret_cast<c
 // one minimum3 for two candidates tells whether the wave has any to decide (a NaN,
 // whose sign says nothing, is one), whose bits are then made from the same
 // differences: 7.8 instructions a candidate, against 10 with a compare and an add for
-// each of two thresholds.  k_build_lists with that and the halves of test32 (us):
-// 8.4M particles 876 -> 840, 1M 103 -> 98, 442k 50.3 -> 48.0.
+// each of two thresholds.
 template <int N>
 __device__ __forceinline__ void test(const float4 &p, const float *X, uint32_t stride,
                                      const DevParams &P, uint32_t &hits, uint32_t &exact) {
@@ -742,6 +756,79 @@ __device__ __forceinline__ void test32(const float4 &p, const float *X, uint32_t
     if ((uint32_t)g < len) test<8>(p, X + g, stride, P, hits, exact);
 }
 
+// The same from the 16-bit coordinates: half the bytes through the vector L1 and 5
+// instructions a candidate; one particle in 20 has a pair to decide exactly.
+// w = r^2 - h^2 + kFixedBand in steps^2: negative for a hit, from 0 to below
+// 2 kFixedBand (unsigned) to be decided.  k_build_lists from the float arrays / from
+// these (us): 8.4M particles 840 / 741, 1M 98 / 88.6, 442k 48.0 / 43.8; the
+// reorder, which writes 6 bytes for 12, 174 / 163, 21.5 / 20.6 and 9.9 / 9.8.
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_2 __attribute__((ext_vector_type(2), aligned(2)));
+
+// z.lo^2 + c or z.hi^2 + c, signed.
+__device__ __forceinline__ int square_lo(s16x2 z, int c) {
+  int w;
+  asm("v_mad_i32_i16 %0, %1, %1, %2" : "=v"(w) : "v"(z), "s"(c));
+  return w;
+}
+__device__ __forceinline__ int square_hi(s16x2 z, int c) {
+  int w;
+  asm("v_mad_i32_i16 %0, %1, %1, %2 op_sel:[1,1,0,0]" : "=v"(w) : "v"(z), "s"(c));
+  return w;
+}
+
+template <int N>
+__device__ __forceinline__ void test_fixed(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
+                                           const uint16_t *Z, uint32_t &hits, uint32_t &exact) {
+  uint32_t xy[N], zz[N / 2];
+#pragma unroll
+  for (int v = 0; v < N / 4; ++v) {
+    const u32x4 a = *reinterpret_cast<const u32x4 *>(XY + 4 * v);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xy[4 * v + t] = a[t];
+  }
+  if constexpr (N == 8) {
+    const u32x4_2 a = *reinterpret_cast<const u32x4_2 *>(Z);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) zz[t] = a[t];
+  } else {
+    static_assert(N == 4, "one load of z");
+    const u32x2_2 a = *reinterpret_cast<const u32x2_2 *>(Z);
+    zz[0] = a[0];
+    zz[1] = a[1];
+  }
+  constexpr int c = kFixedBand - kFixedH * kFixedH;
+  uint32_t w[N], nearest = 0xFFFFFFFFu;
+#pragma unroll
+  for (int t = N - 1; t >= 0; --t) {
+    const s16x2 d = pxy - __builtin_bit_cast(s16x2, xy[t]);
+    const s16x2 z = pzz - __builtin_bit_cast(s16x2, zz[t / 2]);
+    w[t] = (uint32_t)__builtin_amdgcn_sdot2(d, d, t & 1 ? square_hi(z, c) : square_lo(z, c),
+                                            false);
+    hits = __builtin_amdgcn_alignbit(hits, w[t], 31);
+  }
+#pragma unroll
+  for (int t = 0; t < N; t += 2) nearest = min(min(nearest, w[t]), w[t + 1]);
+  exact <<= N;
+  if (__ballot(nearest < 2u * kFixedBand) != 0ull) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) exact |= w[t] < 2u * kFixedBand ? 1u << t : 0u;
+  }
+}
+
+__device__ __forceinline__ void test32_fixed(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
+                                             const uint16_t *Z, uint32_t len, uint32_t &hits,
+                                             uint32_t &exact) {
+#pragma unroll
+  for (int g = 28; g >= 24; g -= 4)
+    if ((uint32_t)g < len) test_fixed<4>(pxy, pzz, XY + g, Z + g, hits, exact);
+#pragma unroll
+  for (int g = 16; g >= 0; g -= 8)
+    if ((uint32_t)g < len) test_fixed<8>(pxy, pzz, XY + g, Z + g, hits, exact);
+}
+
 // One thread per sorted particle.  The 3 cells (dx = -1..1) of each (dz, dy)
 // row are consecutive keys, so each row is one contiguous range of sorted
 // indices; walking rows in (dz, dy) order and indices upward reproduces the
@@ -772,6 +859,11 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
   uint32_t *out = list + (size_t)(s >> 6) * kListStride + (s & 63u) * 4u;
   if (s < n) {
     const float4 p = pos[s];
+    const uint32_t *XY = reinterpret_cast<const uint32_t *>(sx);
+    const uint16_t *Z = reinterpret_cast<const uint16_t *>(sx + stride);
+    const s16x2 pxy = __builtin_bit_cast(s16x2, XY[s]), pzz = {(short)Z[s], (short)Z[s]};
+    // a NaN has no neighbours (two of one cell share their 16-bit coordinate)
+    const bool nan = !(p.x == p.x && p.y == p.y && p.z == p.z);
     const Geo G = geo_of<BATCH>(s, P, B);
     const uint32_t key = key_s[s] - G.base;
     const uint32_t cz = key / G.nxy;
@@ -822,9 +914,10 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
           for (uint32_t cb = j0; cb < j1; cb += 32) {
             const uint32_t len = j1 - cb;
             uint32_t lo = 0u, band = 0u;  // hits, and candidates within the guard band
-            test32(p, sx + cb, stride, len, P, lo, band);
+            test32_fixed(pxy, pzz, XY + cb, Z + cb, len, lo, band);
             uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
             if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
+            if (nan) keep = 0u;
             band &= keep;
             lo &= keep & ~band;
             while (band) {
@@ -2115,11 +2208,16 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
     LAUNCH_TIMED(c, K_PLACE, 0,
                  k_place<<<blocks_for(n), kBlock, 0, s>>>(n, c->keys, c->cell_rank, c->cell_start,
                                                           c->slots, c->cell_count));
-    LAUNCH_TIMED(c, K_REORDER, 0,
-                 k_reorder<<<blocks_for(n), kBlock, 0, s>>>(n, c->slots, c->cell_start,
-                                                            c->xs_can, c->x_can, c->key_s,
-                                                            c->id_s, c->pos, c->xold, c->sx,
-                                                            c->soa_stride));
+    if (n <= kRowBuildMax)
+      LAUNCH_TIMED(c, K_REORDER, 0,
+                   k_reorder<false><<<blocks_for(n), kBlock, 0, s>>>(
+                       n, c->slots, c->cell_start, c->xs_can, c->x_can, c->key_s, c->id_s, c->pos,
+                       c->xold, c->sx, c->soa_stride, 0.0));
+    else
+      LAUNCH_TIMED(c, K_REORDER, 0,
+                   k_reorder<true><<<blocks_for(n), kBlock, 0, s>>>(
+                       n, c->slots, c->cell_start, c->xs_can, c->x_can, c->key_s, c->id_s, c->pos,
+                       c->xold, c->sx, c->soa_stride, c->dev.fixed_scale));
     SPH_HIP(hipGetLastError());
   }
   if (n) {

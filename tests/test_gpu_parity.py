@@ -248,6 +248,34 @@ def test_lists_on_both_sides_of_the_build_kernels_limits(dims, wide):
         assert cnt.max() == orc.MAXN and ol["dropped"] > 0
 
 
+@pytest.mark.parametrize("jitter", [0.0, 1e-4, 0.3])
+def test_lists_from_16_bit_coordinates(jitter):
+    """Above 196,608 particles the list build tests 16-bit coordinates that wrap
+    every 8 h, and decides the pairs near h exactly: an exact lattice, whose pairs
+    lie at h or a rounding beside it, one barely off it, and a loose one, over 29 h.
+    Particles that are not a number have no neighbours and are nobody's."""
+    s = 0.02
+    sc = Scene(s, (1.6, 1.6, 1.6))
+    pos, vel = block_scene((59, 59, 59), s, (0.01, 0.01, 0.01), jitter=jitter, seed=9)
+    bad = np.array([0, 1, 2, 3481, 77_777, 77_778, 205_000])
+    ctx = _staged_search(sc, pos, vel)
+    ol = oracle_lists(sc.o, *_soa(ctx.field(sa.FIELD_POSITION_STAR)))
+    ids, cnt = ctx.neighbors()
+    assert np.array_equal(cnt, ol["cnt"])
+    want, n = ol["nbr"].reshape(len(pos), -1), len(pos)
+    mask = np.arange(orc.MAXN)[None, :] < cnt[:, None]
+    assert np.array_equal(ids.reshape(n, -1)[mask], want[mask])
+    pos[bad[:3], 0] = np.nan
+    pos[bad[3:5], 1] = -np.float32(np.nan)
+    pos[bad[5:]] = np.nan
+    ids, cnt = _staged_search(sc, pos, vel).neighbors()
+    mask &= ~np.isin(want, bad)
+    mask[bad] = False
+    assert np.array_equal(cnt, mask.sum(1))
+    got = np.arange(orc.MAXN)[None, :] < cnt[:, None]
+    assert np.array_equal(ids.reshape(n, -1)[got], want[mask])
+
+
 def test_cell_tables_at_the_grid_ends_and_a_crowded_cell():
     """Cell tables from the sorted keys' run ends: runs in the first and the
     last cell of the grid, particles clamped onto the box faces from outside,
