@@ -108,7 +108,6 @@ static void derive(sph_ctx *c) {
   d.h = (float)h;
   d.h2 = (float)(h * h);
   d.inv_h = (float)(1.0 / h);
-  d.h2_band = (float)(h * h * 1e-5);
   d.fixed_scale = kFixedH / h;
   d.h2d = h * h;
   d.rmin = (float)(h * 0.0001);
@@ -190,7 +189,7 @@ static void free_all(sph_ctx *c) {
                   c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage,
                   c->list, c->list_head,
                   c->stats, c->stats_read, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
-                  c->pw, c->sx, c->lam_acc, c->lam_prev, c->feat, c->scenes_dev, c->scene_of,
+                  c->pw, c->fixed_xy, c->fixed_z, c->lam_acc, c->lam_prev, c->feat, c->scenes_dev, c->scene_of,
                   c->batch_sdf, c->scene_err, c->scene_err0, c->scene_chunks,
                   c->warm_net};
   for (void *b : bufs)
@@ -281,6 +280,8 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
   c->cap = max_particles;
   const size_t f4 = sizeof(float4) * cap, u4 = sizeof(uint32_t) * cap;
   const size_t groups = (cap + kWave - 1) / kWave;
+  const size_t fixed_xy = sizeof(uint32_t) * (cap + kPosPad);
+  const size_t fixed_z = sizeof(uint16_t) * (cap + kPosPad);
   struct {
     void **p;
     size_t bytes;
@@ -291,8 +292,7 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       {(void **)&c->key_s, u4},       {(void **)&c->id_s, u4},
       {(void **)&c->cell_count, sizeof(uint32_t) * (c->cells + 1ull)},
       {(void **)&c->cell_start, sizeof(uint32_t) * (c->cells + 1ull)},
-      {(void **)&c->pos_a, f4 + sizeof(float4) * kPosPad},
-      {(void **)&c->pos_b, f4 + sizeof(float4) * kPosPad},
+      {(void **)&c->pos_a, f4},       {(void **)&c->pos_b, f4},
       {(void **)&c->xold, f4},        {(void **)&c->vel_a, f4},
       {(void **)&c->vel_b, f4},       {(void **)&c->aux, f4},
       {(void **)&c->dpbuf, f4},       {(void **)&c->rho, sizeof(float) * cap},
@@ -300,7 +300,8 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       {(void **)&c->list, sizeof(uint32_t) * groups * kListStride},
       {(void **)&c->list_head, sizeof(uint4) * cap},
       {(void **)&c->pw, f4},
-      {(void **)&c->sx, sizeof(float) * 3 * (cap + kPosPad)},
+      {(void **)&c->fixed_xy, fixed_xy},
+      {(void **)&c->fixed_z, fixed_z},
       // here and not on first use: a search must not end between its counts and
       // their placing, which zeroes them
       {(void **)&c->scan.tile_sums, sizeof(uint32_t) * scan_tiles(c->cells)},
@@ -319,13 +320,13 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
   // C = 0 until a density stage runs (lambda from it is zero, as the
   // reference's from its zero-initialised density array)
   if (e == hipSuccess) e = hipMemsetAsync(c->cstage, 0, sizeof(float) * cap, c->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(c->pos_a, 0, f4 + sizeof(float4) * kPosPad, c->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(c->pos_b, 0, f4 + sizeof(float4) * kPosPad, c->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(c->sx, 0, sizeof(float) * 3 * (cap + kPosPad), c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(c->pos_a, 0, f4, c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(c->pos_b, 0, f4, c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(c->fixed_xy, 0, fixed_xy, c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(c->fixed_z, 0, fixed_z, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return fail(hip_fail(e, "context initialisation"));
   c->pos = c->pos_a;
-  c->soa_stride = (uint32_t)(cap + kPosPad);
   c->scan.tile_cap = scan_tiles(c->cells);
   c->vel = c->vel_a;
   *out = c;

@@ -33,7 +33,7 @@ constexpr int kIoChunks = 16;
 // 9.3, 10.0 / 11.4; confinement 7.9 / 6.3, 7.9 / 6.8, 8.6 / 7.8, 8.7 / 9.0.  Two
 // lanes a particle were slower than either from 1k to 133k.
 constexpr int kQuadMax = 1 << 15;
-// k_build_lists tests candidates by 16-bit fixed-point coordinates of kFixedH steps
+// The list build tests candidates by 16-bit fixed-point coordinates of kFixedH steps
 // per h, modulo 65536 (8 h; the cells searched lie within 2 h): rounded down, a
 // difference is off by less than 1, and r^2 near h^2 by less than 2 sqrt(3) kFixedH +
 // 3, which kFixedBand covers.  kFixedNaN lies more than h and up to 25 / 8 h from what
@@ -51,7 +51,7 @@ constexpr uint32_t kSceneChunk = 4096;
 constexpr uint32_t kHeadCount = 0xFFu;
 constexpr uint32_t kHeadWide = 1u << 31;
 constexpr uint32_t kCompactSpan = 1u << 16;
-// The sorted position arrays hold kPosPad readable entries past the capacity:
+// The 16-bit position arrays hold kPosPad readable entries past the capacity:
 // the list build loads candidates 8 at a time and may read up to 7 entries
 // past the end of a range (their tests are discarded).
 constexpr size_t kPosPad = 8;
@@ -60,7 +60,6 @@ constexpr size_t kPosPad = 8;
 // Device-side constants of one run, all FP32 except the exact-predicate h^2.
 struct DevParams {
   float h, h2, inv_h;
-  float h2_band;             // guard band around h^2 of the list predicate
   double fixed_scale;        // kFixedH / h
   double h2d;                // (double)h * (double)h, exact
   float rmin, rmin2;         // r floor 1e-4 h (particles.c:125,265,344,636,725)
@@ -221,10 +220,9 @@ struct sph_ctx {
   float4 *vel_a = nullptr, *vel_b = nullptr, *vel = nullptr;  // vel: current v
   float4 *aux = nullptr;  // colour normal, then vorticity (w = |omega|)
   float4 *pw = nullptr;   // (x*, |omega|) for the confinement gather
-  // sorted x* again for the list build: three float arrays (x, then y, then z,
-  // soa_stride entries each), or the 16-bit coordinates in the same memory
-  float *sx = nullptr;
-  uint32_t soa_stride = 0;
+  // sorted x* again for the list build, in 16-bit coordinates (x | y << 16, and z)
+  uint32_t *fixed_xy = nullptr;
+  uint16_t *fixed_z = nullptr;
   float4 *dpbuf = nullptr;  // staged delta p
   float *rho = nullptr;
   // stage path: C = rho/rho0 - 1 of the last density stage (read by a lambda

@@ -636,14 +636,13 @@ __global__ __launch_bounds__(kBlock) void k_place(uint32_t n, const uint32_t *__
 // Each particle's place in (cell key, id) order, from the ids of its cell that
 // are below its own (8 or so, read by the cell's lanes together), and x*, x,
 // key and id gathered there.
-// Also x* as the list build reads it: three float arrays, or (FIXED) 16-bit
-// coordinates, x and y in one word and z in an array of its own, in the same memory.
+// Also x* as the list build reads it, in 16-bit coordinates: x and y in one word, z
+// in an array of its own.
 __device__ __forceinline__ uint32_t fixed16(float x, double scale) {
   const double t = (double)x * scale;
   return x == x ? (uint32_t)(t - 65536.0 * floor(t * (1.0 / 65536.0))) & 0xFFFFu : kFixedNaN;
 }
 
-template <bool FIXED>
 __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__restrict__ slots,
                                                     const uint32_t *__restrict__ cell_start,
                                                     const float4 *__restrict__ xs_can,
@@ -652,7 +651,8 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__r
                                                     uint32_t *__restrict__ id_s,
                                                     float4 *__restrict__ pos,
                                                     float4 *__restrict__ xold,
-                                                    float *__restrict__ sx, uint32_t stride,
+                                                    uint32_t *__restrict__ fixed_xy,
+                                                    uint16_t *__restrict__ fixed_z,
                                                     double fixed_scale) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= n) return;
@@ -670,15 +670,8 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__r
   key_s[s] = me.y;
   id_s[s] = me.x;
   pos[s] = q;
-  if (FIXED) {
-    reinterpret_cast<uint32_t *>(sx)[s] =
-        fixed16(q.x, fixed_scale) | fixed16(q.y, fixed_scale) << 16;
-    reinterpret_cast<uint16_t *>(sx + stride)[s] = (uint16_t)fixed16(q.z, fixed_scale);
-  } else {
-    sx[s] = q.x;
-    sx[stride + s] = q.y;
-    sx[2u * stride + s] = q.z;
-  }
+  fixed_xy[s] = fixed16(q.x, fixed_scale) | fixed16(q.y, fixed_scale) << 16;
+  fixed_z[s] = (uint16_t)fixed16(q.z, fixed_scale);
   xold[s] = o;
 }
 
@@ -697,71 +690,22 @@ __device__ __noinline__ bool inside_exact(float px, float py, float pz, float qx
   return r2 < h2d;
 }
 
-// Four consecutive floats from a 4-byte-aligned address (one 16-byte load).
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f4u ld4u(const float *p) { return *reinterpret_cast<const f4u *>(p); }
-
-// Appends the bits of N candidates, from the coordinate arrays at X, to the masks
-// of hits (r^2 < h^2) and of those to be decided exactly (within the guard band of
-// h^2, wider than any rounding of r^2 - h^2); candidate t ends at bit t, so the last
-// are fed first.  Two 16-byte loads per coordinate: a wave's lanes (about 8 cells)
-// then touch 2-3 cache lines per load instead of about 8 for 16-byte records.  Reads
-// up to 7 entries past a range: each array is padded by kPosPad readable entries.
-// Bounded by the vector L1 (12 bytes a candidate and lane) and, close behind, by the
-// VALU.  A candidate's bit is the sign of r^2 - h^2, shifted in by one instruction, and
-// one minimum3 for two candidates tells whether the wave has any to decide (a NaN,
-// whose sign says nothing, is one), whose bits are then made from the same
-// differences: 7.8 instructions a candidate, against 10 with a compare and an add for
-// each of two thresholds.
-template <int N>
-__device__ __forceinline__ void test(const float4 &p, const float *X, uint32_t stride,
-                                     const DevParams &P, uint32_t &hits, uint32_t &exact) {
-  f4u x[N / 4], y[N / 4], z[N / 4];
-#pragma unroll
-  for (int v = 0; v < N / 4; ++v) {
-    x[v] = ld4u(X + 4 * v);
-    y[v] = ld4u(X + stride + 4 * v);
-    z[v] = ld4u(X + 2u * stride + 4 * v);
-  }
-  float u[N], nearest = P.h2;
-#pragma unroll
-  for (int t = N - 1; t >= 0; --t) {
-    const float dx = p.x - x[t / 4][t & 3], dy = p.y - y[t / 4][t & 3],
-                dz = p.z - z[t / 4][t & 3];
-    u[t] = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -P.h2)));
-    hits = __builtin_amdgcn_alignbit(hits, __float_as_uint(u[t]), 31);
-  }
-#pragma unroll
-  for (int t = 0; t < N; t += 2)
-    nearest = __builtin_elementwise_minimum(
-        __builtin_elementwise_minimum(nearest, fabsf(u[t])), fabsf(u[t + 1]));
-  exact <<= N;
-  if (__ballot(!(nearest >= P.h2_band)) != 0ull) {
-#pragma unroll
-    for (int t = 0; t < N; ++t) exact |= fabsf(u[t]) >= P.h2_band ? 0u : 1u << t;
-  }
-}
-
-// The masks of up to 32 candidates.  Groups last to first: a lane skips a suffix of
-// the groups, which then come first, while its masks are still 0.  A row of three
-// cells holds 24 particles or a few more, so the last 8 go in two halves.
-__device__ __forceinline__ void test32(const float4 &p, const float *X, uint32_t stride,
-                                       uint32_t len, const DevParams &P, uint32_t &hits,
-                                       uint32_t &exact) {
-#pragma unroll
-  for (int g = 28; g >= 24; g -= 4)
-    if ((uint32_t)g < len) test<4>(p, X + g, stride, P, hits, exact);
-#pragma unroll
-  for (int g = 16; g >= 0; g -= 8)
-    if ((uint32_t)g < len) test<8>(p, X + g, stride, P, hits, exact);
-}
-
-// The same from the 16-bit coordinates: half the bytes through the vector L1 and 5
-// instructions a candidate; one particle in 20 has a pair to decide exactly.
-// w = r^2 - h^2 + kFixedBand in steps^2: negative for a hit, from 0 to below
-// 2 kFixedBand (unsigned) to be decided.  k_build_lists from the float arrays / from
-// these (us): 8.4M particles 840 / 741, 1M 98 / 88.6, 442k 48.0 / 43.8; the
-// reorder, which writes 6 bytes for 12, 174 / 163, 21.5 / 20.6 and 9.9 / 9.8.
+// Appends the bits of N candidates, from the 16-bit coordinates at XY and Z, to the
+// masks of hits (r^2 < h^2) and of those that the rounding leaves to be decided
+// exactly, one for every 20 particles; candidate t ends at bit t, so the last are fed
+// first.  With w = r^2 - h^2 + kFixedBand in steps^2, negative is a hit, and 0 to below
+// 2 kFixedBand (unsigned) to be decided.  16-byte loads of consecutive candidates: a
+// wave's lanes (about 8 cells) then touch 2-3 cache lines per load instead of about 8
+// for 16-byte records.  Reads up to 7 entries past a range, which kPosPad allows.
+//
+// The walk is bounded by the bytes its loads return through the vector L1 and, close
+// behind, by the VALU.  This takes 6 bytes and 5 instructions a candidate: the squares
+// in one dot product and one multiply-add, the bit from the sign, and one min3 for two
+// candidates to see whether the wave has any to decide.  With float arrays it was 12
+// bytes and 10 instructions, later 7.8.  k_build_lists (us), 12 bytes and 10 / 7.8 and
+// the halves of test32 / this: 8.4M particles 876 / 840 / 741, 1M 103 / 98 / 88.6,
+// 442k 50.3 / 48.0 / 43.8; k_build_rows at 131k 20.2 / 20.2 / 19.1, at 4k 7.4 / 7.4 /
+// 7.5; the reorder, which writes half the bytes, 174 / 174 / 163 at 8.4M.
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_2 __attribute__((ext_vector_type(4), aligned(2)));
@@ -780,8 +724,8 @@ __device__ __forceinline__ int square_hi(s16x2 z, int c) {
 }
 
 template <int N>
-__device__ __forceinline__ void test_fixed(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
-                                           const uint16_t *Z, uint32_t &hits, uint32_t &exact) {
+__device__ __forceinline__ void test(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
+                                     const uint16_t *Z, uint32_t &hits, uint32_t &exact) {
   uint32_t xy[N], zz[N / 2];
 #pragma unroll
   for (int v = 0; v < N / 4; ++v) {
@@ -818,15 +762,18 @@ __device__ __forceinline__ void test_fixed(s16x2 pxy, s16x2 pzz, const uint32_t 
   }
 }
 
-__device__ __forceinline__ void test32_fixed(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
-                                             const uint16_t *Z, uint32_t len, uint32_t &hits,
-                                             uint32_t &exact) {
+// The masks of up to 32 candidates.  Groups last to first: a lane skips a suffix of
+// the groups, which then come first, while its masks are still 0.  A row of three
+// cells holds 24 particles or a few more, so the last 8 go in two halves.
+__device__ __forceinline__ void test32(s16x2 pxy, s16x2 pzz, const uint32_t *XY,
+                                       const uint16_t *Z, uint32_t len, uint32_t &hits,
+                                       uint32_t &exact) {
 #pragma unroll
   for (int g = 28; g >= 24; g -= 4)
-    if ((uint32_t)g < len) test_fixed<4>(pxy, pzz, XY + g, Z + g, hits, exact);
+    if ((uint32_t)g < len) test<4>(pxy, pzz, XY + g, Z + g, hits, exact);
 #pragma unroll
   for (int g = 16; g >= 0; g -= 8)
-    if ((uint32_t)g < len) test_fixed<8>(pxy, pzz, XY + g, Z + g, hits, exact);
+    if ((uint32_t)g < len) test<8>(pxy, pzz, XY + g, Z + g, hits, exact);
 }
 
 // One thread per sorted particle.  The 3 cells (dx = -1..1) of each (dz, dy)
@@ -847,7 +794,7 @@ __device__ __forceinline__ void test32_fixed(s16x2 pxy, s16x2 pzz, const uint32_
 template <bool BATCH>
 __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
     uint32_t n, uint32_t nblocks, const float4 *__restrict__ pos,
-    const float *__restrict__ sx, uint32_t stride,
+    const uint32_t *__restrict__ XY, const uint16_t *__restrict__ Z,
     const uint32_t *__restrict__ key_s, const uint32_t *__restrict__ cstart, DevParams P,
     uint32_t *__restrict__ list, uint4 *__restrict__ head, uint32_t *__restrict__ stats,
     uint32_t *__restrict__ pair_partial, int force_wide, BatchDev B) {
@@ -859,8 +806,6 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
   uint32_t *out = list + (size_t)(s >> 6) * kListStride + (s & 63u) * 4u;
   if (s < n) {
     const float4 p = pos[s];
-    const uint32_t *XY = reinterpret_cast<const uint32_t *>(sx);
-    const uint16_t *Z = reinterpret_cast<const uint16_t *>(sx + stride);
     const s16x2 pxy = __builtin_bit_cast(s16x2, XY[s]), pzz = {(short)Z[s], (short)Z[s]};
     // a NaN has no neighbours (two of one cell share their 16-bit coordinate)
     const bool nan = !(p.x == p.x && p.y == p.y && p.z == p.z);
@@ -914,7 +859,7 @@ __global__ __launch_bounds__(kBlock, 7) void k_build_lists(
           for (uint32_t cb = j0; cb < j1; cb += 32) {
             const uint32_t len = j1 - cb;
             uint32_t lo = 0u, band = 0u;  // hits, and candidates within the guard band
-            test32_fixed(pxy, pzz, XY + cb, Z + cb, len, lo, band);
+            test32(pxy, pzz, XY + cb, Z + cb, len, lo, band);
             uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
             if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
             if (nan) keep = 0u;
@@ -1015,8 +960,9 @@ constexpr uint32_t kOneRowBuildMax = 40960, kRowBuildMax = 196608;
 
 template <bool BATCH, int ROWS>
 __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
-    uint32_t n, const float4 *__restrict__ pos, const float *__restrict__ sx, uint32_t stride,
-    const uint32_t *__restrict__ key_s, const uint32_t *__restrict__ cstart, DevParams P,
+    uint32_t n, const float4 *__restrict__ pos, const uint32_t *__restrict__ XY,
+    const uint16_t *__restrict__ Z, const uint32_t *__restrict__ key_s,
+    const uint32_t *__restrict__ cstart, DevParams P,
     uint32_t *__restrict__ list, uint4 *__restrict__ head, uint32_t *__restrict__ stats,
     uint32_t *__restrict__ pair_partial, int force_wide, BatchDev B) {
   constexpr int WAVES = 9 / ROWS;
@@ -1032,9 +978,13 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
 #pragma unroll
   for (int k = 0; k < ROWS; ++k) j0[k] = j1[k] = 0u;
   float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  bool direct = force_wide != 0;
+  s16x2 pxy = {0, 0}, pzz = {0, 0};
+  bool direct = force_wide != 0, nan = false;
   if (s < n) {
     p = pos[s];
+    pxy = __builtin_bit_cast(s16x2, XY[s]);
+    pzz = s16x2{(short)Z[s], (short)Z[s]};
+    nan = !(p.x == p.x && p.y == p.y && p.z == p.z);
     const Geo G = geo_of<BATCH>(s, P, B);
     const uint32_t key = key_s[s] - G.base;
     const uint32_t cz = key / G.nxy;
@@ -1064,12 +1014,13 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
     }
   }
   // hits of the up to 32 candidates [cb, end) as a mask
-  auto test = [&](uint32_t cb, uint32_t end) {
+  auto hits_of = [&](uint32_t cb, uint32_t end) {
     const uint32_t len = end - cb;
     uint32_t lo = 0u, band = 0u;  // as in k_build_lists
-    test32(p, sx + cb, stride, len, P, lo, band);
+    test32(pxy, pzz, XY + cb, Z + cb, len, lo, band);
     uint32_t keep = len >= 32u ? ~0u : (1u << len) - 1u;
     if (s - cb < 32u) keep &= ~(1u << (s - cb));  // not the particle itself
+    if (nan) keep = 0u;
     band &= keep;
     lo &= keep & ~band;
     while (band) {
@@ -1087,7 +1038,7 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
   for (int k = 0; k < ROWS; ++k) {
     m0[k] = 0u;
     for (uint32_t cb = j0[k]; cb < j1[k]; cb += 32u) {
-      const uint32_t m = test(cb, j1[k]);
+      const uint32_t m = hits_of(cb, j1[k]);
       mine += (uint32_t)__builtin_popcount(m);
       if (cb == j0[k]) m0[k] = m;
     }
@@ -1107,7 +1058,7 @@ __global__ __launch_bounds__(9 / ROWS * kWave, 7) void k_build_rows(
 #pragma unroll
   for (int k = 0; k < ROWS; ++k) {
     for (uint32_t cb = j0[k]; cb < j1[k] && at < (uint32_t)kMaxNb; cb += 32u) {
-      uint32_t m = cb == j0[k] ? m0[k] : test(cb, j1[k]);
+      uint32_t m = cb == j0[k] ? m0[k] : hits_of(cb, j1[k]);
       while (m && at < (uint32_t)kMaxNb) {
         const uint32_t j = cb + (uint32_t)__builtin_ctz(m);
         m &= m - 1u;
@@ -2190,11 +2141,13 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
     } else if (c->nscenes) {
       LAUNCH_TIMED(c, K_HASH, 0,
                    k_hash<true><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last, B));
+                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last,
+                       B));
     } else {
       LAUNCH_TIMED(c, K_HASH, 0,
                    k_hash<false><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last, B));
+                       n, c->xs_can, c->keys, c->cell_rank, c->cell_count, c->dev, c->stats, last,
+                       B));
     }
   } else {
     k_substep_init<<<1, kBlock, 0, s>>>(c->stats);
@@ -2208,16 +2161,10 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
     LAUNCH_TIMED(c, K_PLACE, 0,
                  k_place<<<blocks_for(n), kBlock, 0, s>>>(n, c->keys, c->cell_rank, c->cell_start,
                                                           c->slots, c->cell_count));
-    if (n <= kRowBuildMax)
-      LAUNCH_TIMED(c, K_REORDER, 0,
-                   k_reorder<false><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->slots, c->cell_start, c->xs_can, c->x_can, c->key_s, c->id_s, c->pos,
-                       c->xold, c->sx, c->soa_stride, 0.0));
-    else
-      LAUNCH_TIMED(c, K_REORDER, 0,
-                   k_reorder<true><<<blocks_for(n), kBlock, 0, s>>>(
-                       n, c->slots, c->cell_start, c->xs_can, c->x_can, c->key_s, c->id_s, c->pos,
-                       c->xold, c->sx, c->soa_stride, c->dev.fixed_scale));
+    LAUNCH_TIMED(c, K_REORDER, 0,
+                 k_reorder<<<blocks_for(n), kBlock, 0, s>>>(
+                     n, c->slots, c->cell_start, c->xs_can, c->x_can, c->key_s, c->id_s, c->pos,
+                     c->xold, c->fixed_xy, c->fixed_z, c->dev.fixed_scale));
     SPH_HIP(hipGetLastError());
   }
   if (n) {
@@ -2227,7 +2174,7 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
 #define BUILD_ROWS(BAT, ROWS)                                                                  \
   LAUNCH_TIMED(c, K_BUILD_LISTS, 0,                                                            \
                (k_build_rows<BAT, ROWS><<<groups, 9 / ROWS * kWave, 0, s>>>(                   \
-                   n, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev, c->list,  \
+                   n, c->pos, c->fixed_xy, c->fixed_z, c->key_s, c->cell_start, c->dev, c->list,  \
                    c->list_head, c->stats, c->pair_partial, wide, B)))
       if (n <= kOneRowBuildMax) {
         if (c->nscenes) BUILD_ROWS(true, 1); else BUILD_ROWS(false, 1);
@@ -2242,12 +2189,12 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
       if (c->nscenes)
         LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
                      k_build_lists<true><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
-                         n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
+                         n, nb, c->pos, c->fixed_xy, c->fixed_z, c->key_s, c->cell_start, c->dev,
                          c->list, c->list_head, c->stats, c->pair_partial, wide, B));
       else
         LAUNCH_TIMED(c, K_BUILD_LISTS, 0,
                      k_build_lists<false><<<nb, bs, kLdsHits * bs * sizeof(uint16_t), s>>>(
-                         n, nb, c->pos, c->sx, c->soa_stride, c->key_s, c->cell_start, c->dev,
+                         n, nb, c->pos, c->fixed_xy, c->fixed_z, c->key_s, c->cell_start, c->dev,
                          c->list, c->list_head, c->stats, c->pair_partial, wide, B));
       c->pair_blocks = nb;
     }

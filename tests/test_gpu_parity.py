@@ -249,15 +249,16 @@ def test_lists_on_both_sides_of_the_build_kernels_limits(dims, wide):
 
 
 @pytest.mark.parametrize("jitter", [0.0, 1e-4, 0.3])
-def test_lists_from_16_bit_coordinates(jitter):
-    """Above 196,608 particles the list build tests 16-bit coordinates that wrap
+@pytest.mark.parametrize("side", [30, 50, 59])
+def test_lists_from_16_bit_coordinates(side, jitter):
+    """The list build (one kernel for each side) tests 16-bit coordinates that wrap
     every 8 h, and decides the pairs near h exactly: an exact lattice, whose pairs
-    lie at h or a rounding beside it, one barely off it, and a loose one, over 29 h.
-    Particles that are not a number have no neighbours and are nobody's."""
+    lie at h or a rounding beside it, one barely off it, and a loose one, over 15 to
+    29 h.  Particles that are not a number have no neighbours and are nobody's."""
     s = 0.02
     sc = Scene(s, (1.6, 1.6, 1.6))
-    pos, vel = block_scene((59, 59, 59), s, (0.01, 0.01, 0.01), jitter=jitter, seed=9)
-    bad = np.array([0, 1, 2, 3481, 77_777, 77_778, 205_000])
+    pos, vel = block_scene((side,) * 3, s, (0.01, 0.01, 0.01), jitter=jitter, seed=9)
+    bad = np.array([0, 1, 2, 3481, 17_777, 17_778, 26_000])
     ctx = _staged_search(sc, pos, vel)
     ol = oracle_lists(sc.o, *_soa(ctx.field(sa.FIELD_POSITION_STAR)))
     ids, cnt = ctx.neighbors()
