@@ -78,8 +78,8 @@ __device__ __forceinline__ NbList nb_list(const uint32_t *list, const uint4 *hea
 }
 
 // Launch bounds of the delta-p, density, colour and confinement kernels: at
-// up to 16 gathers in flight at most 128 VGPRs, i.e. 4 waves per SIMD, which all
-// of them meet without spilling (at 3 waves delta p measured 7% slower, colour
+// up to 16 gathers in flight at most 128 VGPRs, i.e. 4 waves per SIMD, which density
+// and delta p meet without spilling, colour and confinement with 15 spilled (at 3 waves delta p measured 7% slower, colour
 // and confinement 2-3%).  Five waves (96 VGPRs) would spill 164-220 bytes.
 #define GATHER_BOUNDS(NB) __launch_bounds__(kBlock, (NB) <= 16 ? 4 : 1)
 
@@ -97,15 +97,18 @@ __device__ __forceinline__ NbList nb_list(const uint32_t *list, const uint4 *hea
 //
 // The first batch's quads are loaded together with the particle and its head
 // (their place does not depend on it), which takes one memory round trip off
-// every pass.  With PREFETCH the quads of batch k+1 are issued right after the
+// every pass.  With kRaw the quads of batch k+1 are issued right after the
 // gathers of batch k and stay raw until their batch: 8 registers, where decoded
 // indices took 16 and spilled (20 bytes in delta p), and a last half batch
 // decodes only its own half.  Decoding in a block of its own, before the first
 // gather issues, keeps the gathers together: interleaved with it, the surface
 // pass took 643 us against 551 and every other pass 1-7% more.  Measured at 8.4M
-// particles against decoded prefetch: density+lambda 358 -> 323 us, delta p 317
-// -> 303, surface 562 -> 551, colour, confinement and vorticity within 1%, XSPH
-// (whose two-array gathers take no prefetch now, 546 us with it) 527 -> 539.
+// particles against decoded prefetch (kIndices): density+lambda 358 -> 323 us, delta p
+// 317 -> 303, surface 562 -> 551, vorticity within 1%, XSPH (whose two-array gathers
+// take no prefetch now, 546 us with it) 527 -> 539.  Colour and confinement at 16
+// gathers, whose arithmetic is shortest, decode the next batch beside it (kIndices):
+// 308 and 337 us against 315 and 344 with raw quads, and 398 and 477 against 413 and
+// 490 where lists are longer (33 on average for 28).
 // Slots past c are never used; their gathers load a valid index (the particle
 // itself in a wide list, the layer-2 base in a compact one, which the build sets
 // to the particle itself when that layer has no candidates), which costs less
@@ -176,11 +179,14 @@ __device__ __forceinline__ void decode(const NbList &nl, const Quads<NB, WIDE> &
   }
 }
 
+// What a batch fetches of the next one's list before its arithmetic.
+enum Prefetch { kNone, kRaw, kIndices };
+
 // A wavefront runs each batch for its longest list.  Batches in which no lane's
 // list ends skip the per-neighbour count test, and a last batch in which every
 // lane ends within NB/2 neighbours runs only NB/2 of them (the wave's longest
 // list, not the mean, sets the work: half batches cut the padding slots).
-template <typename T, int NB, bool PREFETCH, bool WIDE, typename Load, typename Body>
+template <typename T, int NB, int PREFETCH, bool WIDE, typename Load, typename Body>
 __device__ __forceinline__ void gather_loop(const NbList &nl, const uint4 *first, uint32_t self,
                                             Load &load, Body &body) {
   Quads<NB, WIDE> r;
@@ -191,27 +197,33 @@ __device__ __forceinline__ void gather_loop(const NbList &nl, const uint4 *first
 #pragma unroll
     for (int u = 0; u < Quads<NB, WIDE>::kCount; ++u) r.q[u] = first[u];
   }
+  uint32_t j[NB];
+  if (PREFETCH == kIndices) decode<NB>(nl, r, 0, self, j);
   for (int k0 = 0; k0 < c; k0 += NB) {
     // the lanes still in the loop have c > k0
-    if (!PREFETCH && k0 > 0) r.load(nl, k0);
+    if (PREFETCH == kNone && k0 > 0) r.load(nl, k0);
     if (NB >= 16 && __ballot(k0 + NB / 2 < c) == 0ull) {
-      uint32_t j[NB / 2];
-      decode<NB / 2>(nl, r, k0, self, j);
-      __builtin_amdgcn_sched_barrier(0);
+      uint32_t h[NB / 2];
+      if (PREFETCH != kIndices) {
+        decode<NB / 2>(nl, r, k0, self, h);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       T q[NB / 2];
 #pragma unroll
-      for (int b = 0; b < NB / 2; ++b) q[b] = load(j[b]);
+      for (int b = 0; b < NB / 2; ++b) q[b] = load(PREFETCH == kIndices ? j[b] : h[b]);
 #pragma unroll
       for (int b = 0; b < NB / 2; ++b)
         if (k0 + b < c) body(q[b]);
     } else {
-      uint32_t j[NB];
-      decode<NB>(nl, r, k0, self, j);
-      __builtin_amdgcn_sched_barrier(0);
+      if (PREFETCH != kIndices) {
+        decode<NB>(nl, r, k0, self, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       T q[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) q[b] = load(j[b]);
-      if (PREFETCH) r.load(nl, k0 + NB);
+      if (PREFETCH != kNone) r.load(nl, k0 + NB);
+      if (PREFETCH == kIndices) decode<NB>(nl, r, k0 + NB, self, j);
       if (__ballot(k0 + NB > c) == 0ull) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) body(q[b]);
@@ -224,7 +236,7 @@ __device__ __forceinline__ void gather_loop(const NbList &nl, const uint4 *first
   }
 }
 
-template <typename T, int NB, bool PREFETCH = true, typename Load, typename Body>
+template <typename T, int NB, int PREFETCH, typename Load, typename Body>
 __device__ __forceinline__ void for_neighbors(const uint32_t *list, const uint4 *head, uint32_t s,
                                               int *count, Load load, Body body) {
   uint4 first[NB / 8];
@@ -315,7 +327,7 @@ __device__ __forceinline__ void quad_loop(const NbList &nl, const uint4 &first, 
 
 // acc = the sums of term(load(j)) over the neighbours j of particle s, in list
 // order, with NB gathers in flight or (kQuad) four lanes a particle.
-template <typename T, int NB, bool PREFETCH, int NA, int P, typename Load, typename Term>
+template <typename T, int NB, int PREFETCH, int NA, int P, typename Load, typename Term>
 __device__ __forceinline__ void sum_neighbors(const uint32_t *list, const uint4 *head, uint32_t s,
                                               int *count, float (&acc)[NA], Load load,
                                               Term term) {
@@ -1195,13 +1207,13 @@ __global__ GATHER_BOUNDS(NB) void k_density_lambda(
     };
     if constexpr (MODE == 1) {
       float none[1];
-      sum_neighbors<float4, NB, true, 1, 1>(list, head, s, &cnt, none, load,
+      sum_neighbors<float4, NB, kRaw, 1, 1>(list, head, s, &cnt, none, load,
                                             [&](const float4 &q) {
         S += density_term(sq3(p.x - q.x, p.y - q.y, p.z - q.z), P);
         return Terms<1>{{0.0f}, {0.0f}};
       });
     } else {
-      sum_neighbors<float4, NB, true, 4, 1>(list, head, s, &cnt, sg, load, term);
+      sum_neighbors<float4, NB, kRaw, 4, 1>(list, head, s, &cnt, sg, load, term);
     }
     if constexpr (NB == kQuad) S = quad_sum(S);
     float C;
@@ -1302,7 +1314,7 @@ __device__ __forceinline__ float3 dp_sum(const float4 &p, const float4 *pos, uin
   int cnt;
   float a[3];
   const Records16 G(pos, n);
-  sum_neighbors<float4, NB, true, 3, 1>(
+  sum_neighbors<float4, NB, kRaw, 3, 1>(
       list, head, s, &cnt, a, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1488,7 +1500,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_lambda(
     float mx = 0.0f, my = 0.0f, mz = 0.0f, dv = 0.0f;
     const Records16 Gp(pos, n), Go(xold, n);
     auto load = [&](uint32_t j) { return Pair4{Gp[j], Go[j]}; };
-    for_neighbors<Pair4, NB, false>(list, head, s, &cnt, load, [&](const Pair4 &qq) {
+    for_neighbors<Pair4, NB, kNone>(list, head, s, &cnt, load, [&](const Pair4 &qq) {
       const float4 &q = qq.a, &qo = qq.b;
       const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       const float r2 = sq3(dx, dy, dz);
@@ -1701,7 +1713,7 @@ __global__ GATHER_BOUNDS(NB) void k_color(uint32_t n, uint32_t nblocks,
   int cnt;
   float a[3];
   const Records16 G(pos, n);
-  sum_neighbors<float4, NB, true, 3, 1>(
+  sum_neighbors<float4, NB, NB >= 16 ? kIndices : kRaw, 3, 1>(
       list, head, s, &cnt, a, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1735,7 +1747,7 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_surface(uint32_t
   float f[3];
   const Records16 Gp(pos, n), Gc(color, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gc[j]}; };
-  sum_neighbors<Pair4, NB, false, 3, 1>(list, head, s, &cnt, f, load, [&](const Pair4 &qc) {
+  sum_neighbors<Pair4, NB, kNone, 3, 1>(list, head, s, &cnt, f, load, [&](const Pair4 &qc) {
     const float4 &q = qc.a, &cq = qc.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1779,7 +1791,7 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_xsph(uint32_t n,
   float a[3];
   const Records16 Gp(pos, n), Gv(vin, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  sum_neighbors<Pair4, NB, false, 3, 1>(list, head, s, &cnt, a, load, [&](const Pair4 &qv) {
+  sum_neighbors<Pair4, NB, kNone, 3, 1>(list, head, s, &cnt, a, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float u = P.h2 - fmaf(dy * dy * dz, dz, dx * dx);
@@ -1810,7 +1822,7 @@ __global__ __launch_bounds__(kBlock) void k_vorticity(uint32_t n, uint32_t nbloc
   float o[3];
   const Records16 Gp(pos, n), Gv(vel, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  sum_neighbors<Pair4, NB, false, 3, 2>(list, head, s, &cnt, o, load, [&](const Pair4 &qv) {
+  sum_neighbors<Pair4, NB, kNone, 3, 2>(list, head, s, &cnt, o, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
@@ -1849,7 +1861,7 @@ __global__ GATHER_BOUNDS(NB) void k_confine(
   float e[3];
   // only x_j and |omega_j| of the neighbour are needed
   const Records16 G(pw, n);
-  sum_neighbors<float4, NB, true, 3, 1>(
+  sum_neighbors<float4, NB, NB >= 16 ? kIndices : kRaw, 3, 1>(
       list, head, s, &cnt, e, [&](uint32_t j) { return G[j]; }, [&](const float4 &q) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         const float r2c = fmaxf(sq3(dx, dy, dz), P.rmin2);
