@@ -31,7 +31,7 @@ constexpr int kIoChunks = 16;
 // 8.3 / 7.6, 8.4 / 8.6; surface 8.9 / 6.5, 9.2 / 7.8, 9.8 / 8.9, 10.4 / 10.9; XSPH
 // 7.7 / 6.2, 8.0 / 6.9, 8.5 / 8.7, 9.2 / 10.3; vorticity 8.2 / 6.5, 8.3 / 7.5, 9.2 /
 // 9.3, 10.0 / 11.4; confinement 7.9 / 6.3, 7.9 / 6.8, 8.6 / 7.8, 8.7 / 9.0.  Two
-// lanes a particle were slower than either from 1k to 133k.
+// lanes a particle lay between: all the kernels 2% faster at 47k, 1-8% slower elsewhere.
 constexpr int kQuadMax = 1 << 15;
 // The list build tests candidates by 16-bit fixed-point coordinates of kFixedH steps
 // per h, modulo 65536 (8 h; the cells searched lie within 2 h): rounded down, a

@@ -104,11 +104,12 @@ __device__ __forceinline__ NbList nb_list(const uint32_t *list, const uint4 *hea
 // gather issues, keeps the gathers together: interleaved with it, the surface
 // pass took 643 us against 551 and every other pass 1-7% more.  Measured at 8.4M
 // particles against decoded prefetch (kIndices): density+lambda 358 -> 323 us, delta p
-// 317 -> 303, surface 562 -> 551, vorticity within 1%, XSPH (whose two-array gathers
-// take no prefetch now, 546 us with it) 527 -> 539.  Colour and confinement at 16
-// gathers, whose arithmetic is shortest, decode the next batch beside it (kIndices):
-// 308 and 337 us against 315 and 344 with raw quads, and 398 and 477 against 413 and
-// 490 where lists are longer (33 on average for 28).
+// 317 -> 303, surface 562 -> 551, vorticity within 1%.  Colour, confinement and XSPH at
+// 16 gathers, whose arithmetic is shortest, decode the next batch beside it (kIndices):
+// 309, 336 and 500 us against 317, 343 and 504 with raw quads (XSPH: without a
+// prefetch, as with raw quads it is slower still), and 397, 476 and 712 against 414,
+// 490 and 729 where lists are longer (33 on average for 28).  The same made surface
+// 630 us for 499 and vorticity 561 for 530.
 // Slots past c are never used; their gathers load a valid index (the particle
 // itself in a wide list, the layer-2 base in a compact one, which the build sets
 // to the particle itself when that layer has no candidates), which costs less
@@ -222,8 +223,12 @@ __device__ __forceinline__ void gather_loop(const NbList &nl, const uint4 *first
       T q[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) q[b] = load(j[b]);
-      if (PREFETCH != kNone) r.load(nl, k0 + NB);
-      if (PREFETCH == kIndices) decode<NB>(nl, r, k0 + NB, self, j);
+      if (PREFETCH == kRaw) r.load(nl, k0 + NB);
+      if (PREFETCH == kIndices) {
+        Quads<NB, WIDE> next;  // not r, which would be held over the loop
+        next.load(nl, k0 + NB);
+        decode<NB>(nl, next, k0 + NB, self, j);
+      }
       if (__ballot(k0 + NB > c) == 0ull) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) body(q[b]);
@@ -1791,7 +1796,7 @@ __global__ __launch_bounds__(kBlock, (NB) <= 16 ? 3 : 1) void k_xsph(uint32_t n,
   float a[3];
   const Records16 Gp(pos, n), Gv(vin, n);
   auto load = [&](uint32_t j) { return Pair4{Gp[j], Gv[j]}; };
-  sum_neighbors<Pair4, NB, kNone, 3, 1>(list, head, s, &cnt, a, load, [&](const Pair4 &qv) {
+  sum_neighbors<Pair4, NB, NB >= 16 ? kIndices : kNone, 3, 1>(list, head, s, &cnt, a, load, [&](const Pair4 &qv) {
     const float4 &q = qv.a, &vq = qv.b;
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float u = P.h2 - fmaf(dy * dy * dz, dz, dx * dx);
