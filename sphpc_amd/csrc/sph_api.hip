@@ -819,6 +819,7 @@ extern "C" int sph_compute_densities(sph_ctx *c) {
   int rc = require_lists(c);
   if (rc) return rc;
   const int slot = std::min(c->staged_slot, kMaxIters);
+  if ((rc = launch_clear_errors(c, slot))) return rc;
   c->staged_slot++;
   c->last_err_slot = slot;
   // density_to_w keeps rho in pos.w for the velocity passes.  With a fixed
@@ -1006,6 +1007,7 @@ static int substep_graph(sph_ctx *c) {
   c->vel = a.vel;
   c->pair_blocks = a.pair_blocks;
   c->last_err_slot = a.last_err_slot;
+  c->err_cleared = c->P.solve_iterations;  // the captured search's
   c->sorted_valid = c->lists_valid = true;
   substep_finish(c, a.warm);
   return SPH_OK;

@@ -286,6 +286,9 @@ struct sph_ctx {
   } graph_after{};
   int last_err_slot = -1;
   int staged_slot = 0;
+  // error words are of this search's passes up to this iteration: a fused search
+  // clears those of its iterations only, a later density stage its own
+  int err_cleared = -1;
   // state generation: bumped by every call that may change the state; the
   // stage path's density pass records it, and the lambda stage switches to the
   // buffer with that pass's lambda when nothing ran in between
@@ -355,6 +358,8 @@ int launch_xsph(sph_ctx *c);
 int launch_vorticity(sph_ctx *c);
 int launch_confine(sph_ctx *c, bool commit);
 int launch_commit(sph_ctx *c);
+// Clears the error words up to iteration `last` that the last search left.
+int launch_clear_errors(sph_ctx *c, int last);
 int launch_collect_stats(sph_ctx *c);
 int launch_collide_soa(float *x, float *y, float *z, uint32_t n, const SdfDev &o,
                        hipStream_t s);

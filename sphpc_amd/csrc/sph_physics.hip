@@ -1921,6 +1921,14 @@ __global__ __launch_bounds__(kBlock) void k_collect_stats(const uint32_t *__rest
   if (lane == 0) out[STAT_ERR0 + it] = m;
 }
 
+// The error words of iterations first..last, for density stages past those that the
+// last search cleared.
+__global__ __launch_bounds__(kBlock) void k_clear_errors(uint32_t *stats, uint32_t first,
+                                                         uint32_t last) {
+  const uint32_t e = blockIdx.x * kBlock + threadIdx.x;
+  if (e < (last + 1u - first) * kErrSlots) stats[err_word(first, e)] = 0u;
+}
+
 // clear_substep_stats for a context without particles.
 __global__ __launch_bounds__(kBlock) void k_substep_init(uint32_t *stats) {
   clear_substep_stats(stats, kMaxIters);
@@ -2144,6 +2152,7 @@ int launch_neighbor_search(sph_ctx *c, bool fused) {
   const BatchDev B = c->batch();
   // the stage calls may run any number of density passes
   const uint32_t last = (uint32_t)(fused ? c->P.solve_iterations : kMaxIters);
+  c->err_cleared = (int)last;
   if (n) {
     if (fused && c->nscenes) {
       LAUNCH_TIMED(c, K_PREDICT_HASH, 0,
@@ -2590,6 +2599,16 @@ int launch_commit(sph_ctx *c) {
                k_commit<<<blocks_for(n), kBlock, 0, c->stream>>>(n, c->pos, c->vel, c->id_s,
                                                                  c->x_can, c->v_can));
   SPH_HIP(hipGetLastError());
+  return SPH_OK;
+}
+
+int launch_clear_errors(sph_ctx *c, int last) {
+  if (last <= c->err_cleared) return SPH_OK;
+  const uint32_t first = (uint32_t)(c->err_cleared + 1);
+  k_clear_errors<<<blocks_for((last + 1u - first) * kErrSlots), kBlock, 0, c->stream>>>(
+      c->stats, first, (uint32_t)last);
+  SPH_HIP(hipGetLastError());
+  c->err_cleared = last;
   return SPH_OK;
 }
 

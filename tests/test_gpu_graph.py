@@ -218,3 +218,35 @@ def test_update_that_ends_the_substep_equals_separate_passes(iters, tol, depth):
         # no iteration, no density pass: the field holds nothing
         for f in (sa.FIELD_VELOCITY,) + ((sa.FIELD_DENSITY,) if iters else ()):
             assert np.array_equal(ctxs[0].field(f), ctxs[1].field(f)), (step, f)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("passes,iters", [(6, 8), (130, 2)])
+def test_density_stage_after_substeps_of_fewer_iterations(graph, passes, iters):
+    """A density stage reports its own pass's maximum also where its slot (they go on
+    counting over fused substeps, up to 128) holds an older and larger one: of a
+    substep of more iterations than the later ones, or of earlier stages."""
+    s = 0.02
+    sc = Scene(s, (1.0, 1.0, 1.0), iters=iters, lambda_eps=600.0)
+    dense, _ = block_scene((12, 12, 12), 0.8 * s, (0.1, 0.1, 0.1), jitter=0.01, seed=2)
+    loose, _ = block_scene((12, 12, 12), 1.3 * s, (0.1, 0.1, 0.1), jitter=0.01, seed=2)
+    with sc.context(len(dense)) as c:
+        c.set_graph(graph)
+        c.upload(dense)
+        c.predict_positions()
+        c.find_all_neighbors()
+        for _ in range(passes):
+            c.compute_densities()
+        assert c.stats().max_density_error > 0.1
+        c.step(3)
+        c.upload(loose)
+        p = sc.gpu_params()
+        p.solve_iterations = 2
+        c.set_params(p)
+        c.step(3)
+        for _ in range(2):
+            c.compute_densities()
+            assert c.stats().max_density_error == 0.0
+            assert np.max(c.field(sa.FIELD_DENSITY)) < 1000.0
+        c.step(1)
+        assert c.stats().max_density_error == c.residuals()[-1]
