@@ -159,10 +159,11 @@ __device__ __forceinline__ void mlp32_square(const float *ops, const floatx16_t 
 // 1 / (1 + e^-z) to about 1 ulp: e^-z as the hardware exp2 of -z log2(e) in two
 // floats, and the hardware reciprocal with one Newton step (8 VALU and two
 // transcendentals; expf and two IEEE divisions are about 40).  z is held to
-// [-87, 100] for the exponential only, past which e^-z is 0 or the sigmoid
-// below 2e-38.
+// [-88.5, 100] for the exponential only: e^88.5 is still finite, and its reciprocal,
+// below the normal range, is 0 from v_rcp_f32.  So z * sigmoid32(z) ends at 0 however
+// large -z is; a bound with a normal reciprocal leaves 1.6e-38 z (-1.6 at -1e38).
 __device__ __forceinline__ float sigmoid32(float z) {
-  const float zc = __builtin_amdgcn_fmed3f(z, -87.0f, 100.0f);
+  const float zc = __builtin_amdgcn_fmed3f(z, -88.5f, 100.0f);
   const float t = -1.44269504f * zc;  // log2(e) = 1.44269502 + 1.92596303e-8
   const float lo = fmaf(-1.92596303e-8f, zc, fmaf(-1.44269504f, zc, -t));
   const float p = __builtin_amdgcn_exp2f(t);

@@ -167,3 +167,29 @@ def test_training_on_gpu_reduces_loss():
     l1, _ = net.gradient(xb, tb, count)
     record("mlp_training", loss0=l0, loss400=l1)
     assert l1 < 0.1 * l0, (l0, l1)
+
+
+@pytest.mark.parametrize("z", [-3e38, -1e38, -1e34, -1e30, -1e10, -1000.0, -100.0, -89.0, -88.5,
+                               -88.0, -87.5, -87.3, -87.0, -80.0, -20.0, -3.0, 0.0, 3.0, 20.0, 90.0,
+                               110.0, 1e5, 1e38])
+def test_activation_over_the_range_of_floats(z):
+    """One hidden unit's SiLU and its derivative, which goes to 0 (z and 1) however
+    large -z (z) is.  A few ulp, and 1e-36 where the sigmoid leaves the normal range."""
+    theta = np.zeros(sa.MLP_PARAMS, np.float32)
+    theta[5184 + 7] = z    # b2
+    theta[5248 + 7] = 1.0  # w3
+    net = sa.Mlp()
+    net.set_weights(theta)
+    net.set_normalization(np.zeros(12), np.ones(12), 0.0, 1.0)
+    xb = sa.DeviceBuffer.from_array(np.zeros((1, sa.MLP_STRIDE), np.float32))
+    yb = sa.DeviceBuffer(4)
+    net.forward(xb, 1, yb)
+    z = float(np.float32(z))
+    sig = 1.0 / (1.0 + np.exp(min(-z, 700.0)))
+    y, want = float(yb.to_array(np.float32, 1)[0]), z * sig
+    assert abs(y - want) <= 4e-7 * abs(want) + 1e-36, (y, want)
+    if z <= 20.0:  # target y - 1: the residual and the output's gradient are 1
+        tb = sa.DeviceBuffer.from_array(np.array([y - 1.0], np.float32))
+        _, g = net.gradient(xb, tb, 1)
+        dy, want = float(np.float32(y) - np.float32(y - 1.0)), sig * (1.0 + z * (1.0 - sig))
+        assert abs(g[5184 + 7] - dy * want) <= 1e-6 * max(abs(want), sig) + 1e-36, (g[5191], want)
