@@ -6,11 +6,10 @@
 
 #include <algorithm>
 #include <atomic>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "sph_internal.h"
+#include "sph_io.h"
 
 namespace sph {
 
@@ -599,7 +598,6 @@ extern "C" int sph_set_obstacle(sph_ctx *c, const sph_obstacle_desc *o) {
 // host copies the next or the previous one, and several threads copy because one
 // does 27 GB/s.  8.4M particles with velocities: upload 10.2 -> 5.3 ms, download
 // 10.3 -> 4.2 ms; 4096: 23 -> 17 us and 26 -> 17 us (a copy on the device less).
-constexpr int kIoThreads = 4;
 // Below this capacity one chunk and the calling thread (3 MB, 120 us; starting
 // three threads takes 50).
 constexpr int kIoOneChunk = 1 << 17;
@@ -665,34 +663,6 @@ static int io_buffers(sph_ctx *c) {
     return hip_fail(e, "hipHostMalloc (state transfer staging)");
   }
   return SPH_OK;
-}
-
-// Runs work(k) for every chunk k of `chunks`, on this thread and, for more than
-// one chunk, up to kIoThreads - 1 more; without them where none can be started.
-// `mine`, if given, is called on this thread between its own chunks.
-template <class Work, class Mine>
-static void io_chunks(size_t chunks, Work work, Mine mine) {
-  std::atomic<size_t> next{0};
-  auto take = [&]() {
-    const size_t k = next.fetch_add(1);
-    if (k < chunks) work(k);
-    return k < chunks;
-  };
-  std::thread helpers[kIoThreads - 1];
-  for (size_t t = 0; t + 1 < std::min<size_t>(kIoThreads, chunks); ++t) {
-    try {
-      helpers[t] = std::thread([&]() {
-        while (take()) {
-        }
-      });
-    } catch (const std::system_error &) {
-      break;
-    }
-  }
-  while (take()) mine();
-  for (std::thread &h : helpers)
-    if (h.joinable()) h.join();
-  mine();
 }
 
 extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *y,
