@@ -597,15 +597,19 @@ extern "C" int sph_set_obstacle(sph_ctx *c, const sph_obstacle_desc *o) {
 // a thread, 1 KB a wave and array.  Chunks let the bus, at 55 GB/s, run while the
 // host copies the next or the previous one, and several threads copy because one
 // does 27 GB/s.  8.4M particles with velocities: upload 10.2 -> 5.3 ms, download
-// 10.3 -> 4.2 ms; 4096: 23 -> 17 us and 26 -> 17 us (a copy on the device less).
-// Below this capacity one chunk and the calling thread (3 MB, 120 us; starting
-// three threads takes 50).
-constexpr int kIoOneChunk = 1 << 17;
+// 10.3 -> 4.2 ms; 4096: 31 -> 27 us and 33 -> 26 us (a copy on the device less).
+constexpr int kIoChunk = 1 << 15;  // particles, at least (up to kIoChunks chunks)
+// Particles from which helper threads copy too: starting three takes some 30 us.  One
+// thread / four, us: upload 200k particles 152 / 190, 400k 273 / 320, 800k 634 / 550;
+// download 200k 163 / 161, 400k 320 / 285.  131k on one thread in one chunk take 136 and
+// 147 us (up, down), in four 108 and 118; with copies by the DMA engines in place of the
+// kernels' own reads and writes 128 and 163.
+constexpr size_t kIoUploadHelp = 1 << 19, kIoDownloadHelp = 1 << 18;
 
 static size_t io_chunk(const sph_ctx *c) {
   const size_t cap = (size_t)std::max(c->cap, 1);
-  if (cap < (size_t)kIoOneChunk) return (cap + 3) & ~(size_t)3;
-  return std::max<size_t>(32768, ((cap + kIoChunks - 1) / kIoChunks + 1023) & ~(size_t)1023);
+  if (cap <= (size_t)kIoChunk) return (cap + 3) & ~(size_t)3;
+  return std::max<size_t>(kIoChunk, ((cap + kIoChunks - 1) / kIoChunks + 1023) & ~(size_t)1023);
 }
 
 __global__ __launch_bounds__(kBlock) void k_pack_state(uint32_t n, uint32_t chunk,
@@ -653,10 +657,11 @@ __global__ __launch_bounds__(kBlock) void k_unpack_state(uint32_t n, uint32_t ch
 // event per chunk, on first use.
 static int io_buffers(sph_ctx *c) {
   if (c->io_host) return SPH_OK;
-  for (hipEvent_t &e : c->io_done)
-    if (!e) SPH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   const size_t chunk = io_chunk(c), cap = (size_t)std::max(c->cap, 1);
-  const size_t bytes = sizeof(float) * 6 * chunk * ((cap + chunk - 1) / chunk);
+  const size_t chunks = (cap + chunk - 1) / chunk, bytes = sizeof(float) * 6 * chunk * chunks;
+  for (size_t k = 0; chunks > 1 && k < chunks; ++k)
+    if (!c->io_done[k])
+      SPH_HIP(hipEventCreateWithFlags(&c->io_done[k], hipEventDisableTiming));
   const hipError_t e = hipHostMalloc(&c->io_host, bytes, hipHostMallocDefault);
   if (e != hipSuccess) {
     c->io_host = nullptr;
@@ -688,7 +693,7 @@ extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *
     std::atomic<bool> staged[kIoChunks] = {};
     size_t sent = 0;
     io_chunks(
-        chunks,
+        chunks, un >= kIoUploadHelp ? kIoThreads : 1,
         [&](size_t k) {
           const size_t first = k * chunk, m = std::min(chunk, un - first);
           float *to = c->io_host + 6 * first;
@@ -736,7 +741,7 @@ extern "C" int sph_download_state(sph_ctx *c, float *x, float *y, float *z, floa
     if (chunks == 1) SPH_HIP(hipStreamSynchronize(c->stream));
     std::atomic<int> failed{hipSuccess};
     io_chunks(
-        chunks,
+        chunks, un >= kIoDownloadHelp ? kIoThreads : 1,
         [&](size_t k) {
           if (chunks > 1) {
             const hipError_t e = hipEventSynchronize(c->io_done[k]);

@@ -141,6 +141,15 @@ def test_state_transfer_round_trip(n, cap):
         assert np.array_equal(y, vel[:, 1]) and np.array_equal(vz, pos[:, 2])
 
 
+@pytest.mark.parametrize("n,cap", [(1 << 15,) * 2, ((1 << 15) + 1,) * 2, (1 << 15, 1 << 20),
+                                   ((1 << 18) - 1,) * 2, (1 << 18,) * 2, ((1 << 19) - 1,) * 2,
+                                   (1 << 19,) * 2])
+def test_state_transfer_at_the_limits_of_its_chunks(n, cap):
+    """One chunk up to 2^15 particles of capacity; helper threads from 2^18 particles
+    (download) and 2^19 (upload)."""
+    test_state_transfer_round_trip(n, cap)
+
+
 # ---------------------------------------------------------------------------
 # Neighbour search in the staged pipeline (neighbors.c:68-298)
 # ---------------------------------------------------------------------------

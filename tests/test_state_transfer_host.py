@@ -29,7 +29,7 @@ extern "C" int transfer(size_t chunks) {  // as a C entry: nothing may be thrown
   static std::atomic<int> done[64];
   for (auto &d : done) d = 0;
   int calls = 0;
-  sph::io_chunks(chunks, [&](size_t k) { done[k]++; }, [&]() { ++calls; });
+  sph::io_chunks(chunks, sph::kIoThreads, [&](size_t k) { done[k]++; }, [&]() { ++calls; });
   for (size_t k = 0; k < 64; ++k)
     if (done[k] != (k < chunks ? 1 : 0)) return 1;
   return calls > 0 ? 0 : 1;
