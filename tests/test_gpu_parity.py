@@ -236,6 +236,31 @@ def test_counting_sort_of_scattered_ids(n, cells_used):
             assert np.array_equal(en, np.searchsorted(k, c, "right"))
 
 
+@pytest.mark.parametrize("crowd", [15, 16, 17, 18, 32, 33, 34, 64, 81, 500])
+def test_counting_sort_of_crowded_cells(crowd):
+    """Cells of one population, ids scattered over them: a particle's place among its
+    cell's ids is counted sixteen at a time past 16, and as scalars by wavefronts that
+    lie in one cell."""
+    sc = Scene(0.02, (1.0, 0.8, 0.6))
+    rng = np.random.default_rng(crowd)
+    cells = rng.permutation(1000)[:max(3, 5000 // crowd)]
+    corner = np.stack([cells % 10, cells // 10 % 10, cells // 100], 1) * sc.h
+    pos = np.repeat(corner, crowd, 0) + rng.uniform(0.1, 0.9, (len(cells) * crowd, 3)) * sc.h
+    pos = pos[rng.permutation(len(pos))].astype(np.float32)
+    n = len(pos)
+    with sc.context(n) as ctx:
+        ctx.upload(pos)
+        ctx.predict_positions()
+        ctx.find_all_neighbors()
+        xs, ys, zs = _soa(ctx.field(sa.FIELD_POSITION_STAR))
+        keys = np.zeros(n, np.uint32)
+        L.orc_hash_particles(n, xs, ys, zs, C.byref(sc.o), keys, np.zeros(n, np.uint32))
+        assert set(np.unique(keys, return_counts=True)[1]) == {crowd}
+        order = np.argsort(keys, kind="stable").astype(np.uint32)
+        k, i = ctx.sorted_pairs()
+        assert np.array_equal(i, order) and np.array_equal(k, keys[order])
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("dims", [(1, 1, 1), (13, 5, 1), (34, 34, 35), (35, 35, 34),
                                   (58, 58, 58), (59, 59, 59)])
