@@ -187,7 +187,7 @@ static void free_all(sph_ctx *c) {
                   c->key_s, c->id_s, c->cell_count, c->cell_start, c->pos_a, c->pos_b, c->xold,
                   c->vel_a, c->vel_b, c->aux, c->dpbuf, c->rho, c->cstage,
                   c->list, c->list_head,
-                  c->stats, c->stats_read, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
+                  c->stats, c->pair_partial, c->red, c->sdf_buf, c->scan.tile_sums,
                   c->pw, c->fixed_xy, c->fixed_z, c->lam_acc, c->lam_prev, c->feat, c->scenes_dev, c->scene_of,
                   c->batch_sdf, c->scene_err, c->scene_err0, c->scene_chunks,
                   c->warm_net};
@@ -305,7 +305,6 @@ static int ctx_allocate(sph_ctx *c, int max_particles, sph_ctx **out) {
       // their placing, which zeroes them
       {(void **)&c->scan.tile_sums, sizeof(uint32_t) * scan_tiles(c->cells)},
       {(void **)&c->stats, sizeof(uint32_t) * STAT_WORDS},
-      {(void **)&c->stats_read, sizeof(uint32_t) * STAT_READ_WORDS},
       {(void **)&c->pair_partial, sizeof(uint32_t) * blocks_for((uint32_t)cap, kWave)},
       {(void **)&c->red, sizeof(double) * std::max<size_t>(4, blocks_for((uint32_t)cap))},
   };
@@ -653,20 +652,22 @@ __global__ __launch_bounds__(kBlock) void k_unpack_state(uint32_t n, uint32_t ch
   if (with_velocity) put(v, 3);
 }
 
-// Pinned staging (6 floats per particle of the capacity, in whole chunks) and an
-// event per chunk, on first use.
+// Pinned staging (6 floats per particle of the capacity, in whole chunks, and the
+// statistics' words) and an event per chunk, on first use.
 static int io_buffers(sph_ctx *c) {
   if (c->io_host) return SPH_OK;
   const size_t chunk = io_chunk(c), cap = (size_t)std::max(c->cap, 1);
-  const size_t chunks = (cap + chunk - 1) / chunk, bytes = sizeof(float) * 6 * chunk * chunks;
+  const size_t chunks = (cap + chunk - 1) / chunk, words = 6 * chunk * chunks;
   for (size_t k = 0; chunks > 1 && k < chunks; ++k)
     if (!c->io_done[k])
       SPH_HIP(hipEventCreateWithFlags(&c->io_done[k], hipEventDisableTiming));
-  const hipError_t e = hipHostMalloc(&c->io_host, bytes, hipHostMallocDefault);
+  const hipError_t e = hipHostMalloc(&c->io_host, sizeof(float) * (words + STAT_READ_WORDS),
+                                     hipHostMallocDefault);
   if (e != hipSuccess) {
     c->io_host = nullptr;
     return hip_fail(e, "hipHostMalloc (state transfer staging)");
   }
+  c->stats_host = reinterpret_cast<uint32_t *>(c->io_host + words);
   return SPH_OK;
 }
 
@@ -1091,14 +1092,20 @@ extern "C" int sph_synchronize(sph_ctx *c) {
   return SPH_OK;
 }
 
-static int fetch_stats(sph_ctx *c, std::vector<uint32_t> *w) {
-  const int rc = launch_collect_stats(c);
-  return rc ? rc : fetch(c, (const uint32_t *)c->stats_read, STAT_READ_WORDS, w);
+// The statistics, written by the GPU into the pinned words: a launch and a wait, 15 us
+// (sph_get_residuals; with a copy into pageable memory after the launch 25).
+static int fetch_stats(sph_ctx *c, const uint32_t **w) {
+  int rc = io_buffers(c);
+  if (!rc) rc = launch_collect_stats(c, c->stats_host);
+  if (rc) return rc;
+  SPH_HIP(hipStreamSynchronize(c->stream));
+  *w = c->stats_host;
+  return SPH_OK;
 }
 
 // Maximum density error of iteration `it` of fetched statistics; a single scene
 // that fell back from its warm start went on from the error before it.
-static float fetched_error(const sph_ctx *c, const std::vector<uint32_t> &w, int it) {
+static float fetched_error(const sph_ctx *c, const uint32_t *w, int it) {
   if (it == 1 && !c->nscenes && w[STAT_FALLBACK]) it = 0;
   float f;
   memcpy(&f, &w[STAT_ERR0 + it], sizeof(f));
@@ -1107,7 +1114,7 @@ static float fetched_error(const sph_ctx *c, const std::vector<uint32_t> &w, int
 
 extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
   if (!c || !st) return arg_error("NULL argument");
-  std::vector<uint32_t> w;
+  const uint32_t *w = nullptr;
   int rc = fetch_stats(c, &w);
   if (rc) return rc;
   memset(st, 0, sizeof(*st));
@@ -1136,7 +1143,7 @@ extern "C" int sph_get_stats(sph_ctx *c, sph_stats *st) {
 
 extern "C" int sph_get_residuals(sph_ctx *c, float *err, int cap, int *count) {
   if (!c || !err || !count) return arg_error("NULL argument");
-  std::vector<uint32_t> w;
+  const uint32_t *w = nullptr;
   int rc = fetch_stats(c, &w);
   if (rc) return rc;
   // one density pass before each applied update; with a tolerance, one more

@@ -235,7 +235,7 @@ struct sph_ctx {
   float *io_host = nullptr;
   hipEvent_t io_done[sph::kIoChunks] = {};
   uint32_t *stats = nullptr;  // sph::STAT_WORDS words
-  uint32_t *stats_read = nullptr;  // sph::STAT_READ_WORDS words
+  uint32_t *stats_host = nullptr;  // sph::STAT_READ_WORDS words at the end of io_host
   uint32_t *pair_partial = nullptr;  // per-block list-length sums of the last search
   uint32_t pair_blocks = 0;
   double *red = nullptr;      // FP64 reduction scratch
@@ -360,7 +360,7 @@ int launch_confine(sph_ctx *c, bool commit);
 int launch_commit(sph_ctx *c);
 // Clears the error words up to iteration `last` that the last search left.
 int launch_clear_errors(sph_ctx *c, int last);
-int launch_collect_stats(sph_ctx *c);
+int launch_collect_stats(sph_ctx *c, uint32_t *out);
 int launch_collide_soa(float *x, float *y, float *z, uint32_t n, const SdfDev &o,
                        hipStream_t s);
 int launch_collide_soa_f64(double *x, double *y, double *z, uint32_t n, const SdfDev &o,

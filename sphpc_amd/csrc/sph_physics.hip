@@ -2641,11 +2641,11 @@ int launch_clear_errors(sph_ctx *c, int last) {
   return SPH_OK;
 }
 
-int launch_collect_stats(sph_ctx *c) {
+int launch_collect_stats(sph_ctx *c, uint32_t *out) {
   static_assert(STAT_ERR0 == kWave, "a wave copies the flags");
   constexpr uint32_t its = kMaxIters + 1;
   k_collect_stats<<<blocks_for(its, kBlock / kWave), kBlock, 0, c->stream>>>(c->stats, its,
-                                                                            c->stats_read);
+                                                                            out);
   SPH_HIP(hipGetLastError());
   return SPH_OK;
 }
