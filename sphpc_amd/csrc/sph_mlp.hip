@@ -532,6 +532,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_mlp_forward(uint64_t count,
 }
 
 // BF16 MFMA inference of a standalone batch (the path fused into the solver).
+template <bool AHEAD>
 __global__ __launch_bounds__(kBlock) void k_mlp_infer(uint64_t count, const float *__restrict__ x,
                                                       const MlpPacked *__restrict__ M,
                                                       float *__restrict__ y) {
@@ -546,9 +547,14 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(uint64_t count, const floa
     f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
     f[8] = c.x; f[9] = c.y; f[10] = c.z; f[11] = c.w;
   }
-  const float out = mlp_wave(f, M);  // whole wave, including lanes past the end
+  const float out = mlp_wave<AHEAD>(f, M);  // whole wave, including lanes past the end
   if (s < count) y[s] = out;
 }
+
+// Rows up to which a wave has a SIMD to itself, or shares it with one more (us, without /
+// with the operands loaded ahead): 4096 rows 7.0 / 5.8, 65,536 7.4 / 6.0, 131,072 8.3 /
+// 8.2, 262,144 13.4 / 13.8, a million 42.7 / 47.2.
+constexpr uint64_t kInferAhead = 1 << 17;
 
 // Packs FP32 master weights into MFMA operand order (BF16) for inference.
 __global__ __launch_bounds__(kBlock) void k_mlp_pack(const float *__restrict__ theta,
@@ -912,8 +918,9 @@ extern "C" int sph_mlp_infer_bf16(sph_mlp *m, const float *x, size_t count, floa
   if (((uintptr_t)x & 15u) != 0) return mlp_arg("features must be 16-byte aligned");
   int rc = mlp_pack(m, m->packed, m->stream);
   if (rc || !count) return rc;
-  k_mlp_infer<<<(unsigned)((count + kBlock - 1) / kBlock), kBlock, 0, m->stream>>>(
-      count, x, m->packed, y);
+  const auto infer = count <= kInferAhead ? k_mlp_infer<true> : k_mlp_infer<false>;
+  infer<<<(unsigned)((count + kBlock - 1) / kBlock), kBlock, 0, m->stream>>>(count, x, m->packed,
+                                                                             y);
   SPH_HIP(hipGetLastError());
   SPH_HIP(hipStreamSynchronize(m->stream));
   return SPH_OK;

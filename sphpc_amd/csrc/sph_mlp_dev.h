@@ -69,6 +69,10 @@ __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 u) { return __builtin_bit_ca
 // (unnormalised) features of this lane's particle; every lane of the wave must
 // call it (inactive lanes pass zeros).  Returns the network output in target
 // units (y * y_scale + y_shift).
+// AHEAD: each step's operands are loaded a step before.  Left to the compiler they are
+// loaded where they are used, and a lone wave waits for memory six times; where others
+// run meanwhile, the registers weigh more (kInferAhead).
+template <bool AHEAD>
 __device__ __forceinline__ float mlp_wave(const float (&f)[kMlpPad], const MlpPacked *__restrict__ M) {
   const int lane = threadIdx.x & 63;
   const int half = lane >> 5;
@@ -93,23 +97,44 @@ __device__ __forceinline__ float mlp_wave(const float (&f)[kMlpPad], const MlpPa
                          : make_uint4(olo[0], olo[1], olo[2], olo[3]);
   const bf16x8_t xcol[2] = {as_bf16x8(xb0), as_bf16x8(xb1)};
 
+  auto vec = [&](const float4 *v, int rb, float (&out)[16]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 b = v[(rb * 2 + half) * 4 + q];
+      out[4 * q] = b.x; out[4 * q + 1] = b.y; out[4 * q + 2] = b.z; out[4 * q + 3] = b.w;
+    }
+  };
+  uint4 a1[2], a2[2][4];
+  float b1[2][16], b2[2][16], w3[2][16];
+  if (AHEAD) {
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      a1[rb] = M->a1[rb * 64 + lane];
+      vec(M->b1, rb, b1[rb]);
+    }
+  }
+  // loads of layer 2's row block ob; other instructions may cross, loads not
+  auto load2 = [&](int ob) {
+    __builtin_amdgcn_sched_barrier(0x48F);
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) a2[ob][kc] = M->a2[(ob * 4 + kc) * 64 + lane];
+    vec(M->b2, ob, b2[ob]);
+    vec(M->w3, ob, w3[ob]);
+    __builtin_amdgcn_sched_barrier(0x48F);
+  };
   uint4 h1[2][4];  // [column block][k chunk] layer 2 B operands
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
-    const bf16x8_t a = as_bf16x8(M->a1[rb * 64 + lane]);
-    float bias[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 b = M->b1[(rb * 2 + half) * 4 + q];
-      bias[4 * q] = b.x; bias[4 * q + 1] = b.y; bias[4 * q + 2] = b.z; bias[4 * q + 3] = b.w;
-    }
+    if (AHEAD && rb == 1) load2(0);
+    const bf16x8_t a = as_bf16x8(AHEAD ? a1[rb] : M->a1[rb * 64 + lane]);
+    if (!AHEAD) vec(M->b1, rb, b1[rb]);
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
       floatx16_t acc = {};
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, xcol[cb], acc, 0, 0, 0);
       float h[16];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) h[v] = silu_infer(acc[v] + bias[v]);
+      for (int v = 0; v < 16; ++v) h[v] = silu_infer(acc[v] + b1[rb][v]);
       h1[cb][2 * rb] = make_uint4(pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3]),
                                   pack_bf16x2(h[4], h[5]), pack_bf16x2(h[6], h[7]));
       h1[cb][2 * rb + 1] = make_uint4(pack_bf16x2(h[8], h[9]), pack_bf16x2(h[10], h[11]),
@@ -119,23 +144,21 @@ __device__ __forceinline__ float mlp_wave(const float (&f)[kMlpPad], const MlpPa
   float part[2] = {0.0f, 0.0f};
 #pragma unroll
   for (int ob = 0; ob < 2; ++ob) {
-    float bias[16], w[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 b = M->b2[(ob * 2 + half) * 4 + q];
-      const float4 u = M->w3[(ob * 2 + half) * 4 + q];
-      bias[4 * q] = b.x; bias[4 * q + 1] = b.y; bias[4 * q + 2] = b.z; bias[4 * q + 3] = b.w;
-      w[4 * q] = u.x; w[4 * q + 1] = u.y; w[4 * q + 2] = u.z; w[4 * q + 3] = u.w;
+    if (AHEAD && ob == 0) load2(1);
+    if (!AHEAD) {
+      vec(M->b2, ob, b2[ob]);
+      vec(M->w3, ob, w3[ob]);
     }
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
       floatx16_t acc = {};
 #pragma unroll
       for (int kc = 0; kc < 4; ++kc)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(M->a2[(ob * 4 + kc) * 64 + lane]),
-                                                      as_bf16x8(h1[cb][kc]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_bf16x8(AHEAD ? a2[ob][kc] : M->a2[(ob * 4 + kc) * 64 + lane]),
+            as_bf16x8(h1[cb][kc]), acc, 0, 0, 0);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) part[cb] += w[v] * silu_infer(acc[v] + bias[v]);
+      for (int v = 0; v < 16; ++v) part[cb] += w3[ob][v] * silu_infer(acc[v] + b2[ob][v]);
     }
   }
 #pragma unroll

@@ -1585,7 +1585,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_lambda(
       row[3] = make_float4(denom, lam0, 0.0f, 0.0f);
     }
   } else {
-    const float y = mlp_wave(f, net);
+    const float y = mlp_wave<false>(f, net);
     const float ymax = net->norm[kNormYMax], step = net->norm[kNormStep];
     const float ce = ymax > 0.0f ? fminf(fmaxf(y, 0.0f), ymax) : fmaxf(y, 0.0f);
     lam = lam0 - (step > 0.0f ? step : 1.0f) * ce / denom;

@@ -193,3 +193,9 @@ def test_activation_over_the_range_of_floats(z):
         _, g = net.gradient(xb, tb, 1)
         dy, want = float(np.float32(y) - np.float32(y - 1.0)), sig * (1.0 + z * (1.0 - sig))
         assert abs(g[5184 + 7] - dy * want) <= 1e-6 * max(abs(want), sig) + 1e-36, (g[5191], want)
+
+
+@pytest.mark.parametrize("count", [1 << 17, (1 << 17) + 1])
+def test_infer_bf16_at_the_limit_of_its_kernels(count):
+    """Operands loaded a step ahead up to 2^17 rows, where they are used above."""
+    test_infer_bf16_matches_emulation(count)
