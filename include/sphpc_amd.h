@@ -333,10 +333,14 @@ int sph_profile_kernel_count(void);
  * neighbour-gather kernel, with an obstacle the push fused into the
  * position update or as a separate pass, and compact (16-bit offsets) versus
  * wide (32-bit indices) neighbour lists; in a small scene also four lanes a
- * particle, which no field of sph_tuning names (the context keeps that until
- * the next sph_set_tuning).  Keeps the fastest choice per kernel.  Results do not
- * depend on the choice. */
+ * particle, as kernels by rule have them there.  Keeps the fastest choice per kernel.
+ * Results do not depend on the choice.
+ *
+ * A kernel that nobody chose a launch for follows a rule by kernel and particle count
+ * (up to 32,768 particles four lanes a particle).  Bit k of block[SPH_TUNE_BY_RULE] says
+ * so of kernel k; its own entries then hold 256 and 16. */
 #define SPH_TUNE_KERNELS 32
+#define SPH_TUNE_BY_RULE 31
 typedef struct sph_tuning {
   int split_collide;              /* obstacle push as a separate pass */
   int wide_lists;                 /* 32-bit list entries for every wavefront */
@@ -347,9 +351,10 @@ typedef struct sph_tuning {
 } sph_tuning;
 int sph_autotune(sph_ctx *ctx, int substeps, sph_tuning *result);
 /* The context's current launch choices (timings zero), and applying a saved
- * set: block 0 / depth 0 keep the default (by kernel and particle count);
- * other values must be 64, 128 or 256 and 8, 16 or 32.  Entries of kernels that
- * are not tuned are ignored. */
+ * set; a set as read changes nothing.  A kernel is by rule if its two entries are 0, or
+ * if its bit of block[SPH_TUNE_BY_RULE] is set and they are 0 or 256 and 0 or 16;
+ * otherwise they must be 64, 128 or 256 and 8, 16 or 32, and 0 beside a chosen one
+ * stands for 256 or 16.  Entries of kernels that are not tuned are ignored. */
 int sph_get_tuning(sph_ctx *ctx, sph_tuning *out);
 int sph_set_tuning(sph_ctx *ctx, const sph_tuning *tuning);
 

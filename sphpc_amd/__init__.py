@@ -58,6 +58,9 @@ class Scene(C.Structure):
                 ("size_z", C.c_double), ("obstacle", ObstacleDesc)]
 
 
+TUNE_BY_RULE = 31  # entry of Tuning.block: bits of the kernels left to the rule
+
+
 class Tuning(C.Structure):
     _fields_ = [("split_collide", C.c_int), ("wide_lists", C.c_int), ("block", C.c_int * 32),
                 ("depth", C.c_int * 32), ("ms_per_substep_default", C.c_double),
@@ -311,13 +314,15 @@ class Context:
         names = kernel_names()
         return dict(block={names[k]: t.block[k] for k in range(len(names))},
                     depth={names[k]: t.depth[k] for k in range(len(names))},
+                    by_rule=[n for k, n in enumerate(names) if t.block[TUNE_BY_RULE] >> k & 1],
                     split_collide=bool(t.split_collide), wide_lists=bool(t.wide_lists),
                     ms_per_substep_default=t.ms_per_substep_default,
                     ms_per_substep_tuned=t.ms_per_substep_tuned)
 
     def autotune(self, substeps=3):
         """Launch autotuner; returns {kernel name: threads per block}, gathers in
-        flight, obstacle-push split, list format and timings."""
+        flight, the kernels left to the library's rule, obstacle-push split, list
+        format and timings."""
         t = Tuning()
         check(lib().sph_autotune(self._h, int(substeps), C.byref(t)))
         return self._tuning_dict(t)
@@ -329,14 +334,17 @@ class Context:
         return self._tuning_dict(t)
 
     def set_tuning(self, block=None, depth=None, split_collide=None, wide_lists=None):
-        """Applies launch choices; dicts map kernel names to values, unnamed
-        kernels keep their current choice."""
+        """Applies launch choices; dicts map kernel names to values (0 in both: by
+        rule), unnamed kernels keep their current choice or rule."""
         t = Tuning()
         check(lib().sph_get_tuning(self._h, C.byref(t)))
         names = kernel_names()
         for src, dst in ((block, t.block), (depth, t.depth)):
             for name, v in (src or {}).items():
-                dst[names.index(name)] = int(v)
+                k = names.index(name)
+                dst[k] = int(v)
+                if v:
+                    t.block[TUNE_BY_RULE] &= ~(1 << k)
         if split_collide is not None:
             t.split_collide = int(bool(split_collide))
         if wide_lists is not None:

@@ -1366,6 +1366,8 @@ extern "C" int sph_memcpy_dtoh(void *dst, const void *src, size_t bytes) {
 static const int kTunable[] = {K_BUILD_LISTS, K_DENSITY_LAMBDA, K_DENSITY, K_LAMBDA, K_DP,
                                K_DP_UPDATE, K_COLOR, K_SURFACE, K_XSPH, K_VORTICITY,
                                K_CONFINE, K_WARM_LAMBDA};
+// Gathers in flight that stand in sph_tuning for a kernel by rule (with kBlock threads).
+constexpr uint8_t kRuleDepth = 16;
 
 extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
   if (c) c->gen++;
@@ -1432,9 +1434,8 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
     graph_reset(c);
     rc = trial(cur, &before);  // as the context was
   }
-  for (int k : kTunable) c->tune.quad[k] = false;
   for (int b = 0; b < 3 && e == hipSuccess && !rc; ++b) {
-    for (int k : kTunable) c->tune.block[k] = sizes[b];
+    for (int k : kTunable) c->tune.block[k] = sizes[b], c->tune.depth[k] = kRuleDepth;
     graph_reset(c);
     rc = trial(cur, &total);
     if (rc) break;
@@ -1460,13 +1461,16 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
         best_depth[k] = depths[d];
       }
   }
-  for (int k : kTunable) c->tune.depth[k] = best_depth[k] ? best_depth[k] : (uint8_t)16;
-  // four lanes a particle, where the scene is small enough for them
-  if (e == hipSuccess && !rc && c->n <= (uint32_t)sph::kQuadMax) {
-    for (int k : kTunable) c->tune.quad[k] = true;
+  for (int k : kTunable) c->tune.depth[k] = best_depth[k] ? best_depth[k] : kRuleDepth;
+  // by rule (four lanes a particle), where the scene is small enough for them
+  if (e == hipSuccess && !rc && c->n <= sph::kQuadMax) {
+    const auto chosen = c->tune;
+    for (int k : kTunable) c->tune.block[k] = 0, c->tune.depth[k] = 0;
     graph_reset(c);
     rc = trial(cur, &total);
-    for (int k : kTunable) c->tune.quad[k] = cur[k] > 0.0 && cur[k] < best[k];
+    for (int k : kTunable)
+      if (!(cur[k] > 0.0 && cur[k] < best[k]))
+        c->tune.block[k] = chosen.block[k], c->tune.depth[k] = chosen.depth[k];
   }
   bool split_best = c->tune.split_collide;
   double after = 0.0;
@@ -1518,10 +1522,12 @@ extern "C" int sph_get_tuning(sph_ctx *c, sph_tuning *out) {
   memset(out, 0, sizeof(*out));
   out->split_collide = c->tune.split_collide;
   out->wide_lists = c->tune.wide_lists;
-  for (int k = 0; k < K_COUNT && k < SPH_TUNE_KERNELS; ++k) {
+  for (int k = 0; k < K_COUNT; ++k) {
     out->block[k] = c->tune.block[k] ? c->tune.block[k] : kBlock;
-    out->depth[k] = c->tune.depth[k] ? c->tune.depth[k] : 16;
+    out->depth[k] = c->tune.depth[k] ? c->tune.depth[k] : kRuleDepth;
   }
+  for (int k : kTunable)
+    if (!c->tune.depth[k]) out->block[SPH_TUNE_BY_RULE] |= 1 << k;
   return SPH_OK;
 }
 
@@ -1534,9 +1540,10 @@ extern "C" int sph_set_tuning(sph_ctx *c, const sph_tuning *t) {
       return arg_error("threads per block must be 0, 64, 128 or 256");
     if (d != 0 && d != 8 && d != 16 && d != 32)
       return arg_error("gathers in flight must be 0, 8, 16 or 32");
-    tune.block[k] = (uint16_t)b;
-    tune.depth[k] = (uint8_t)d;
-    tune.quad[k] = false;
+    const bool marked = (t->block[SPH_TUNE_BY_RULE] >> k & 1) != 0;
+    const bool rule = (!b && !d) || (marked && (!b || b == kBlock) && (!d || d == kRuleDepth));
+    tune.block[k] = (uint16_t)(rule ? 0 : b ? b : kBlock);
+    tune.depth[k] = (uint8_t)(rule ? 0 : d ? d : kRuleDepth);
   }
   tune.split_collide = t->split_collide != 0;
   tune.wide_lists = t->wide_lists != 0;

@@ -22,7 +22,7 @@ static_assert((kMaxParticles + 64ull) * 16ull <= (1ull << 32), "32-bit byte offs
 // Chunks of a state transfer, at most.
 constexpr int kIoChunks = 16;
 // Most particles of the gather kernels with four lanes a particle (sum_neighbors),
-// if nobody chose a launch or the autotuner measured them fastest.  A wave of 64
+// if nobody chose a launch.  A wave of 64
 // particles leaves most SIMDs without one up to here, and each lane's gathers come
 // in four or more rounds one after the other; four lanes need one or two.  Measured
 // (us, events included: about 3.5 of each; one lane a particle / four): density 8.9
@@ -174,6 +174,7 @@ enum KernelId {
   K_POS_STARS, K_VELOCITY, K_COLOR, K_SURFACE, K_XSPH, K_VORTICITY, K_CONFINE, K_COMMIT,
   K_AUX, K_WARM_LAMBDA, K_COLLIDE, K_LAMBDA_COPY, K_PLACE, K_COUNT
 };
+static_assert(K_COUNT <= SPH_TUNE_BY_RULE, "a bit and an entry of sph_tuning for each");
 
 struct ScanScratch {
   uint32_t *tile_sums = nullptr;
@@ -267,11 +268,11 @@ struct sph_ctx {
     // the push fused a frame's kernels take 3.7 ms instead of 4.3 at 131k
     // particles, 7.9 instead of 8.1 at 1M, 60.2 instead of 60.8 at 8.4M)
     bool split_collide = false;
-    uint16_t block[sph::K_COUNT] = {};  // threads per block of gather kernels (0: by rule)
-    uint8_t depth[sph::K_COUNT] = {};   // gathers in flight per wave: 8, 16, 32 (0: by rule)
+    // threads per block of gather kernels and gathers in flight per wave (8, 16 or
+    // 32); both 0: by rule
+    uint16_t block[sph::K_COUNT] = {};
+    uint8_t depth[sph::K_COUNT] = {};
     bool wide_lists = false;  // 32-bit list entries for every wave
-    // four lanes a particle measured fastest (the autotuner; not part of sph_tuning)
-    bool quad[sph::K_COUNT] = {};
   } tune;
   // whole-substep HIP graph (sph_set_graph)
   bool graph_on = false;

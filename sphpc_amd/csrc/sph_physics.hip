@@ -2086,8 +2086,8 @@ __global__ __launch_bounds__(kBlock) void k_kinetic_energy(uint32_t n,
 // 1M 69.9 / 72.0; surface 681k 48.8 / 50.6, 1M 70.1 / 76.8.
 static inline int tuned_depth(const sph_ctx *c, int kernel) {
   const int d = c->tune.depth[kernel];
-  if (c->n <= kQuadMax && (c->tune.quad[kernel] || (!d && !c->tune.block[kernel]))) return kQuad;
   if (d) return d;
+  if (c->n <= kQuadMax) return kQuad;
   int most = 1 << 19;
   if (kernel == K_DENSITY_LAMBDA || kernel == K_DENSITY || kernel == K_LAMBDA) most = 1 << 21;
   if (kernel == K_DP || kernel == K_DP_UPDATE) most = 1 << 20;

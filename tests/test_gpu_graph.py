@@ -4,6 +4,8 @@ Every kernel of the substep is deterministic (integer atomics and max
 reductions only), so a replayed graph must give bit-identical states and
 statistics.  The graph is replayed several times with eager work and host
 synchronisations in between, and every replay is compared."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -250,3 +252,63 @@ def test_density_stage_after_substeps_of_fewer_iterations(graph, passes, iters):
             assert np.max(c.field(sa.FIELD_DENSITY)) < 1000.0
         c.step(1)
         assert c.stats().max_density_error == c.residuals()[-1]
+
+
+GATHERS = ("density_lambda", "density", "lambda", "dp", "dp_update", "color", "surface", "xsph",
+           "vorticity", "confine")
+
+
+def _raw(ctx):
+    t = sa.Tuning()
+    sa.check(sa.lib().sph_get_tuning(ctx.handle, C.byref(t)))
+    return t
+
+
+def test_tuning_as_read_changes_nothing():
+    """Kernels by rule stay by rule through a read and a write, through one that names
+    another field or kernel, and in another context; naming a kernel takes it out (what
+    is not named of it is 256 or 16), zeros put it back."""
+    sc, (a, b) = _pair(0.0)
+    rule = a.tuning()["by_rule"]
+    assert set(GATHERS) <= set(rule) and "predict_hash" not in rule
+    sa.check(sa.lib().sph_set_tuning(a.handle, C.byref(_raw(a))))
+    assert a.tuning() == b.tuning()
+    a.set_tuning(wide_lists=True, split_collide=True)
+    assert a.tuning()["by_rule"] == rule
+    a.set_tuning(block={"xsph": 64}, depth={"color": 8, "surface": 16})
+    t = a.tuning()
+    assert t["by_rule"] == [k for k in rule if k not in ("xsph", "color", "surface")]
+    assert (t["block"]["xsph"], t["depth"]["xsph"]) == (64, 16)
+    assert (t["block"]["color"], t["depth"]["color"]) == (256, 8)
+    sa.check(sa.lib().sph_set_tuning(b.handle, C.byref(_raw(a))))
+    assert b.tuning() == t
+    a.set_tuning(block={"xsph": 0, "color": 0}, depth={"xsph": 0, "color": 0})
+    assert a.tuning()["by_rule"] == [k for k in rule if k != "surface"]
+    sa.check(sa.lib().sph_set_tuning(a.handle, C.byref(sa.Tuning())))
+    assert a.tuning()["by_rule"] == rule
+    a.autotune(1)
+    sa.check(sa.lib().sph_set_tuning(b.handle, C.byref(_raw(a))))
+    assert b.tuning() == a.tuning()
+    for step in range(2):
+        a.upload(*b.download())
+        a.step(1)
+        b.step(1)
+        pa, va = a.download()
+        pb, vb = b.download()
+        assert np.array_equal(pa, pb) and np.array_equal(va, vb), step
+
+
+@pytest.mark.parametrize("n,squeeze,wide,calls", [
+    (1, 1.0, True, "staged"), (3, 1.0, False, "fused"), (15, 1.0, True, "fused"),
+    (16, 1.0, False, "staged"), (65, 1.0, True, "staged"), (4099, 0.85, False, "staged"),
+    (4099, 0.85, True, "fused"), (32768, 0.85, True, "fused")])
+def test_four_lanes_by_rule_equal_one(n, squeeze, wide, calls):
+    """More shapes of the comparison above, where the context of the default rule is known
+    to be by rule also after the list format was chosen (one lane from 32,769 particles
+    and for the kernels of the other context)."""
+    with Scene(0.02, (1.0, 1.0, 1.0)).context(n) as c:
+        c.set_tuning(wide_lists=wide)
+        assert set(GATHERS) <= set(c.tuning()["by_rule"])
+        c.set_tuning(depth={k: 16 for k in GATHERS})
+        assert not set(GATHERS) & set(c.tuning()["by_rule"])
+    test_four_lanes_a_particle_equal_one(n, squeeze, wide, calls)
