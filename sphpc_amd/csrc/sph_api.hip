@@ -1357,12 +1357,13 @@ extern "C" int sph_memcpy_dtoh(void *dst, const void *src, size_t bytes) {
 // --------------------------------------------------------------------------
 // Timing
 // --------------------------------------------------------------------------
-// Launch autotuner.  Tries 64, 128 and 256 threads per block and then 8, 16
-// and 32 gathers in flight per wave for every neighbour-gather kernel and,
+// Launch autotuner.  Tries the rule, 64, 128 and 256 threads per block and then
+// 8, 16 and 32 gathers in flight per wave for every neighbour-gather kernel and,
 // with an obstacle, the fused versus separate obstacle push, timing
 // `substeps` substeps of each candidate with HIP events from the same saved
-// state; keeps the fastest choice per kernel and restores the state.  None of
-// the choices changes any result.
+// state; keeps the fastest choice per kernel, or all as it was if the choices
+// together are no faster, and restores the state.  None of the choices changes
+// any result.
 static const int kTunable[] = {K_BUILD_LISTS, K_DENSITY_LAMBDA, K_DENSITY, K_LAMBDA, K_DP,
                                K_DP_UPDATE, K_COLOR, K_SURFACE, K_XSPH, K_VORTICITY,
                                K_CONFINE, K_WARM_LAMBDA};
@@ -1426,7 +1427,7 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
     c->prof.on = false;
     return SPH_OK;
   };
-  double best[K_COUNT], cur[K_COUNT], total = 0.0, before = 0.0;
+  double best[K_COUNT], rule[K_COUNT], cur[K_COUNT] = {}, total = 0.0, before = 0.0;
   uint16_t best_bs[K_COUNT] = {};
   for (int k = 0; k < K_COUNT; ++k) best[k] = 1e300;
   const uint16_t sizes[3] = {64, 128, 256};
@@ -1434,6 +1435,14 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
     graph_reset(c);
     rc = trial(cur, &before);  // as the context was
   }
+  bool chosen = false;
+  for (int k : kTunable) chosen = chosen || c->tune.depth[k] != 0;
+  if (chosen && e == hipSuccess && !rc) {
+    for (int k : kTunable) c->tune.block[k] = 0, c->tune.depth[k] = 0;
+    graph_reset(c);
+    rc = trial(cur, &total);
+  }
+  for (int k = 0; k < K_COUNT; ++k) rule[k] = cur[k];
   for (int b = 0; b < 3 && e == hipSuccess && !rc; ++b) {
     for (int k : kTunable) c->tune.block[k] = sizes[b], c->tune.depth[k] = kRuleDepth;
     graph_reset(c);
@@ -1461,16 +1470,13 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
         best_depth[k] = depths[d];
       }
   }
-  for (int k : kTunable) c->tune.depth[k] = best_depth[k] ? best_depth[k] : kRuleDepth;
-  // by rule (four lanes a particle), where the scene is small enough for them
-  if (e == hipSuccess && !rc && c->n <= sph::kQuadMax) {
-    const auto chosen = c->tune;
-    for (int k : kTunable) c->tune.block[k] = 0, c->tune.depth[k] = 0;
-    graph_reset(c);
-    rc = trial(cur, &total);
-    for (int k : kTunable)
-      if (!(cur[k] > 0.0 && cur[k] < best[k]))
-        c->tune.block[k] = chosen.block[k], c->tune.depth[k] = chosen.depth[k];
+  // the fastest, by rule if that is as fast; kernels that did not run stay as they were
+  for (int k : kTunable) {
+    c->tune.depth[k] = best_depth[k];
+    if (!best_depth[k])
+      c->tune.block[k] = tune0.block[k], c->tune.depth[k] = tune0.depth[k];
+    else if (rule[k] <= best[k])
+      c->tune.block[k] = 0, c->tune.depth[k] = 0;
   }
   bool split_best = c->tune.split_collide;
   double after = 0.0;
@@ -1498,7 +1504,10 @@ extern "C" int sph_autotune(sph_ctx *c, int substeps, sph_tuning *out) {
     else
       c->tune.wide_lists = wide0;
   }
-  if (rc || e != hipSuccess) c->tune = tune0;
+  if (rc || e != hipSuccess || !(after < before)) {  // what was found stays, if as fast
+    c->tune = tune0;
+    after = before;
+  }
   const hipError_t er = copy_state(false);
   release();
   prof_zero(c);

@@ -312,3 +312,27 @@ def test_four_lanes_by_rule_equal_one(n, squeeze, wide, calls):
         c.set_tuning(depth={k: 16 for k in GATHERS})
         assert not set(GATHERS) & set(c.tuning()["by_rule"])
     test_four_lanes_a_particle_equal_one(n, squeeze, wide, calls)
+
+
+@pytest.mark.parametrize("n", [1, 200, 4000])
+def test_autotuner_keeps_nothing_slower_than_it_found(n):
+    """The set it reports took no longer than the context's own launches, which stay if
+    nothing was faster (small scenes, where times differ by chance alone), also where
+    they were chosen before; kernels that did not run stay as they were."""
+    sc = Scene(0.02, (1.0, 1.0, 1.0), iters=2, lambda_eps=600.0)
+    side = int(np.ceil(np.cbrt(n) - 1e-9))
+    pos = block_scene((side,) * 3, 0.02, (0.1, 0.1, 0.1))[0][:n]
+    for chosen in ({}, {"dp_update": 8, "color": 32}):
+        with sc.context(n) as c:
+            c.upload(pos)
+            for _ in range(3):
+                c.set_tuning(depth=chosen)
+                was = c.tuning()
+                t = c.autotune(1)
+                assert t["ms_per_substep_tuned"] <= t["ms_per_substep_default"]
+                for k in ("color", "xsph", "dp"):
+                    assert (t["block"][k], t["depth"][k]) == (was["block"][k], was["depth"][k])
+                    assert (k in t["by_rule"]) == (k in was["by_rule"])
+                if t["ms_per_substep_tuned"] == t["ms_per_substep_default"]:
+                    for k in ("block", "depth", "by_rule", "split_collide", "wide_lists"):
+                        assert t[k] == was[k]
