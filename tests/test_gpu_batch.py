@@ -87,6 +87,42 @@ def test_batch_bit_identical_to_separate_contexts(graph):
            graph=int(graph))
 
 
+@pytest.mark.parametrize("side,count", [(26, 3), (44, 3)])
+def test_larger_batches_bit_identical_to_separate_contexts(side, count):
+    """Scenes whose list build is the one of a wavefront per layer (50k to 70k particles
+    together) and per 64 particles (250k), alone another kernel's; scenes end inside
+    wavefronts."""
+    s = float(np.float32(0.02))
+    scenes = []
+    for k in range(count):
+        nb = (side + k, side - 1, side)
+        pos = sa.scene_lattice([sa.Block(*nb, 0.0, 0.0, 0.0)], 0.9 * s, jitter=0.01, seed=k)
+        vel = np.random.default_rng(k).normal(0, 0.1, pos.shape).astype(np.float32)
+        size = tuple(round(1.3 * n * s, 2) for n in nb)
+        scenes.append(dict(particles=len(pos), size=size, sdf=None, pos=pos, vel=vel))
+    total = sum(sc["particles"] for sc in scenes)
+    assert 40960 < total <= 196608 if side < 40 else total > 196608
+    p = _params(s)
+    with sa.BatchContext(p, scenes) as batch:
+        batch.upload(np.concatenate([sc["pos"] for sc in scenes]),
+                     np.concatenate([sc["vel"] for sc in scenes]))
+        batch.step(2)
+        bp, bv = batch.download()
+        ids, cnt = batch.neighbors()
+        ids = ids.reshape(-1, sa.MAX_NEIGHBORS)
+        for k, sc in enumerate(scenes):
+            a, b = batch.first[k], batch.first[k + 1]
+            with sa.Context(p, sc["size"], sc["particles"]) as c:
+                c.upload(sc["pos"], sc["vel"])
+                c.step(2)
+                sp, sv = c.download()
+                one, n = c.neighbors()
+            assert np.array_equal(bp[a:b], sp) and np.array_equal(bv[a:b], sv), k
+            assert np.array_equal(cnt[a:b], n), k
+            used = np.arange(sa.MAX_NEIGHBORS)[None, :] < n[:, None]
+            assert np.array_equal(ids[a:b][used], one.reshape(-1, sa.MAX_NEIGHBORS)[used] + a), k
+
+
 def _stage_substep(ctx, iters):
     """One substep through the stage entry points, in the reference's order."""
     ctx.apply_gravity()

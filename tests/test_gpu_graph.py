@@ -336,3 +336,25 @@ def test_autotuner_keeps_nothing_slower_than_it_found(n):
                 if t["ms_per_substep_tuned"] == t["ms_per_substep_default"]:
                     for k in ("block", "depth", "by_rule", "split_collide", "wide_lists"):
                         assert t[k] == was[k]
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("block", [64, 128])
+def test_list_build_does_not_depend_on_its_threads(block, wide):
+    """Above 196,608 particles the list build takes the threads per block that are asked
+    for; the lists are those of 256."""
+    sc = Scene(0.02, (2.0, 2.0, 2.0))
+    pos, vel = block_scene((59, 59, 59), 0.02 * 0.8, (0.0, 0.0, 0.0), jitter=0.05, seed=6)
+    lists = []
+    for b in (0, block):
+        with sc.context(len(pos)) as c:
+            c.set_tuning(block={"build_lists": b}, wide_lists=wide)
+            c.upload(pos, vel)
+            c.predict_positions()
+            c.find_all_neighbors()
+            lists.append(c.neighbors() + (c.stats().neighbor_pairs, c.stats().neighbor_overflow))
+    (ids, cnt, pairs, lost), (ids2, cnt2, pairs2, lost2) = lists
+    assert np.array_equal(cnt, cnt2) and (pairs, lost) == (pairs2, lost2) and pairs == cnt.sum()
+    used = np.arange(sa.MAX_NEIGHBORS)[None, :] < cnt[:, None]
+    shape = (len(pos), sa.MAX_NEIGHBORS)
+    assert np.array_equal(ids.reshape(shape)[used], ids2.reshape(shape)[used])
