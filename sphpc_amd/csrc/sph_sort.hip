@@ -236,6 +236,7 @@ int scan(const uint32_t *in, uint32_t *out, uint32_t len, bool inclusive, bool w
   if (!self && sc->tile_cap < tiles) {
     if (sc->tile_sums) SPH_HIP(hipFree(sc->tile_sums));
     sc->tile_sums = nullptr;
+    sc->tile_cap = 0;
     SPH_HIP(hipMalloc(&sc->tile_sums, sizeof(uint32_t) * tiles));
     sc->tile_cap = tiles;
   }
