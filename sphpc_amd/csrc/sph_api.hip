@@ -597,18 +597,29 @@ extern "C" int sph_set_obstacle(sph_ctx *c, const sph_obstacle_desc *o) {
 // host copies the next or the previous one, and several threads copy because one
 // does 27 GB/s.  8.4M particles with velocities: upload 10.2 -> 5.3 ms, download
 // 10.3 -> 4.2 ms; 4096: 31 -> 27 us and 33 -> 26 us (a copy on the device less).
-constexpr int kIoChunk = 1 << 15;  // particles, at least (up to kIoChunks chunks)
-// Particles from which helper threads copy too: starting three takes some 30 us.  One
-// thread / four, us: upload 200k particles 152 / 190, 400k 273 / 320, 800k 634 / 550;
-// download 200k 163 / 161, 400k 320 / 285.  131k on one thread in one chunk take 136 and
-// 147 us (up, down), in four 108 and 118; with copies by the DMA engines in place of the
-// kernels' own reads and writes 128 and 163.
-constexpr size_t kIoUploadHelp = 1 << 19, kIoDownloadHelp = 1 << 18;
+constexpr size_t kIoOneChunk = 1 << 15;  // particles of capacity, at most
+// Capacity from which all threads copy chunks of 2^15 particles or more; below it three
+// chunks, uploaded by the calling thread alone (one helper for a download): starting three
+// threads takes some 30 us, and one thread hides more of the bus behind three chunks than
+// behind four or more.  Upload, us, changing arrays (out of cache): in one chunk / three
+// by one thread / eight or sixteen by four, 60k 86 (156) / 79 (137) / 152, 131k 181 (259)
+// / 141 (207) / 184, 200k 267 (355) / 203 (278) / 255, 330k 450 (515) / 307 (416) / 333
+// (405), 524k 714 (807) / 480 (624) / 461 (525).  Download: 131k 186 (240) / three by two
+// threads 125 (171) / 145, 200k 277 (333) / 200 (248) / 177 (230), 330k 450 / 297 (360) /
+// 258 (306).
+constexpr size_t kIoManyChunks = 1 << 18;
 
 static size_t io_chunk(const sph_ctx *c) {
   const size_t cap = (size_t)std::max(c->cap, 1);
-  if (cap <= (size_t)kIoChunk) return (cap + 3) & ~(size_t)3;
-  return std::max<size_t>(kIoChunk, ((cap + kIoChunks - 1) / kIoChunks + 1023) & ~(size_t)1023);
+  if (cap <= kIoOneChunk) return (cap + 3) & ~(size_t)3;
+  const size_t parts = cap < kIoManyChunks ? 3 : kIoChunks;
+  const size_t chunk = ((cap + parts - 1) / parts + 1023) & ~(size_t)1023;
+  return cap < kIoManyChunks ? chunk : std::max<size_t>(32768, chunk);
+}
+
+// Threads that copy, the calling one among them.
+static int io_threads(const sph_ctx *c, bool upload) {
+  return (size_t)c->cap >= kIoManyChunks ? kIoThreads : upload ? 1 : 2;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pack_state(uint32_t n, uint32_t chunk,
@@ -694,7 +705,7 @@ extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *
     std::atomic<bool> staged[kIoChunks] = {};
     size_t sent = 0;
     io_chunks(
-        chunks, un >= kIoUploadHelp ? kIoThreads : 1,
+        chunks, io_threads(c, true),
         [&](size_t k) {
           const size_t first = k * chunk, m = std::min(chunk, un - first);
           float *to = c->io_host + 6 * first;
@@ -742,7 +753,7 @@ extern "C" int sph_download_state(sph_ctx *c, float *x, float *y, float *z, floa
     if (chunks == 1) SPH_HIP(hipStreamSynchronize(c->stream));
     std::atomic<int> failed{hipSuccess};
     io_chunks(
-        chunks, un >= kIoDownloadHelp ? kIoThreads : 1,
+        chunks, io_threads(c, false),
         [&](size_t k) {
           if (chunks > 1) {
             const hipError_t e = hipEventSynchronize(c->io_done[k]);

@@ -142,11 +142,10 @@ def test_state_transfer_round_trip(n, cap):
 
 
 @pytest.mark.parametrize("n,cap", [(1 << 15,) * 2, ((1 << 15) + 1,) * 2, (1 << 15, 1 << 20),
-                                   ((1 << 18) - 1,) * 2, (1 << 18,) * 2, ((1 << 19) - 1,) * 2,
-                                   (1 << 19,) * 2])
+                                   (70000, 70001), (30000, 70001), ((1 << 18) - 1,) * 2,
+                                   (1 << 18,) * 2])
 def test_state_transfer_at_the_limits_of_its_chunks(n, cap):
-    """One chunk up to 2^15 particles of capacity; helper threads from 2^18 particles
-    (download) and 2^19 (upload)."""
+    """One chunk up to 2^15 particles of capacity, three below 2^18, more from there on."""
     test_state_transfer_round_trip(n, cap)
 
 
