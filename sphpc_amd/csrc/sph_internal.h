@@ -340,9 +340,9 @@ int count_keys(const uint32_t *keys, uint32_t n, uint32_t *count, uint32_t cells
 int launch_gravity(sph_ctx *c);
 int launch_predict(sph_ctx *c);
 int launch_neighbor_search(sph_ctx *c, bool fused);
-// mode 0: density + lambda (fused substep), 1: density, 2: lambda, 3: density
-// with rho into pos.w (tolerance loop), 4: density + lambda with rho into pos.w
-// and (x*, lambda) into the other position buffer (the stage path)
+// mode 0: density + lambda (fused substep), 2: lambda, 3: density with rho into pos.w
+// (tolerance loop), 4: density + lambda with rho into pos.w and (x*, lambda) into the
+// other position buffer (the stage path)
 int launch_density(sph_ctx *c, int mode, int err_slot);
 // xnext: also the position update of launch_position_stars, into xnext
 int launch_dp(sph_ctx *c, int substep, float4 *xnext = nullptr);

@@ -2271,7 +2271,7 @@ static float stiffness_scale(const sph_ctx *c, int substep) {
 int launch_density(sph_ctx *c, int mode, int err_slot) {
   const uint32_t n = c->n;
   if (!n) return SPH_OK;
-  const int kernel = mode == 0 || mode == 4 ? K_DENSITY_LAMBDA : mode == 2 ? K_LAMBDA : K_DENSITY;
+  const int kernel = mode == 2 ? K_LAMBDA : mode == 3 ? K_DENSITY : K_DENSITY_LAMBDA;
   const Gather g = gather_launch(c, kernel, K_DENSITY_LAMBDA);
   const uint32_t bs = g.threads, nb = g.blocks;
   hipStream_t s = c->stream;
@@ -2282,14 +2282,6 @@ int launch_density(sph_ctx *c, int mode, int err_slot) {
                    k_density_lambda<0, NBv><<<nb, bs, 0, s>>>(
                        n, nb, c->pos, c->list, c->list_head, c->dev, c->rho, nullptr, c->stats,
                        err_slot, c->P.density_tolerance > 0, 0, nullptr));
-    });
-  else if (mode == 1)
-    with_depth(g.depth, [&](auto D_) {
-      constexpr int NBv = decltype(D_)::value;
-      LAUNCH_TIMED(c, K_DENSITY, 0,
-                   k_density_lambda<1, NBv><<<nb, bs, 0, s>>>(
-                       n, nb, c->pos, c->list, c->list_head, c->dev, c->rho, c->cstage, c->stats,
-                       err_slot, 0, 0, nullptr));
     });
   else if (mode == 4)  // density and lambda in one gather: rho into w, (x*, lambda) aside
     with_depth(g.depth, [&](auto D_) {
