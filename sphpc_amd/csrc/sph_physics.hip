@@ -685,26 +685,28 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint2 *__r
   // 100,000 particles in one cell this kernel takes 7.8 ms with four ids in flight, 2.6
   // with sixteen, 2.1 with scalars (the list build 4.7); with 250,000 21.2, 9.7 and 4.9
   // (29.2).
-  const uint32_t wave_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
-  if (__ballot(a != wave_a) == 0ull) {
-    const uint32_t wave_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
-    uint32_t k = wave_a;
-    for (; wave_b - k > 16u; k += 16) {
-      const Slots8 lo = *reinterpret_cast<const Slots8 *>(slots + k);
-      const Slots8 hi = *reinterpret_cast<const Slots8 *>(slots + k + 8);
+  if (__ballot(b - a > 16u) != 0ull) {
+    const uint32_t wave_a = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    if (__ballot(a != wave_a) == 0ull) {
+      const uint32_t wave_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+      uint32_t k = wave_a;
+      for (; wave_b - k > 16u; k += 16) {
+        const Slots8 lo = *reinterpret_cast<const Slots8 *>(slots + k);
+        const Slots8 hi = *reinterpret_cast<const Slots8 *>(slots + k + 8);
 #pragma unroll
-      for (int u = 0; u < 16; u += 2) s += lo[u] < me.x ? 1u : 0u;
+        for (int u = 0; u < 16; u += 2) s += lo[u] < me.x ? 1u : 0u;
 #pragma unroll
-      for (int u = 0; u < 16; u += 2) s += hi[u] < me.x ? 1u : 0u;
+        for (int u = 0; u < 16; u += 2) s += hi[u] < me.x ? 1u : 0u;
+      }
+      m = k;
     }
-    m = k;
-  }
-  for (; b - m > 16u; m += 16) {
-    uint32_t id[16];
+    for (; b - m > 16u; m += 16) {
+      uint32_t id[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) id[u] = slots[m + u].x;
+      for (int u = 0; u < 16; ++u) id[u] = slots[m + u].x;
 #pragma unroll
-    for (int u = 0; u < 16; ++u) s += id[u] < me.x ? 1u : 0u;
+      for (int u = 0; u < 16; ++u) s += id[u] < me.x ? 1u : 0u;
+    }
   }
   for (; m < b; m += 4) {  // four ids in flight
     uint32_t id[4];
