@@ -597,16 +597,14 @@ extern "C" int sph_set_obstacle(sph_ctx *c, const sph_obstacle_desc *o) {
 // host copies the next or the previous one, and several threads copy because one
 // does 27 GB/s.  8.4M particles with velocities: upload 10.2 -> 5.3 ms, download
 // 10.3 -> 4.2 ms; 4096: 31 -> 27 us and 33 -> 26 us (a copy on the device less).
-constexpr size_t kIoOneChunk = 1 << 15;  // particles of capacity, at most
+constexpr size_t kIoOneChunk = 3 << 15;  // particles of capacity, at most
 // Capacity from which all threads copy chunks of 2^15 particles or more; below it three
-// chunks, uploaded by the calling thread alone (one helper for a download): starting three
-// threads takes some 30 us, and one thread hides more of the bus behind three chunks than
-// behind four or more.  Upload, us, changing arrays (out of cache): in one chunk / three
-// by one thread / eight or sixteen by four, 60k 86 (156) / 79 (137) / 152, 131k 181 (259)
-// / 141 (207) / 184, 200k 267 (355) / 203 (278) / 255, 330k 450 (515) / 307 (416) / 333
-// (405), 524k 714 (807) / 480 (624) / 461 (525).  Download: 131k 186 (240) / three by two
-// threads 125 (171) / 145, 200k 277 (333) / 200 (248) / 177 (230), 330k 450 / 297 (360) /
-// 258 (306).
+// chunks, uploaded by the calling thread alone (one helper for a download), for starting
+// three threads takes some 30 us.  Frames of two substeps on changing arrays, us (of
+// which the upload): 65k in one chunk 402 (90), three 420 (117); 90k 505 (123), 492
+// (141); 131k in one 638 (174), three 575 (174), four by all threads 616 (203); 180k
+// 820 (234), 724 (225), 728 (232); 229k 1010 (290), 876 (280), 856 (268).  Copies by the
+// DMA engines took 92, 118, 163, 215 and 270 up.
 constexpr size_t kIoManyChunks = 1 << 18;
 
 static size_t io_chunk(const sph_ctx *c) {

@@ -141,11 +141,12 @@ def test_state_transfer_round_trip(n, cap):
         assert np.array_equal(y, vel[:, 1]) and np.array_equal(vz, pos[:, 2])
 
 
-@pytest.mark.parametrize("n,cap", [(1 << 15,) * 2, ((1 << 15) + 1,) * 2, (1 << 15, 1 << 20),
-                                   (70000, 70001), (30000, 70001), ((1 << 18) - 1,) * 2,
+@pytest.mark.parametrize("n,cap", [(3 << 15,) * 2, ((3 << 15) + 1,) * 2, (1 << 15, 1 << 20),
+                                   (100001, 100003), (30000, 100003), ((1 << 18) - 1,) * 2,
                                    (1 << 18,) * 2])
 def test_state_transfer_at_the_limits_of_its_chunks(n, cap):
-    """One chunk up to 2^15 particles of capacity, three below 2^18, more from there on."""
+    """One chunk up to 3 2^15 particles of capacity, three below 2^18, more from there
+    on."""
     test_state_transfer_round_trip(n, cap)
 
 
