@@ -615,9 +615,11 @@ static size_t io_chunk(const sph_ctx *c) {
   return cap < kIoManyChunks ? chunk : std::max<size_t>(32768, chunk);
 }
 
-// Threads that copy, the calling one among them.
-static int io_threads(const sph_ctx *c, bool upload) {
-  return (size_t)c->cap >= kIoManyChunks ? kIoThreads : upload ? 1 : 2;
+// Threads that copy, the calling one among them.  The first upload also takes the page
+// faults of the staging, which several threads take side by side (131k 1.4 ms by one
+// thread, 0.8 by three).
+static int io_threads(const sph_ctx *c, bool upload, bool first = false) {
+  return first || (size_t)c->cap >= kIoManyChunks ? kIoThreads : upload ? 1 : 2;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pack_state(uint32_t n, uint32_t chunk,
@@ -696,6 +698,7 @@ extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *
   if (n != c->n) graph_reset(c);
   SPH_HIP(hipStreamSynchronize(c->stream));
   if (n) {
+    const bool first = !c->io_host;
     int rc = io_buffers(c);
     if (rc) return rc;
     const size_t un = (size_t)n, chunk = io_chunk(c), chunks = (un + chunk - 1) / chunk;
@@ -703,7 +706,7 @@ extern "C" int sph_upload_state(sph_ctx *c, int n, const float *x, const float *
     std::atomic<bool> staged[kIoChunks] = {};
     size_t sent = 0;
     io_chunks(
-        chunks, io_threads(c, true),
+        chunks, io_threads(c, true, first),
         [&](size_t k) {
           const size_t first = k * chunk, m = std::min(chunk, un - first);
           float *to = c->io_host + 6 * first;
