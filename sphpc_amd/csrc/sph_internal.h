@@ -235,6 +235,7 @@ struct sph_ctx {
   // memory, by chunks, and each chunk's end of unpacking (on first use)
   float *io_host = nullptr;
   hipEvent_t io_done[sph::kIoChunks] = {};
+  bool io_downloaded = false;
   uint32_t *stats = nullptr;  // sph::STAT_WORDS words
   uint32_t *stats_host = nullptr;  // sph::STAT_READ_WORDS words at the end of io_host
   uint32_t *pair_partial = nullptr;  // per-block list-length sums of the last search
